@@ -31,6 +31,7 @@
 #include <type_traits>
 
 #include "../../include/gsbn_amd.h"
+#include "detfast.h"
 #include "detmath.h"
 #include "gsbn_core.h"
 #include "philox.h"
@@ -259,7 +260,7 @@ __device__ float unit_dsup(const gsbn_pop_args& a, int h, int j, const float* ef
   const int64_t N = (int64_t)a.H * a.M;
   const int idx = h * a.M + j;
   float z;
-  gsbn_draw_unit(a.seed, (uint32_t)a.pop_id, (uint32_t)a.simstep, (uint32_t)idx, u, &z);
+  gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)a.simstep, (uint32_t)idx, u, &z);
   *xi = a.snoise * z;
   float wsup = 0.0f;
   for (int m = 0; m < a.nproj_in; ++m) wsup += a.bj[m * N + idx] + efin[m];
@@ -766,7 +767,7 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
   float u = 0.0f, xi = 0.0f;
   if (live) {
     float z;
-    gsbn_draw_unit(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)idx, &u, &z);
+    gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)idx, &u, &z);
     xi = a.snoise * z;
   }
   float pj_n = 0.0f, ej_n = 0.0f, zj_n = 0.0f, bj_n = 0.0f;
@@ -780,7 +781,7 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
     ej_n = ej0 + (zj0 - ej0) * p0.ke;
     zj_n = zj0 * (1 - p0.kzj);
     bj_w = kp != 0.0f;
-    if (bj_w) bj_n = p0.bgain * gsbn_logf(pj_n + p0.eps);
+    if (bj_w) bj_n = p0.bgain * gsbn_logf_guarded(pj_n + p0.eps);
   }
   if (j > 0 && j < nin) sh_pend[j] = a.projs[j].pend_cnt[h];
   __syncthreads();
@@ -855,10 +856,10 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
 
   /* soft-max (Pop.cpp:280-302); the normaliser is summed in ascending unit
    * order by one thread, four LDS words per read */
-  const float maxact = gsbn_expf(a.wtagain * maxdsup);
+  const float maxact = gsbn_expf_guarded(a.wtagain * maxdsup);
   float act = 0.0f;
   if (live) {
-    act = gsbn_expf(a.wtagain * (dsup - maxdsup));
+    act = gsbn_expf_guarded(a.wtagain * (dsup - maxdsup));
     if (maxact < 1.0f) act *= maxact;
     sh_f[j] = act;
   }
@@ -1003,7 +1004,7 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
       ej += (zj - ej) * p.ke;
       zj *= (1 - p.kzj);
       if (spk > 0) zj += p.kftj;
-      if (kp != 0.0f) a.bj[m * N + idx] = p.bgain * gsbn_logf(pj + p.eps);
+      if (kp != 0.0f) a.bj[m * N + idx] = p.bgain * gsbn_logf_guarded(pj + p.eps);
       p.pj[idx] = pj;
       p.ej[idx] = ej;
       p.zj[idx] = zj;
@@ -1249,7 +1250,7 @@ __device__ __forceinline__ void pop_body_w(const gsbn_pop_args& a, const PopStep
     bj_w[u] = false;
     if (j < M) {
       float z;
-      gsbn_draw_unit(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)(h * M + j), &ud[u],
+      gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)(h * M + j), &ud[u],
                      &z);
       xi[u] = a.snoise * z;
       if (ps.do_jxx && nin > 0) {
@@ -1258,7 +1259,7 @@ __device__ __forceinline__ void pop_body_w(const gsbn_pop_args& a, const PopStep
         ej_n[u] = ej0[u] + (zj0[u] - ej0[u]) * p0.ke;
         zj_n[u] = zj0[u] * (1 - p0.kzj);
         bj_w[u] = kp != 0.0f;
-        if (bj_w[u]) bj_n[u] = p0.bgain * gsbn_logf(pj_n[u] + p0.eps);
+        if (bj_w[u]) bj_n[u] = p0.bgain * gsbn_logf_guarded(pj_n[u] + p0.eps);
       }
     }
   }
@@ -1301,14 +1302,14 @@ __device__ __forceinline__ void pop_body_w(const gsbn_pop_args& a, const PopStep
   }
 
   /* soft-max (Pop.cpp:280-302), the normaliser in ascending unit order */
-  const float maxact = gsbn_expf(a.wtagain * maxdsup);
+  const float maxact = gsbn_expf_guarded(a.wtagain * maxdsup);
   float act[UPL];
 #pragma unroll
   for (int u = 0; u < UPL; ++u) {
     const int j = lane + 64 * u;
     act[u] = 0.0f;
     if (j < M) {
-      act[u] = gsbn_expf(a.wtagain * (dsup[u] - maxdsup));
+      act[u] = gsbn_expf_guarded(a.wtagain * (dsup[u] - maxdsup));
       if (maxact < 1.0f) act[u] *= maxact;
       sh_f[j] = act[u];
     }
@@ -2284,13 +2285,13 @@ __global__ void device_math_kernel(int op, int64_t n, const uint32_t* in, uint32
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (op == 0) {
-      out[i] = gsbn_fbits(gsbn_expf(gsbn_bitsf(in[i])));
+      out[i] = gsbn_fbits(gsbn_expf_guarded(gsbn_bitsf(in[i])));
     } else if (op == 1) {
-      out[i] = gsbn_fbits(gsbn_logf(gsbn_bitsf(in[i])));
+      out[i] = gsbn_fbits(gsbn_logf_guarded(gsbn_bitsf(in[i])));
     } else if (op == 2) {
       float u, z;
       const uint64_t seed = (uint64_t)in[4 * i] | ((uint64_t)in[4 * i + 1] << 32);
-      gsbn_draw_unit(seed, 0u, in[4 * i + 2], in[4 * i + 3], &u, &z);
+      gsbn_draw_unit_guarded(seed, 0u, in[4 * i + 2], in[4 * i + 3], &u, &z);
       out[2 * i] = gsbn_fbits(u);
       out[2 * i + 1] = gsbn_fbits(z);
     } else if (op == 3) {

@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "../../include/gsbn_amd.h"
+#include "detfast.h"
 #include "detmath.h"
 #include "gsbn_core.h"
 #include "philox.h"
@@ -116,7 +117,7 @@ __global__ void __launch_bounds__(RE_THREADS_MAX) recall_step_kernel(ReArgs a, i
   float u = 0.0f, dsup = 0.0f, E = 0.0f;
   if (live) {
     float z;
-    gsbn_draw_unit(a.seed + (uint64_t)b, 0u, (uint32_t)t, (uint32_t)n, &u, &z);
+    gsbn_draw_unit_guarded(a.seed + (uint64_t)b, 0u, (uint32_t)t, (uint32_t)n, &u, &z);
     const float xi = a.snoise * z;
     E = a.epsc[bn];
     float wsup = 0.0f;
@@ -141,10 +142,10 @@ __global__ void __launch_bounds__(RE_THREADS_MAX) recall_step_kernel(ReArgs a, i
   }
   __syncthreads();
   /* soft-max (Pop.cpp:280-302) */
-  const float maxact = gsbn_expf(a.wtagain * maxdsup);
+  const float maxact = gsbn_expf_guarded(a.wtagain * maxdsup);
   float act = 0.0f;
   if (live) {
-    act = gsbn_expf(a.wtagain * (dsup - maxdsup));
+    act = gsbn_expf_guarded(a.wtagain * (dsup - maxdsup));
     if (maxact < 1.0f) act *= maxact;
     sh_f[j] = act;
   }
@@ -289,7 +290,7 @@ __global__ void __launch_bounds__(256) recall_pop_wave_kernel(ReArgs a, int t) {
       const float d0 = a.dsup[bn];
       if (t > a.count_from) cnt[i] = a.count[bn];
       float z;
-      gsbn_draw_unit(a.seed + (uint64_t)b, 0u, (uint32_t)t, (uint32_t)n, &u[i], &z);
+      gsbn_draw_unit_guarded(a.seed + (uint64_t)b, 0u, (uint32_t)t, (uint32_t)n, &u[i], &z);
       const float xi = a.snoise * z;
       float wsup = 0.0f;
       wsup += bjv + E;
@@ -312,13 +313,13 @@ __global__ void __launch_bounds__(256) recall_pop_wave_kernel(ReArgs a, int t) {
     }
   }
   /* soft-max (Pop.cpp:280-302) */
-  const float maxact = gsbn_expf(a.wtagain * maxdsup);
+  const float maxact = gsbn_expf_guarded(a.wtagain * maxdsup);
   float act[UPL];
 #pragma unroll
   for (int i = 0; i < UPL; ++i) {
     act[i] = 0.0f;
     if (lane + 64 * i < M) {
-      act[i] = gsbn_expf(a.wtagain * (dsup[i] - maxdsup));
+      act[i] = gsbn_expf_guarded(a.wtagain * (dsup[i] - maxdsup));
       if (maxact < 1.0f) act[i] *= maxact;
       row[lane + 64 * i] = act[i];
     }

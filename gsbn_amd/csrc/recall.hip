@@ -17,7 +17,8 @@
  * Pop.cpp:59), an empty delay queue and E = 0, and draws with Philox key
  * seed + b, population 0.
  *
- * Two support paths:
+ * Both modes run in recall_wave_kernel, several steps per launch, where it
+ * covers the population (see gsbn_recall_new).  Two support paths:
  *   exact  float weights, the additions in the reference's ascending row
  *          order: identical to a single-cue run of the solver (and the
  *          oracle) with the same weights;
@@ -77,7 +78,17 @@ struct ReArgs {
   uint16_t* S;            /* [RE_RING][B][Kp] bf16 0/1 (mfma) */
   const int16_t* clamp;   /* [B][H] */
   const float* wmask;     /* [B][H] */
-  int8_t* raster;         /* [B][N] spikes of the step, or NULL */
+  int8_t* raster;         /* spikes, [steps kept][B][N] from step raster_t0, or NULL */
+  /* the wave kernel (recall_wave_kernel) */
+  int R, L, raster_t0, Np;
+  float dsup0;
+  const int32_t* one;     /* [H][N] slot of a source in an HCU: -1 none, -2 several (exact) */
+  const uint16_t* Wb;     /* [H][N][M] bf16 weights by source (mfma) */
+  const uint16_t* WT;     /* [Np][Kp] bf16 weights by destination unit (mfma) */
+  int32_t* src_cnt;       /* [R][B] spikes of a step */
+  uint16_t* src_list;     /* [R][B][N] their units, in no order */
+  int32_t* out_idx;       /* [B][H] */
+  int32_t* out_cnt;
 };
 
 inline int ret(hipError_t e) { return e == hipSuccess ? 0 : (int)e; }
@@ -344,6 +355,397 @@ __global__ void __launch_bounds__(256) recall_pop_wave_kernel(ReArgs a, int t) {
   }
 }
 
+#define RW_WAVES 4 /* cues per workgroup of recall_wave_kernel */
+
+/* LDS operations of a wave are processed in order; this only keeps the
+ * compiler from moving them across */
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+/* acc[u] (unit lane + 64 u) += W's 16-source block `blk`, sources of `bits`,
+ * by the matrix instruction of spike_gemm_kernel on the same operands: rows 0
+ * and 4 of the A block hold the cue, so accumulator 0 of a lane (row 0 for
+ * lanes 0-31, row 4 for lanes 32-63) is that lane's unit of the column block.
+ * Called by whole waves. */
+template <int UPL>
+__device__ __forceinline__ void add_block_mfma(const ReArgs& a, int h, int blk, uint32_t bits,
+                                               int lane, float* acc) {
+  union {
+    gsbn_bf16x8 v;
+    uint16_t u[8];
+  } A;
+  const uint32_t mine = (lane & 27) == 0 ? (bits >> ((lane >> 5) * 8)) & 0xffu : 0u;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) A.u[q] = ((mine >> q) & 1u) ? (uint16_t)0x3F80u : (uint16_t)0u;
+#pragma unroll
+  for (int u = 0; u < UPL; ++u) {
+    float r[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      int n = h * a.M + 64 * u + 32 * c + (lane & 31);
+      n = n < a.Np ? n : a.Np - 1;
+      const gsbn_bf16x8 B = *reinterpret_cast<const gsbn_bf16x8*>(
+          a.WT + (int64_t)n * a.Kp + blk * 16 + (lane >> 5) * 8);
+      gsbn_f32x16 C;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) C[q] = 0.0f;
+      C[0] = acc[u];
+      C = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v, B, C, 0, 0, 0);
+      r[c] = C[0];
+      /* one block's accumulators at a time */
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    acc[u] = lane < 32 ? r[0] : r[1];
+  }
+}
+
+/* Steps t0 .. t0 + nt - 1 of the recall, one wave per (HCU, cue), UPL units
+ * per lane.  A row active at t has a source that spiked at t - di - 2, so
+ * the steps of a run of L = dmin + 2 read only spikes of earlier launches:
+ * a wave keeps its pair's state in registers for L steps.  Per step: the
+ * population update (Pop.cpp:229-323), the spikes appended to the cue's list
+ * of the step, and the support update from the cue's list of step t - d - 2:
+ * its sources' rows sorted by rank (at most 64; more, or several delays or
+ * slots per source, go through bitmap windows), weights read row by row.
+ *   exact: E = E (1 - kepsc), then + Wij of each row in ascending row order.
+ *   mfma (BF): E = E (1 - kepsc) + SW, SW with the bits of the dense product:
+ *   that product adds, 16 sources at a time, mostly zeros, which change
+ *   nothing; where every sum of the nonzero terms is exact (one term per
+ *   block, s - a == b and s - b == a) its value is the float sum, and
+ *   otherwise the nonzero blocks go through the same matrix instruction.
+ *
+ * What bounds it: issue (Philox and the double sequences of the draw and the
+ * soft-max): 630 vector instructions per step of up to 128 units, the vector
+ * units 77 % busy.  Hence one wave per
+ * pair without idle waves, the normalisers of a workgroup's pairs summed by
+ * as many lanes at once (100 dependent additions for one lane would
+ * be 400 issue cycles per pair), and the maximum's exponential evaluated by
+ * the lane that holds the maximum, whose own is 1.  Workgroup i runs on XCD
+ * i % 8: an XCD takes one HCU at a time for all cues, so that the HCU's
+ * weights (4 MB at 100 x 100) stay in its L2.  Four waves per workgroup and
+ * six waves per SIMD for exact (eight and four: 68.5 ms); the mfma form's
+ * accumulators hold it at four.
+ * 8192 cues x 50 steps at 100 x 100: exact 54.5 ms (a workgroup per pair and
+ * one step per launch: 106.8 ms), mfma 68.2 ms (dense product 75 ms and
+ * population step 43 ms: 120 ms); one cue at 10 x 10: 0.23 ms (0.94 ms). */
+template <int UPL, bool BF>
+__global__ void __launch_bounds__(64 * RW_WAVES, BF ? (UPL == 1 ? 5 : UPL == 2 ? 4 : 3) : UPL <= 2 ? 6 : 4)
+    recall_wave_kernel(ReArgs a, int t0, int nt, int last) {
+  __shared__ __attribute__((aligned(16))) float sh_act[RW_WAVES][64 * UPL + 4];
+  __shared__ float sh_sum[RW_WAVES];
+  __shared__ uint32_t sh_bm[RW_WAVES][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int nb8 = (a.B + RW_WAVES - 1) / RW_WAVES;
+  const int xcd = blockIdx.x & 7, bi = blockIdx.x >> 3;
+  const int h = xcd + 8 * (bi / nb8);
+  if (h >= a.H) return; /* the whole workgroup */
+  const int b = (bi % nb8) * RW_WAVES + wave;
+  const bool on = b < a.B; /* uniform per wave; the others only meet the barriers */
+  const int M = a.M, N = a.N, B = a.B;
+  const int64_t pair = (int64_t)b * a.H + h;
+  const int64_t bn0 = (int64_t)b * N + (int64_t)h * M;
+
+  float dsup[UPL], E[UPL], bjv[UPL];
+  int cnt[UPL];
+  int cl = -1;
+  float wm = 0.0f;
+  if (on) {
+    cl = a.clamp[pair];
+    wm = a.wmask[pair];
+#pragma unroll
+    for (int i = 0; i < UPL; ++i) {
+      const int j = lane + 64 * i;
+      dsup[i] = a.dsup0;
+      E[i] = 0.0f;
+      cnt[i] = 0;
+      bjv[i] = 0.0f;
+      if (j < M) {
+        bjv[i] = a.bj[h * M + j];
+        if (t0 > 1) {
+          dsup[i] = a.dsup[bn0 + j];
+          E[i] = a.epsc[bn0 + j];
+          cnt[i] = a.count[bn0 + j];
+        }
+      }
+    }
+    /* the counters of the next launch's steps (their slots' previous steps
+     * are no longer read) */
+    if (h == 0 && lane < a.L) a.src_cnt[(int64_t)((t0 + nt + lane) % a.R) * B + b] = 0;
+  }
+  const bool single = a.dmin == a.dmax;
+
+  for (int t = t0; t < t0 + nt; ++t) {
+    /* the sources active at t and their rows, looked up before the draws */
+    int nsrc = 0, key = -1;
+    bool general = false;
+    if (on && single) {
+      const int s = t - a.dmin - 2;
+      if (s >= 1) {
+        const int64_t sb = (int64_t)(s % a.R) * B + b;
+        nsrc = __builtin_amdgcn_readfirstlane(a.src_cnt[sb]);
+        general = nsrc > 64;
+        if (!general && lane < nsrc) {
+          const int src = a.src_list[sb * N + lane];
+          key = BF ? src : a.one[(int64_t)h * N + src];
+        }
+      }
+    } else if (on) {
+      general = a.dmax > 0;
+    }
+    float u[UPL], act[UPL];
+    if (on) {
+      /* support, dsup (Pop.cpp:229-261) */
+#pragma unroll
+      for (int i = 0; i < UPL; ++i) {
+        const int j = lane + 64 * i;
+        float z;
+        gsbn_draw_unit_guarded(a.seed + (uint64_t)b, 0u, (uint32_t)t, (uint32_t)(h * M + j), &u[i], &z);
+        const float xi = a.snoise * z;
+        float wsup = 0.0f;
+        wsup += bjv[i] + E[i];
+        const float lginp = cl == j ? a.lg_on : a.lg_off;
+        float sup = a.lgbias + a.igain * lginp + xi;
+        sup += (a.wgain * wm) * wsup;
+        dsup[i] = dsup[i] + (sup - dsup[i]) * a.taumdt;
+      }
+      /* WTA maximum: each 64-unit range by a wave scan, left to right */
+      float maxdsup = 0.0f;
+#pragma unroll
+      for (int i = 0; i < UPL; ++i) {
+        const float mv = wave_max_left(lane + 64 * i < M ? dsup[i] : -INFINITY);
+        if (i == 0) {
+          maxdsup = mv;
+        } else if (64 * i < M && mv > maxdsup) {
+          maxdsup = mv;
+        }
+      }
+      /* soft-max (Pop.cpp:280-302).  exp(wtagain * maxdsup) comes from a lane
+       * whose dsup is the maximum (its own activity is exp(0) = 1); without
+       * one (NaN), or with an infinite gain, it is evaluated by itself */
+      const float xmax = a.wtagain * maxdsup;
+      float maxact = 0.0f;
+      bool have = false;
+#pragma unroll
+      for (int i = 0; i < UPL; ++i) {
+        const float diff = dsup[i] - maxdsup;
+        const bool top = lane + 64 * i < M && diff == 0.0f && a.wtagain * diff == 0.0f;
+        const float e = gsbn_expf_guarded(top ? xmax : a.wtagain * diff);
+        act[i] = top ? 1.0f : e;
+        const uint64_t tb = __ballot(top);
+        if (tb && !have) {
+          maxact = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), __builtin_ctzll(tb)));
+          have = true;
+        }
+      }
+      if (!have) maxact = gsbn_expf_guarded(xmax);
+#pragma unroll
+      for (int i = 0; i < UPL; ++i) {
+        if (maxact < 1.0f) act[i] *= maxact;
+        sh_act[wave][lane + 64 * i] = act[i];
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < RW_WAVES) sh_sum[threadIdx.x] = ordered_sum_lds(sh_act[threadIdx.x], M);
+    __syncthreads();
+    if (!on) continue;
+    const float vsum = sh_sum[wave];
+    /* spikes (Pop.cpp:305-323), appended to the cue's list of this step */
+    int spk[UPL], tot = 0, before[UPL];
+#pragma unroll
+    for (int i = 0; i < UPL; ++i) {
+      const int j = lane + 64 * i;
+      float ac = act[i];
+      if (vsum > 1.0f) ac /= vsum;
+      spk[i] = (j < M && u[i] < ac * a.maxfqdt) ? 1 : 0;
+      const uint64_t bal = __ballot(spk[i]);
+      before[i] = tot + __popcll(bal & ((1ull << lane) - 1ull));
+      tot += __popcll(bal);
+      if (t > a.count_from) cnt[i] += spk[i];
+      if (a.raster && j < M) a.raster[(int64_t)(t - a.raster_t0) * B * N + bn0 + j] = (int8_t)spk[i];
+    }
+    if (tot) {
+      const int64_t sb = (int64_t)(t % a.R) * B + b;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&a.src_cnt[sb], tot);
+      base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+      for (int i = 0; i < UPL; ++i)
+        if (spk[i]) a.src_list[sb * N + base + before[i]] = (uint16_t)(h * M + lane + 64 * i);
+    }
+    /* support update */
+    float e[UPL];
+#pragma unroll
+    for (int i = 0; i < UPL; ++i) e[i] = BF ? 0.0f : E[i] * (1 - a.kepsc);
+    if (!BF && __ballot(key == -2)) general = true;
+    if (!general) {
+      const uint64_t m = __ballot(key >= 0);
+      const int nk = __popcll(m);
+      if (nk) {
+        /* ascending keys: lane r holds the r-th */
+        int rank = 0;
+        for (uint64_t mm = m; mm; mm &= mm - 1)
+          rank += __builtin_amdgcn_readlane(key, __builtin_ctzll(mm)) < key;
+        if (key < 0) rank = nk + __popcll(~m & ((1ull << lane) - 1ull));
+        const int ks = __builtin_amdgcn_ds_permute(rank << 2, key);
+        bool exactly = true;
+        if (BF) {
+          const int nx = __builtin_amdgcn_ds_bpermute(((lane + 1) & 63) << 2, ks);
+          if (__ballot(lane + 1 < nk && (nx >> 4) == (ks >> 4))) exactly = false;
+        }
+        if (exactly) {
+          bool off = false;
+          const int64_t hrow = (int64_t)h * (BF ? N : a.C);
+          constexpr int G = UPL <= 2 ? 8 : 4;
+          for (int r = 0; r < nk; r += G) {
+            float v[G][UPL];
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+              const int k = __builtin_amdgcn_readlane(ks, r + q < nk ? r + q : nk - 1);
+              const int64_t at = (hrow + k) * M;
+#pragma unroll
+              for (int i = 0; i < UPL; ++i) {
+                int j = lane + 64 * i;
+                j = j < M ? j : M - 1;
+                v[q][i] = BF ? __uint_as_float((uint32_t)a.Wb[at + j] << 16) : a.wij[at + j];
+              }
+            }
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+              if (r + q < nk) {
+#pragma unroll
+                for (int i = 0; i < UPL; ++i) {
+                  const float s = e[i] + v[q][i];
+                  if (BF) off = off || !(s - e[i] == v[q][i] && s - v[q][i] == e[i]);
+                  e[i] = s;
+                }
+              }
+            }
+          }
+          if (BF && __ballot(off)) exactly = false;
+        }
+        if (BF && !exactly) {
+#pragma unroll
+          for (int i = 0; i < UPL; ++i) e[i] = 0.0f;
+          for (int r = 0; r < nk;) {
+            const int blk = __builtin_amdgcn_readlane(ks, r) >> 4;
+            uint32_t bits = 0;
+            int k;
+            while (r < nk && ((k = __builtin_amdgcn_readlane(ks, r)) >> 4) == blk) {
+              bits |= 1u << (k & 15);
+              ++r;
+            }
+            add_block_mfma<UPL>(a, h, blk, bits, lane, e);
+          }
+        }
+      }
+    } else {
+      /* any number of rows: windows of 2048 keys (slots, or sources) */
+      const int span = BF ? N : a.C;
+      for (int w0 = 0; w0 < span; w0 += 2048) {
+        sh_bm[wave][lane] = 0u;
+        wave_lds_fence();
+        for (int d = a.dmin; d <= a.dmax; ++d) {
+          const int s = t - d - 2;
+          if (s < 1) break;
+          const int64_t sb = (int64_t)(s % a.R) * B + b;
+          const int n = __builtin_amdgcn_readfirstlane(a.src_cnt[sb]);
+          for (int i = lane; i < n; i += 64) {
+            const int src = a.src_list[sb * N + i];
+            if (BF) {
+              const int k = src - w0;
+              if (k >= 0 && k < 2048) atomicOr(&sh_bm[wave][k >> 5], 1u << (k & 31));
+            } else {
+              const int32_t* off = a.inv_off + (int64_t)h * (N + 1);
+              for (int q = off[src]; q < off[src + 1]; ++q) {
+                const int slot = a.inv_slot[q], k = slot - w0;
+                if (k >= 0 && k < 2048 && a.di[(int64_t)h * a.C + slot] == d)
+                  atomicOr(&sh_bm[wave][k >> 5], 1u << (k & 31));
+              }
+            }
+          }
+        }
+        wave_lds_fence();
+        const int word = (int)sh_bm[wave][lane];
+        wave_lds_fence();
+        for (uint64_t nz = __ballot(word != 0); nz; nz &= nz - 1) {
+          const int l = __builtin_ctzll(nz);
+          uint32_t bits = (uint32_t)__builtin_amdgcn_readlane(word, l);
+          const int k0 = w0 + 32 * l;
+          if (BF) {
+            if (bits & 0xffffu) add_block_mfma<UPL>(a, h, k0 >> 4, bits & 0xffffu, lane, e);
+            if (bits >> 16) add_block_mfma<UPL>(a, h, (k0 >> 4) + 1, bits >> 16, lane, e);
+          } else {
+            while (bits) {
+              const int64_t at = ((int64_t)h * a.C + k0 + __builtin_ctz(bits)) * M;
+              bits &= bits - 1;
+#pragma unroll
+              for (int i = 0; i < UPL; ++i) {
+                const int j = lane + 64 * i;
+                e[i] = e[i] + a.wij[at + (j < M ? j : M - 1)];
+              }
+            }
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < UPL; ++i) E[i] = BF ? (1 - a.kepsc) * E[i] + e[i] : e[i];
+  }
+  if (!on) return;
+  if (!last) {
+#pragma unroll
+    for (int i = 0; i < UPL; ++i) {
+      const int j = lane + 64 * i;
+      if (j < M) {
+        a.dsup[bn0 + j] = dsup[i];
+        a.epsc[bn0 + j] = E[i];
+        a.count[bn0 + j] = cnt[i];
+      }
+    }
+    return;
+  }
+  /* first strict maximum of the counts (ProcCheck/Pop.cpp:35-50) */
+  int mc = 0;
+#pragma unroll
+  for (int i = 0; i < UPL; ++i) mc = max(mc, lane + 64 * i < M ? cnt[i] : 0);
+  for (int o = 32; o; o >>= 1) mc = max(mc, __shfl_xor(mc, o));
+  int mi = -1;
+#pragma unroll
+  for (int i = 0; i < UPL; ++i) {
+    const uint64_t bal = __ballot(lane + 64 * i < M && cnt[i] == mc);
+    if (mi < 0 && mc > 0 && bal) mi = 64 * i + __builtin_ctzll(bal);
+  }
+  if (lane == 0) {
+    a.out_idx[pair] = mi;
+    a.out_cnt[pair] = mc;
+  }
+}
+
+/* bf16 weights of the mfma mode from the float weights: one workgroup per
+ * (HCU, source), the source's slots summed in double in ascending order
+ * (CSR), stored by source (Wb, where given) and by destination unit (WT);
+ * *nonfinite is set when one is infinite or NaN. */
+__global__ void recall_weights_kernel(int H, int M, int C, int N, int Kp, const float* wij,
+                                      const int32_t* inv_off, const int32_t* inv_slot, uint16_t* Wb,
+                                      uint16_t* WT, int32_t* nonfinite) {
+  const int src = blockIdx.x;
+  for (int h = blockIdx.y; h < H; h += gridDim.y) {
+    const int32_t* off = inv_off + (int64_t)h * (N + 1);
+    const int q0 = off[src], q1 = off[src + 1];
+    for (int j = threadIdx.x; j < M; j += blockDim.x) {
+      double acc = 0.0;
+      for (int q = q0; q < q1; ++q)
+        acc += (double)wij[((int64_t)h * C + inv_slot[q]) * M + j];
+      const uint16_t v = gsbn_f32_to_bf16((float)acc);
+      if ((v & 0x7f80u) == 0x7f80u) *nonfinite = 1;
+      if (Wb) Wb[((int64_t)h * N + src) * M + j] = v;
+      WT[((int64_t)h * M + j) * Kp + src] = v;
+    }
+  }
+}
+
 /* E[b][n] = beta E[b][n] + sum_k S[b][k] WT[n][k]: bf16 inputs, float
  * accumulation on v_mfma_f32_32x32x16_bf16.  S and WT have Kp columns (Kp a
  * multiple of GM_BK, zero padded); S has ceil(B / GM_BM) * GM_BM rows and WT
@@ -507,6 +909,8 @@ struct DBuf {
     if (p) (void)hipFree(p);
   }
   hipError_t alloc(size_t count) {
+    if (p) (void)hipFree(p);
+    p = nullptr;
     n = count;
     return count ? hipMalloc(&p, count * sizeof(T)) : hipSuccess;
   }
@@ -522,9 +926,11 @@ struct DBuf {
 struct gsbn_recall {
   gsbn_recall_desc d;
   int N = 0, Kp = 0, Np = 0, Bp = 0, W = 0, dmin = 1, dmax = 0, delay = 0;
+  int R = 0, L = 0;
+  bool wave = false; /* recall_wave_kernel covers this population */
   DBuf<float> dsup, epsc, bj, wij;
-  DBuf<int32_t> count, di, inv_off, inv_slot, spk_cnt, out_idx, out_cnt;
-  DBuf<uint16_t> spk_list, S, WT;
+  DBuf<int32_t> count, di, inv_off, inv_slot, spk_cnt, out_idx, out_cnt, one, src_cnt;
+  DBuf<uint16_t> spk_list, S, WT, Wb, src_list;
   DBuf<int16_t> clamp;
   DBuf<float> wmask;
   DBuf<int8_t> raster;
@@ -623,30 +1029,76 @@ gsbn_recall* gsbn_recall_new(const gsbn_recall_desc* d) {
   ok(r->out_cnt.alloc((size_t)B * H));
   ok(r->clamp.alloc((size_t)B * H));
   ok(r->wmask.alloc((size_t)B * H));
+  /* one wave per (HCU, cue) up to 256 units and 65536 sources (its lists hold
+   * 16-bit units); the workgroup-per-pair kernels take larger populations */
+  r->wave = M <= 256 && N <= 65536;
+  r->L = std::min(dmin + 2, 8);
+  r->R = std::max(dmax, dmin) + 2 + 2 * r->L;
   if (d->mode == GSBN_RECALL_EXACT) {
     ok(r->wij.upload(d->wij, (size_t)(R * M)));
     ok(r->di.upload(d->di, (size_t)R));
     ok(r->inv_off.upload(off.data(), off.size()));
     ok(r->inv_slot.upload(slots.data(), slots.size()));
-    ok(r->spk_cnt.alloc((size_t)RE_RING * B * H));
-    ok(r->spk_list.alloc((size_t)RE_RING * B * N));
+    if (r->wave) {
+      std::vector<int32_t> one((size_t)H * N);
+      for (int h = 0; h < H; ++h) {
+        const int32_t* o = off.data() + (size_t)h * (N + 1);
+        for (int n = 0; n < N; ++n)
+          one[(size_t)h * N + n] =
+              o[n + 1] == o[n] ? -1 : o[n + 1] == o[n] + 1 ? slots[(size_t)o[n]] : -2;
+      }
+      ok(r->one.upload(one.data(), one.size()));
+    } else {
+      ok(r->spk_cnt.alloc((size_t)RE_RING * B * H));
+      ok(r->spk_list.alloc((size_t)RE_RING * B * N));
+    }
   } else {
-    /* dense W^T [n][src] in bf16: the rows of HCU h(n) whose source is src */
+    /* dense W in bf16, by destination unit (WT, for the product) and by
+     * source (Wb, for the wave kernel), from the slots of each source */
     r->Kp = (N + GM_BK - 1) / GM_BK * GM_BK;
     r->Np = (N + GM_BN - 1) / GM_BN * GM_BN;
-    std::vector<double> acc((size_t)r->Np * r->Kp, 0.0);
-    for (int h = 0; h < H; ++h)
-      for (int k = 0; k < C; ++k) {
-        const int s = d->ii[(int64_t)h * C + k];
-        if (s < 0) continue;
-        for (int j = 0; j < M; ++j)
-          acc[(size_t)(h * M + j) * r->Kp + s] += (double)d->wij[((int64_t)h * C + k) * M + j];
-      }
-    std::vector<uint16_t> wt(acc.size());
-    for (size_t i = 0; i < acc.size(); ++i) wt[i] = gsbn_f32_to_bf16((float)acc[i]);
-    ok(r->WT.upload(wt.data(), wt.size()));
     r->Bp = (B + GM_BM - 1) / GM_BM * GM_BM;
-    ok(r->S.alloc((size_t)RE_RING * r->Bp * r->Kp));
+    /* The dense product costs 2 M N flops per pair and step whatever spikes;
+     * the wave kernel only its population step and the active rows.  Measured
+     * per pair and step, product with its population step against the wave
+     * kernel: 3.0 / 1.6 ns at 100 x 100 (8192 cues), 3.3 / 1.7 at 40 x 128,
+     * 0.72 / 0.80 at 60 x 20 and 0.81 / 0.89 at 180 x 12, where the product
+     * is small and the leaner population step of its path wins: the line is
+     * at M N = 60000.  Below it small batches still gain, because the wave
+     * kernel takes L steps per launch instead of two launches per step
+     * (about 4 us a step, 0.1 ns for each of 40000 pairs).  The rates hold up
+     * to one active source per two hypercolumns and step (6.06 ms for 20
+     * steps of 2048 cues at maxfq dt = 0.5 against 5.86 at 0.1); a
+     * hypercolumn's activities sum to at most 1, so maxfq dt bounds them. */
+    if (!(d->maxfqdt <= 0.5f) ||
+        ((int64_t)M * N < 60000 && (int64_t)B * H >= 40000))
+      r->wave = false;
+    DBuf<float> w;
+    DBuf<int32_t> o, sl, bad;
+    const int32_t zero = 0;
+    ok(w.upload(d->wij, (size_t)(R * M)));
+    ok(o.upload(off.data(), off.size()));
+    ok(sl.upload(slots.data(), slots.size()));
+    ok(bad.upload(&zero, 1));
+    if (r->wave) ok(r->Wb.alloc((size_t)H * N * M));
+    ok(r->WT.alloc((size_t)r->Np * r->Kp));
+    if (e == hipSuccess) {
+      const int64_t nw = (int64_t)r->Np * r->Kp / 2;
+      hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(nw)), dim3(256), 0, 0,
+                         reinterpret_cast<float*>(r->WT.p), nw, 0.0f);
+      hipLaunchKernelGGL(recall_weights_kernel, dim3(N, std::min(H, 65535)), dim3(M <= 64 ? 64 : 128), 0, 0, H, M, C, N,
+                         r->Kp, w.p, o.p, sl.p, r->Wb.p, r->WT.p, bad.p);
+      ok(hipGetLastError());
+      int32_t nonfinite = 0;
+      ok(hipMemcpy(&nonfinite, bad.p, sizeof(nonfinite), hipMemcpyDeviceToHost));
+      /* an infinite or NaN weight reaches every cue through the product's
+       * zeros; only the dense product has that */
+      if (nonfinite) r->wave = false;
+    }
+  }
+  if (r->wave) {
+    ok(r->src_cnt.alloc((size_t)r->R * B));
+    ok(r->src_list.alloc((size_t)r->R * B * N));
   }
   ok(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
   ok(hipEventCreate(&r->ev0));
@@ -656,6 +1108,67 @@ gsbn_recall* gsbn_recall_new(const gsbn_recall_desc* d) {
 }
 
 void gsbn_recall_free(gsbn_recall* r) { delete r; }
+
+}  // extern "C"
+
+namespace {
+
+/* the run by recall_wave_kernel, L steps per launch */
+int run_wave(gsbn_recall* r, ReArgs a, int steps, int8_t* raster) {
+  hipStream_t s = r->stream;
+  const gsbn_recall_desc& d = r->d;
+  const int B = d.batch;
+  const int64_t BN = (int64_t)B * r->N, nc = (int64_t)r->R * B;
+  hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(nc)), dim3(256), 0, s,
+                     reinterpret_cast<float*>(r->src_cnt.p), nc, 0.0f);
+  /* raster steps kept on the device before a copy to the host */
+  int64_t keep = 0;
+  if (raster) {
+    keep = std::min<int64_t>(steps, std::max<int64_t>(1, ((int64_t)256 << 20) / BN));
+    if ((int64_t)r->raster.n < keep * BN) {
+      const hipError_t e = r->raster.alloc((size_t)(keep * BN));
+      if (e != hipSuccess) return fail((int)e, "gsbn_recall_run: raster buffer");
+    }
+    a.raster = r->raster.p;
+  }
+  a.raster_t0 = 1;
+  const int upl = (d.M + 63) / 64;
+  const dim3 grid((unsigned)(8 * ((d.H + 7) / 8) * ((B + RW_WAVES - 1) / RW_WAVES)));
+  const dim3 block(64 * RW_WAVES);
+  const bool bf = d.mode == GSBN_RECALL_MFMA;
+  for (int t = 1; t <= steps;) {
+    int nt = std::min(r->L, steps - t + 1);
+    if (raster) nt = (int)std::min<int64_t>(nt, a.raster_t0 + keep - t);
+    const int last = t + nt > steps ? 1 : 0;
+#define RW_LAUNCH(U, F) \
+  hipLaunchKernelGGL((recall_wave_kernel<U, F>), grid, block, 0, s, a, t, nt, last)
+    if (upl == 1) {
+      if (bf) RW_LAUNCH(1, true);
+      else RW_LAUNCH(1, false);
+    } else if (upl == 2) {
+      if (bf) RW_LAUNCH(2, true);
+      else RW_LAUNCH(2, false);
+    } else {
+      if (bf) RW_LAUNCH(4, true);
+      else RW_LAUNCH(4, false);
+    }
+#undef RW_LAUNCH
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail((int)e, "recall_wave_kernel");
+    t += nt;
+    if (raster && (t > steps || t == a.raster_t0 + keep)) {
+      e = hipMemcpyAsync(raster + (int64_t)(a.raster_t0 - 1) * BN, r->raster.p,
+                         (size_t)((t - a.raster_t0) * BN), hipMemcpyDeviceToHost, s);
+      if (e != hipSuccess) return fail((int)e, "gsbn_recall_run: raster");
+      a.raster_t0 = t;
+    }
+  }
+  return 0;
+}
+
+}  // namespace
+
+extern "C" {
 
 int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, int32_t steps,
                     int32_t count_from, int32_t* out_idx, int32_t* out_cnt, int8_t* raster,
@@ -670,24 +1183,34 @@ int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, in
   if (e == hipSuccess)
     e = hipMemcpyAsync(r->wmask.p, wmask, (size_t)B * H * 4, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return fail((int)e, "gsbn_recall_run: upload");
+  /* the product's time is wanted: one product per step, as below */
+  const bool wave = r->wave && steps > 0 && !(support_ms && d.mode == GSBN_RECALL_MFMA);
   /* initial state: dsup = log(1/M) (Pop.cpp:59), E = 0, counts 0, empty queue */
   const float dsup0 = (float)log(1.0 / M);
-  hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(BN)), dim3(256), 0, s, r->dsup.p, BN, dsup0);
-  hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(BN)), dim3(256), 0, s, r->epsc.p, BN, 0.0f);
-  hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(BN)), dim3(256), 0, s,
-                     reinterpret_cast<float*>(r->count.p), BN, 0.0f);
-  if (d.mode == GSBN_RECALL_EXACT) {
-    const int64_t nc = (int64_t)RE_RING * B * H;
-    hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(nc)), dim3(256), 0, s,
-                       reinterpret_cast<float*>(r->spk_cnt.p), nc, 0.0f);
-  } else {
-    const int64_t ns = (int64_t)RE_RING * r->Bp * r->Kp / 2;
-    hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(ns)), dim3(256), 0, s,
-                       reinterpret_cast<float*>(r->S.p), ns, 0.0f);
-  }
-  if (raster && !r->raster.p) {
-    e = r->raster.alloc((size_t)BN);
-    if (e != hipSuccess) return fail((int)e, "gsbn_recall_run: raster buffer");
+  if (!wave) {
+    hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(BN)), dim3(256), 0, s, r->dsup.p, BN, dsup0);
+    hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(BN)), dim3(256), 0, s, r->epsc.p, BN, 0.0f);
+    hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(BN)), dim3(256), 0, s,
+                       reinterpret_cast<float*>(r->count.p), BN, 0.0f);
+    if (d.mode == GSBN_RECALL_EXACT) {
+      if (!r->spk_cnt.p) {
+        /* no steps: the lists are not used */
+      } else {
+        const int64_t nc = (int64_t)RE_RING * B * H;
+        hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(nc)), dim3(256), 0, s,
+                           reinterpret_cast<float*>(r->spk_cnt.p), nc, 0.0f);
+      }
+    } else {
+      const int64_t ns = (int64_t)RE_RING * r->Bp * r->Kp;
+      if (!r->S.p && (e = r->S.alloc((size_t)ns)) != hipSuccess)
+        return fail((int)e, "gsbn_recall_run: spike matrices");
+      hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(ns / 2)), dim3(256), 0, s,
+                         reinterpret_cast<float*>(r->S.p), ns / 2, 0.0f);
+    }
+    if (raster && (int64_t)r->raster.n < BN) {
+      e = r->raster.alloc((size_t)BN);
+      if (e != hipSuccess) return fail((int)e, "gsbn_recall_run: raster buffer");
+    }
   }
   ReArgs a;
   memset(&a, 0, sizeof(a));
@@ -728,6 +1251,21 @@ int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, in
   a.clamp = r->clamp.p;
   a.wmask = r->wmask.p;
   a.raster = raster ? r->raster.p : nullptr;
+  a.R = r->R;
+  a.L = r->L;
+  a.Np = r->Np;
+  a.dsup0 = dsup0;
+  a.one = r->one.p;
+  a.Wb = r->Wb.p;
+  a.WT = r->WT.p;
+  a.src_cnt = r->src_cnt.p;
+  a.src_list = r->src_list.p;
+  a.out_idx = r->out_idx.p;
+  a.out_cnt = r->out_cnt.p;
+  if (wave) {
+    const int rc = run_wave(r, a, steps, raster);
+    if (rc) return rc;
+  }
   const int threads = ((M + 63) / 64) * 64;
   const size_t lds = d.mode == GSBN_RECALL_EXACT ? ((size_t)r->W + RE_ROWS_MAX) * 4 : 0;
   const float beta = 1 - d.kepsc;
@@ -736,7 +1274,7 @@ int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, in
   const int upl = (M + 63) / 64;
   const bool wave_step = d.mode == GSBN_RECALL_MFMA && upl <= 4;
   const unsigned wave_grid = (unsigned)(((int64_t)B * H + 3) / 4);
-  for (int t = 1; t <= steps; ++t) {
+  for (int t = 1; !wave && t <= steps; ++t) {
     if (wave_step) {
       if (upl == 1)
         hipLaunchKernelGGL(recall_pop_wave_kernel<1>, dim3(wave_grid), dim3(256), 0, s, a, t);
@@ -775,8 +1313,9 @@ int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, in
     }
   }
   const int64_t BH = (int64_t)B * H;
-  hipLaunchKernelGGL(recall_argmax_kernel, dim3(grid_of(BH)), dim3(256), 0, s, B, H, M, r->count.p,
-                     r->out_idx.p, r->out_cnt.p);
+  if (!wave)
+    hipLaunchKernelGGL(recall_argmax_kernel, dim3(grid_of(BH)), dim3(256), 0, s, B, H, M,
+                       r->count.p, r->out_idx.p, r->out_cnt.p);
   e = hipMemcpyAsync(out_idx, r->out_idx.p, (size_t)BH * 4, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess)
     e = hipMemcpyAsync(out_cnt, r->out_cnt.p, (size_t)BH * 4, hipMemcpyDeviceToHost, s);

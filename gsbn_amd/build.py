@@ -56,7 +56,7 @@ def build(verbose: bool = False) -> str:
                 print(o)
     tmp = LIB + ".tmp"
     _run([HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", tmp] + [o for _, o in jobs]
-         + ["-L" + os.path.join(ROCM, "lib"), "-lamdhip64"])
+         + ["-L" + os.path.join(ROCM, "lib"), "-lamdhip64", "-lpthread"])
     os.replace(tmp, LIB)
     return LIB
 

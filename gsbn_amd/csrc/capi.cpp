@@ -72,7 +72,7 @@ int gsbn_solver_snapshot(gsbn_solver* s, const char* path) {
     glv.geti("simstep", simstep);
     glv.getf("dt", dt);
     glv.getf("prn", prn);
-    gsbn::active_stream() = s->s->stream();
+    s->s->activate();
     s->s->db().save_state(path, simstep * dt, prn);
     return 0;
   });
@@ -155,6 +155,7 @@ gsbn_solver* gsbn_solver_new(const char* net_path, const char* snapshot_path) {
       gsbn::hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     } catch (...) {
       delete h;
+      gsbn::active_memory() = nullptr; /* was the failed solver's */
       throw;
     }
     return h;
@@ -203,7 +204,7 @@ int gsbn_solver_sync(gsbn_solver* s) {
 int64_t gsbn_solver_vector_info(gsbn_solver* s, const char* name, int* dtype) {
   try {
     if (!s || !s->s || !name) throw Error(GSBN_ERR_ARG, "null argument");
-    gsbn::active_stream() = s->s->stream(); /* host copies sync on this solver's stream */
+    s->s->activate(); /* host copies sync on this solver's stream */
     gsbn::VecBase* v = s->s->db().find(name);
     if (!v) throw Error(GSBN_ERR_NAME, std::string("no vector named ") + name);
     if (dynamic_size(name)) (void)v->host_ptr_sync();
@@ -217,9 +218,15 @@ int64_t gsbn_solver_vector_info(gsbn_solver* s, const char* name, int* dtype) {
 int64_t gsbn_solver_vector_read(gsbn_solver* s, const char* name, void* out, int64_t cap) {
   try {
     if (!s || !s->s || !name) throw Error(GSBN_ERR_ARG, "null argument");
-    gsbn::active_stream() = s->s->stream(); /* host copies sync on this solver's stream */
+    s->s->activate(); /* host copies sync on this solver's stream */
     gsbn::VecBase* v = s->s->db().find(name);
     if (!v) throw Error(GSBN_ERR_NAME, std::string("no vector named ") + name);
+    /* a large vector read whole goes from the device to the caller's memory
+     * without a host copy of its own (which small ones keep: procedures and
+     * later reads share it) */
+    if (out && !dynamic_size(name) && cap >= (int64_t)v->size() &&
+        v->size() * v->elem_size() >= ((size_t)1 << 20) && v->read_device(out))
+      return (int64_t)v->size();
     void* p = v->host_ptr_sync();
     int64_t n = (int64_t)v->size();
     if (out && cap > 0 && n > 0) memcpy(out, p, (size_t)std::min(n, cap) * v->elem_size());
@@ -232,7 +239,7 @@ int64_t gsbn_solver_vector_read(gsbn_solver* s, const char* name, void* out, int
 int gsbn_solver_vector_write(gsbn_solver* s, const char* name, const void* in, int64_t count) {
   return guard([&] {
     if (!s || !s->s || !name || (!in && count)) throw Error(GSBN_ERR_ARG, "null argument");
-    gsbn::active_stream() = s->s->stream(); /* host copies sync on this solver's stream */
+    s->s->activate(); /* host copies sync on this solver's stream */
     gsbn::VecBase* v = s->s->db().find(name);
     if (!v) throw Error(GSBN_ERR_NAME, std::string("no vector named ") + name);
     if (count != (int64_t)v->size())

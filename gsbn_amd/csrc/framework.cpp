@@ -4,8 +4,10 @@
  */
 #include "framework.h"
 
+#include <sys/mman.h>
 #include <sys/stat.h>
 
+#include <algorithm>
 #include <cctype>
 #include <cmath>
 #include <cerrno>
@@ -14,6 +16,8 @@
 #include <fstream>
 #include <iostream>
 #include <sstream>
+#include <system_error>
+#include <thread>
 
 namespace gsbn {
 
@@ -33,6 +37,153 @@ void op_check(int rc, const char* what) {
 hipStream_t& active_stream() {
   static hipStream_t s = nullptr;
   return s;
+}
+
+/* ------------------------------------------------------------------ */
+/* ------------------------------------------------------------------ */
+/* SolverMemory */
+
+SolverMemory*& active_memory() {
+  static thread_local SolverMemory* m = nullptr;
+  return m;
+}
+
+SolverMemory::~SolverMemory() {
+  for (auto& c : _chunks) (void)hipFree(c.base);
+  if (_ring) (void)hipHostFree(_ring);
+  if (_bounce) (void)hipHostFree(_bounce);
+  for (hipEvent_t e : _bounce_ev)
+    if (e) (void)hipEventDestroy(e);
+}
+
+void* SolverMemory::alloc(size_t bytes) {
+  std::lock_guard<std::mutex> lock(_mutex);
+  const size_t need = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+  /* a released array of at most twice the size */
+  auto f = _free.lower_bound(need);
+  if (f != _free.end() && f->first <= 2 * need) {
+    void* p = f->second;
+    _live[p] = f->first;
+    _free.erase(f);
+    return p;
+  }
+  /* the chunk with the smallest tail that holds it */
+  Chunk* at = nullptr;
+  for (auto& c : _chunks)
+    if (c.size - c.used >= need && (!at || c.size - c.used < at->size - at->used)) at = &c;
+  if (!at) {
+    /* chunks grow with what the solver holds already, from 4 MB to 1 GB, so
+     * a solver makes few of them and leaves at most a third of its memory, or
+     * 1 GB, unused */
+    const size_t mb = (size_t)1 << 20;
+    size_t size = std::min(std::max(_total / 2, 4 * mb), 1024 * mb);
+    size = std::max(size, need);
+    size = (size + 2 * mb - 1) / (2 * mb) * (2 * mb);
+    char* base = nullptr;
+    hipError_t e = hipMalloc(&base, size);
+    if (e != hipSuccess && size > need) {
+      (void)hipGetLastError();
+      size = need;
+      e = hipMalloc(&base, size);
+    }
+    hip_check(e, "hipMalloc");
+    _chunks.push_back({base, size, 0});
+    _total += size;
+    at = &_chunks.back();
+  }
+  void* p = at->base + at->used;
+  at->used += need;
+  _live[p] = need;
+  return p;
+}
+
+void SolverMemory::release(void* p) {
+  std::lock_guard<std::mutex> lock(_mutex);
+  auto it = _live.find(p);
+  if (it == _live.end()) return;
+  _free.emplace(it->second, p);
+  _live.erase(it);
+}
+
+/* Up to 8 MB go through the pinned ring and return without waiting; when the
+ * ring is full, the copies out of it are waited for.  Larger ones wait for
+ * their own copy. */
+void SolverMemory::upload(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  const size_t kMax = (size_t)8 << 20;
+  if (!bytes) return;
+  if (bytes > kMax) {
+    hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s), "H2D");
+    hip_check(hipStreamSynchronize(s), "sync");
+    return;
+  }
+  const size_t need = (bytes + 255) & ~(size_t)255;
+  if (_ring_pos + need > _ring_size) {
+    hip_check(hipStreamSynchronize(s), "sync");
+    _ring_pos = 0;
+    if (2 * need > _ring_size) {
+      size_t size = std::max<size_t>(_ring_size, (size_t)1 << 20);
+      while (size < 2 * need) size *= 2;
+      if (_ring) hip_check(hipHostFree(_ring), "hipHostFree");
+      _ring = nullptr;
+      _ring_size = 0;
+      hip_check(hipHostMalloc(&_ring, size, hipHostMallocDefault), "hipHostMalloc");
+      _ring_size = size;
+    }
+  }
+  memcpy(_ring + _ring_pos, src, bytes);
+  hip_check(hipMemcpyAsync(dst, _ring + _ring_pos, bytes, hipMemcpyHostToDevice, s), "H2D");
+  _ring_pos += need;
+}
+
+/* Large copies alternate between two pinned halves, four threads moving one
+ * to its destination while the other is filled: 400 MB to fresh pages in 12
+ * ms, against 100 ms by one pageable copy, which waits for the page faults
+ * (huge pages are asked for, 4 KB ones cost 30 ms more). */
+void SolverMemory::download(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  hip_check(hipStreamSynchronize(s), "sync");
+  const size_t half = (size_t)8 << 20;
+  if (bytes < half) {
+    if (bytes) hip_check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "D2H");
+    return;
+  }
+  if (!_bounce) {
+    hip_check(hipHostMalloc(&_bounce, 2 * half, hipHostMallocDefault), "hipHostMalloc");
+    for (auto& e : _bounce_ev)
+      hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+  }
+  const uintptr_t page = (uintptr_t)2 << 20;
+  const uintptr_t lo = ((uintptr_t)dst + page - 1) / page * page;
+  const uintptr_t hi = ((uintptr_t)dst + bytes) / page * page;
+  if (hi > lo) (void)madvise((void*)lo, hi - lo, MADV_HUGEPAGE); /* a hint */
+  char* out = static_cast<char*>(dst);
+  const char* in = static_cast<const char*>(src);
+  const size_t n = (bytes + half - 1) / half;
+  auto size_of = [&](size_t i) { return std::min(half, bytes - i * half); };
+  auto fetch = [&](size_t i) {
+    hip_check(hipMemcpyAsync(_bounce + (i & 1) * half, in + i * half, size_of(i),
+                             hipMemcpyDeviceToHost, s),
+              "D2H");
+    hip_check(hipEventRecord(_bounce_ev[i & 1], s), "hipEventRecord");
+  };
+  fetch(0);
+  for (size_t i = 0; i < n; ++i) {
+    if (i + 1 < n) fetch(i + 1);
+    hip_check(hipEventSynchronize(_bounce_ev[i & 1]), "hipEventSynchronize");
+    const char* from = _bounce + (i & 1) * half;
+    char* to = out + i * half;
+    const size_t len = size_of(i), part = (len / 4 + 4095) & ~(size_t)4095;
+    std::thread th[3];
+    int started = 0;
+    size_t at = 0;
+    try {
+      for (; started < 3 && at + part < len; ++started, at += part)
+        th[started] = std::thread([=] { memcpy(to + at, from + at, part); });
+    } catch (const std::system_error&) {
+      /* no more threads: the rest is copied below */
+    }
+    memcpy(to + at, from + at, len - at);
+    for (int k = 0; k < started; ++k) th[k].join();
+  }
 }
 
 /* ------------------------------------------------------------------ */
@@ -193,7 +344,7 @@ Solver::Solver(type_t type, string n_path, string s_path) {
   GlobalVar::clear();
   SolverParam solver_param = parse_solver_param_file(n_path);
   hip_check(hipStreamCreateWithFlags(&_stream, hipStreamNonBlocking), "hipStreamCreate");
-  active_stream() = _stream;
+  activate();
   string log_dir = solver_param.rec_param.directory;
   if (log_dir.empty()) log_dir = "./";
   if (log_dir.back() != '/') log_dir += "/";
@@ -239,10 +390,11 @@ Solver::~Solver() {
     (void)hipStreamDestroy(_stream);
   }
   if (active_stream() == _stream) active_stream() = nullptr;
+  if (active_memory() == _mem.get()) active_memory() = nullptr;
 }
 
 int Solver::step() {
-  active_stream() = _stream;
+  activate();
   _upd.update();
   int f = 0;
   _glv.geti("cycle-flag", f);

@@ -28,6 +28,7 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <set>
 #include <stdexcept>
 #include <string>
@@ -53,6 +54,82 @@ void hip_check(hipError_t e, const char* what);
 void op_check(int rc, const char* what);
 /* the stream all framework copies and kernels use (the current solver's) */
 hipStream_t& active_stream();
+
+/* The device memory of one solver and its host transfers.
+ *
+ * A batch of networks owns about forty device arrays per network.  Each as
+ * an allocation of its own cost 10-60 us to make and 60-250 us to free, each
+ * vector's own pinned staging buffer another 80 and 180 us, and each upload a
+ * wait of 14-75 us: 0.75 s of a 128-network run of 1.0 s.  Here arrays are
+ * carved from a few chunks that go back to the device with the solver, and
+ * uploads are staged through one pinned ring in stream order.  A released
+ * array is reused by later ones of about its size: every use of the memory
+ * is ordered by the solver's stream. */
+class SolverMemory : public std::enable_shared_from_this<SolverMemory> {
+ public:
+  ~SolverMemory();
+  void* alloc(size_t bytes); /* 256-byte aligned; throws when memory is out */
+  void release(void* p);
+  /* host -> device on stream s; src may change as soon as this returns */
+  void upload(void* dst, const void* src, size_t bytes, hipStream_t s);
+  /* device -> host after the work queued on s; dst is complete on return */
+  void download(void* dst, const void* src, size_t bytes, hipStream_t s);
+
+ private:
+  struct Chunk {
+    char* base;
+    size_t size, used;
+  };
+  std::mutex _mutex; /* arrays may be released from another thread */
+  vector<Chunk> _chunks;
+  map<void*, size_t> _live;
+  std::multimap<size_t, void*> _free; /* released arrays by size */
+  size_t _total = 0;
+  char* _ring = nullptr; /* pinned, for uploads */
+  size_t _ring_size = 0, _ring_pos = 0;
+  char* _bounce = nullptr; /* pinned, two halves for large downloads */
+  hipEvent_t _bounce_ev[2] = {nullptr, nullptr};
+};
+/* the memory of the solver that is being built or stepped on this thread */
+SolverMemory*& active_memory();
+
+/* a device array of the active solver */
+template <typename T>
+struct DevBuf {
+  T* p = nullptr;
+  size_t n = 0;
+  DevBuf() {}
+  DevBuf(const DevBuf&) = delete;
+  DevBuf& operator=(const DevBuf&) = delete;
+  ~DevBuf() { release(); }
+  void alloc(size_t count) {
+    release();
+    if (count) {
+      if (!active_memory()) throw Error(-4, "device array outside a solver");
+      mem = active_memory()->shared_from_this();
+      p = static_cast<T*>(mem->alloc(count * sizeof(T)));
+    }
+    n = count;
+  }
+  void release() {
+    if (p) mem->release(p);
+    p = nullptr;
+    n = 0;
+  }
+  void upload(const T* h, size_t count) {
+    if (count > n) alloc(count);
+    if (count) mem->upload(p, h, count * sizeof(T), active_stream());
+  }
+  void download(T* h, size_t count) const {
+    if (count)
+      mem->download(h, p, count * sizeof(T), active_stream());
+    else
+      hip_check(hipStreamSynchronize(active_stream()), "sync");
+  }
+
+ private:
+  std::shared_ptr<SolverMemory> mem;
+};
 
 /* ------------------------------------------------------------------ */
 class GlobalVar {
@@ -99,6 +176,13 @@ struct VecView {
   virtual ~VecView() {}
   virtual void pull(VecBase* v) = 0; /* device state -> host copy */
   virtual void push(VecBase* v) = 0; /* host copy -> device state */
+  /* device state -> n elements at out, without the vector's host copy;
+   * false where the view has no such way */
+  virtual bool pull_to(void* out, size_t n) {
+    (void)out;
+    (void)n;
+    return false;
+  }
 };
 
 class VecBase {
@@ -111,6 +195,10 @@ class VecBase {
   virtual void* host_ptr_sync() = 0;     /* host copy, brought up to date */
   virtual void* host_ptr_mutable() = 0;  /* same, then host becomes authoritative */
   virtual void resize_raw(size_t n) = 0;
+  /* the whole vector from the device to `out`, past the host copy (which
+   * stays as it is); false when the host copy is the current one or the view
+   * cannot */
+  virtual bool read_device(void* out) = 0;
   string name;
   DType type;
   int ld_ = 0;
@@ -136,12 +224,7 @@ class SyncVector : public VecBase {
  public:
   explicit SyncVector(const string& n) : VecBase(n, dtype_of<T>::v) {}
   ~SyncVector() override {
-    if (stage_ev_) {
-      (void)hipEventSynchronize(stage_ev_);
-      (void)hipEventDestroy(stage_ev_);
-    }
-    if (stage_) (void)hipHostFree(stage_);
-    if (d_) (void)hipFree(d_);
+    if (d_) mem_->release(d_);
   }
   size_t size() const override { return n_; }
   size_t elem_size() const override { return sizeof(T); }
@@ -215,12 +298,16 @@ class SyncVector : public VecBase {
       view->pull(this);
     } else {
       h_.resize(n_);
-      if (n_) {
-        hip_check(hipStreamSynchronize(stream()), "sync");
-        hip_check(hipMemcpy(h_.data(), d_, n_ * sizeof(T), hipMemcpyDeviceToHost), "D2H");
-      }
+      if (n_) mem_->download(h_.data(), d_, n_ * sizeof(T), stream());
     }
     status = SYNCED;
+  }
+  bool read_device(void* out) override {
+    if (status != DEVICE_NEWER || !n_) return false;
+    if (before_host_read) before_host_read();
+    if (view) return view->pull_to(out, n_);
+    mem_->download(out, d_, n_ * sizeof(T), stream());
+    return true;
   }
   void to_device() {
     if (view) {
@@ -233,16 +320,20 @@ class SyncVector : public VecBase {
     if (n_ != d_n_) {
       /* (re)allocate; keep the host copy authoritative */
       if (status == DEVICE_NEWER) to_host();
-      if (d_) hip_check(hipFree(d_), "free");
+      if (d_) mem_->release(d_);
       d_ = nullptr;
-      if (n_) hip_check(hipMalloc(&d_, n_ * sizeof(T)), "hipMalloc");
+      if (n_) {
+        if (!active_memory()) throw Error(-4, "vector " + name + " outside a solver");
+        mem_ = active_memory()->shared_from_this();
+        d_ = static_cast<T*>(mem_->alloc(n_ * sizeof(T)));
+      }
       d_n_ = n_;
       if (status == SYNCED) status = HOST_NEWER;
     }
     if (status == HOST_NEWER) {
       if (n_) {
         if (h_.size() < n_) h_.resize(n_);
-        upload();
+        mem_->upload(d_, h_.data(), n_ * sizeof(T), stream());
       }
       status = SYNCED;
     }
@@ -250,38 +341,7 @@ class SyncVector : public VecBase {
   vector<T>& raw_host() { return h_; }
 
  private:
-  /* host -> device copy in stream order.  Vectors of up to kStageMax bytes
-   * (stimulus rows of every network of a batch, masks, counters) go through
-   * a pinned staging buffer of their own, so the call returns without
-   * waiting for the device work queued before it; the buffer is refilled
-   * only after its previous copy has run (an event).  Larger vectors wait
-   * for their copy. */
-  static constexpr size_t kStageMax = (size_t)64 << 20;
-  void upload() {
-    const size_t bytes = n_ * sizeof(T);
-    if (bytes <= kStageMax) {
-      if (stage_ev_)
-        hip_check(hipEventSynchronize(stage_ev_), "staging event");
-      else
-        hip_check(hipEventCreateWithFlags(&stage_ev_, hipEventDisableTiming), "hipEventCreate");
-      if (stage_n_ < bytes) {
-        if (stage_) hip_check(hipHostFree(stage_), "hipHostFree");
-        stage_ = nullptr;
-        stage_n_ = 0;
-        hip_check(hipHostMalloc(&stage_, bytes, hipHostMallocDefault), "hipHostMalloc");
-        stage_n_ = bytes;
-      }
-      memcpy(stage_, h_.data(), bytes);
-      hip_check(hipMemcpyAsync(d_, stage_, bytes, hipMemcpyHostToDevice, stream()), "H2D");
-      hip_check(hipEventRecord(stage_ev_, stream()), "hipEventRecord");
-      return;
-    }
-    hip_check(hipMemcpyAsync(d_, h_.data(), bytes, hipMemcpyHostToDevice, stream()), "H2D");
-    hip_check(hipStreamSynchronize(stream()), "sync");
-  }
-  void* stage_ = nullptr;
-  size_t stage_n_ = 0;
-  hipEvent_t stage_ev_ = nullptr;
+  std::shared_ptr<SolverMemory> mem_;
 
   size_t offset(int i) const {
     if (i <= 0) return 0;
@@ -532,8 +592,14 @@ class Solver {
   Database& db() { return _database; }
   Upd& upd() { return _upd; }
   hipStream_t stream() const { return _stream; }
+  /* this solver's stream and memory become the calling thread's */
+  void activate() {
+    active_stream() = _stream;
+    active_memory() = _mem.get();
+  }
 
  private:
+  std::shared_ptr<SolverMemory> _mem = std::make_shared<SolverMemory>();
   Upd _upd;
   Database _database;
   GlobalVar _glv;

@@ -43,37 +43,6 @@
 namespace gsbn {
 namespace proc_upd_lazy {
 
-template <typename T>
-struct DevBuf {
-  T* p = nullptr;
-  size_t n = 0;
-  DevBuf() {}
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-  ~DevBuf() { release(); }
-  void alloc(size_t count) {
-    release();
-    n = count;
-    if (count) hip_check(hipMalloc(&p, count * sizeof(T)), "hipMalloc");
-  }
-  void release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    n = 0;
-  }
-  void upload(const T* h, size_t count) {
-    if (count > n) alloc(count);
-    if (count)
-      hip_check(hipMemcpyAsync(p, h, count * sizeof(T), hipMemcpyHostToDevice, active_stream()),
-                "H2D");
-    hip_check(hipStreamSynchronize(active_stream()), "sync");
-  }
-  void download(T* h, size_t count) const {
-    hip_check(hipStreamSynchronize(active_stream()), "sync");
-    if (count) hip_check(hipMemcpy(h, p, count * sizeof(T), hipMemcpyDeviceToHost), "D2H");
-  }
-};
-
 class Proj;
 
 class Pop {
@@ -304,11 +273,21 @@ struct SynField : VecView {
   void pull(VecBase* v) override {
     p->flush_deferred();
     p->materialize_kicks();
+    copy_to(raw_data(v));
+  }
+  bool pull_to(void* out, size_t n) override {
+    if (n != (size_t)p->nsyn) return false;
+    p->flush_deferred();
+    p->materialize_kicks();
+    copy_to(out);
+    return true;
+  }
+  void copy_to(void* out) {
     const size_t n = (size_t)p->nsyn;
     DevBuf<uint32_t> tmp;
     tmp.alloc(n);
     p->syn_field(field, tmp.p, 0);
-    tmp.download((uint32_t*)raw_data(v), n);
+    tmp.download((uint32_t*)out, n);
   }
   void push(VecBase* v) override {
     const size_t n = (size_t)p->nsyn;

@@ -532,7 +532,6 @@ void ProcSpkRec::update_gpu() {
 class ProcCheck : public ProcedureBase {
   REGISTER(ProcCheck)
  public:
-  ~ProcCheck() override;
   void init_new(SolverParam solver_param, Database& db) override;
   void init_copy(SolverParam solver_param, Database& db) override { init_new(solver_param, db); }
   void update_cpu() override { update_gpu(); }
@@ -547,7 +546,7 @@ class ProcCheck : public ProcedureBase {
   struct PopInfo {
     int H, M;
     SyncVector<int8_t>* spike;
-    int32_t* count;
+    int32_t* count; /* its part of _counts */
   };
   void report(bool final_line);
   GlobalVar _glv;
@@ -559,25 +558,18 @@ class ProcCheck : public ProcedureBase {
   int _cursor = 0;
   bool _updated_flag = false;
   string _logfile;
-  int32_t* _res_idx = nullptr; /* [windows][total_hcu] */
-  int32_t* _res_cnt = nullptr;
+  DevBuf<int32_t> _res_idx; /* [windows][total_hcu] */
+  DevBuf<int32_t> _res_cnt;
+  DevBuf<int32_t> _counts;
   vector<int> _window_mode;    /* mode index of each scored window */
   int _reported = 0;
   int _correct = 0, _total = 0;
   vector<int> _flags;
   vector<gsbn_check_item> _items;
-  gsbn_check_item* _items_dev = nullptr;
+  DevBuf<gsbn_check_item> _items_dev;
   bool _final_done = false;
 };
 REGISTERIMPL(ProcCheck);
-
-ProcCheck::~ProcCheck() {
-  for (auto& p : _pops)
-    if (p.count) (void)hipFree(p.count);
-  if (_res_idx) (void)hipFree(_res_idx);
-  if (_items_dev) (void)hipFree(_items_dev);
-  if (_res_cnt) (void)hipFree(_res_cnt);
-}
 
 void ProcCheck::init_new(SolverParam solver_param, Database& db) {
   string log_dir;
@@ -609,6 +601,7 @@ void ProcCheck::init_new(SolverParam solver_param, Database& db) {
   _lgidx = db.sync_vector_i32(".lgidx");
   GSBN_CHECK(_lgidx, ".lgidx missing (ProcExtGen must come first)");
   int pid = 0;
+  int64_t units = 0;
   for (auto& pp : solver_param.net_param.pop_param) {
     for (uint32_t k = 0; k < pp.pop_num; ++k) {
       PopInfo pi;
@@ -616,18 +609,25 @@ void ProcCheck::init_new(SolverParam solver_param, Database& db) {
       pi.M = pp.mcu_num;
       pi.spike = db.sync_vector_i8("spike_" + std::to_string(pid));
       GSBN_CHECK(pi.spike, "spike vector missing");
-      hip_check(hipMalloc(&pi.count, sizeof(int32_t) * pi.H * pi.M), "hipMalloc");
-      op_check(gsbn_i32_fill(pi.count, (int64_t)pi.H * pi.M, 0, active_stream()), "gsbn_i32_fill");
+      pi.count = nullptr;
       _total_hcu += pi.H;
+      units += (int64_t)pi.H * pi.M;
       _pops.push_back(pi);
       ++pid;
     }
   }
+  _counts.alloc((size_t)units);
+  op_check(gsbn_i32_fill(_counts.p, units, 0, active_stream()), "gsbn_i32_fill");
+  units = 0;
+  for (auto& p : _pops) {
+    p.count = _counts.p + units;
+    units += (int64_t)p.H * p.M;
+  }
   Parser par(get_proc_param(solver_param));
   if (!par.argi("threashold", _threshold)) _threshold = 0;
   size_t nwin = _list_mode.size() ? _list_mode.size() : 1;
-  hip_check(hipMalloc(&_res_idx, sizeof(int32_t) * nwin * _total_hcu), "hipMalloc");
-  hip_check(hipMalloc(&_res_cnt, sizeof(int32_t) * nwin * _total_hcu), "hipMalloc");
+  _res_idx.alloc(nwin * (size_t)_total_hcu);
+  _res_cnt.alloc(nwin * (size_t)_total_hcu);
   std::fstream out(_logfile, std::ios::out | std::ofstream::trunc);
   out << "result | reference pattern | recorded pattern | recorded pattern spike count" << std::endl;
   _cursor = 0;
@@ -670,11 +670,9 @@ void ProcCheck::update_gpu() {
           it.push_back(c);
         }
         _items = it;
-        hip_check(hipMalloc(&_items_dev, sizeof(gsbn_check_item) * it.size()), "hipMalloc");
-        hip_check(hipMemcpy(_items_dev, it.data(), sizeof(gsbn_check_item) * it.size(),
-                            hipMemcpyHostToDevice), "H2D");
+        _items_dev.upload(it.data(), it.size());
       }
-      op_check(gsbn_check_count_multi(_items_dev, (int32_t)_items.size(), active_stream()),
+      op_check(gsbn_check_count_multi(_items_dev.p, (int32_t)_items.size(), active_stream()),
                "gsbn_check_count_multi");
     }
     _updated_flag = true;
@@ -685,16 +683,16 @@ void ProcCheck::update_gpu() {
     return;
   }
   const int w = (int)_window_mode.size();
-  if (_items_dev) {
-    op_check(gsbn_check_argmax_multi(_items_dev, (int32_t)_items.size(),
-                                     _res_idx + (int64_t)w * _total_hcu,
-                                     _res_cnt + (int64_t)w * _total_hcu, active_stream()),
+  if (_items_dev.p) {
+    op_check(gsbn_check_argmax_multi(_items_dev.p, (int32_t)_items.size(),
+                                     _res_idx.p + (int64_t)w * _total_hcu,
+                                     _res_cnt.p + (int64_t)w * _total_hcu, active_stream()),
              "gsbn_check_argmax_multi");
   } else {
     int hoff = 0;
     for (auto& p : _pops) {
-      op_check(gsbn_check_argmax(p.H, p.M, p.count, _res_idx + (int64_t)w * _total_hcu + hoff,
-                                 _res_cnt + (int64_t)w * _total_hcu + hoff, active_stream()),
+      op_check(gsbn_check_argmax(p.H, p.M, p.count, _res_idx.p + (int64_t)w * _total_hcu + hoff,
+                                 _res_cnt.p + (int64_t)w * _total_hcu + hoff, active_stream()),
                "gsbn_check_argmax");
       hoff += p.H;
     }
@@ -710,8 +708,8 @@ void ProcCheck::report(bool final_line) {
   if (nw > _reported) {
     hip_check(hipStreamSynchronize(active_stream()), "sync");
     vector<int32_t> idx((size_t)nw * _total_hcu), cnt((size_t)nw * _total_hcu);
-    hip_check(hipMemcpy(idx.data(), _res_idx, idx.size() * 4, hipMemcpyDeviceToHost), "D2H");
-    hip_check(hipMemcpy(cnt.data(), _res_cnt, cnt.size() * 4, hipMemcpyDeviceToHost), "D2H");
+    hip_check(hipMemcpy(idx.data(), _res_idx.p, idx.size() * 4, hipMemcpyDeviceToHost), "D2H");
+    hip_check(hipMemcpy(cnt.data(), _res_cnt.p, cnt.size() * 4, hipMemcpyDeviceToHost), "D2H");
     std::fstream out(_logfile, std::ios::out | std::ios::app);
     for (int w = _reported; w < nw; ++w) {
       const mode_t& m = _list_mode[_window_mode[w]];

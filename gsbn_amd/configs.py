@@ -159,6 +159,10 @@ class NetSpec:
     # through rings of K spike steps per postsynaptic unit; 0: eager; None:
     # ProcUpdLazy's default (where it applies: 8 for one network, 16 for a batch)
     deferred_columns: Optional[int] = None
+    # deferred_sweeps 0: every learning-rate change sweeps all synapses at
+    # once; 1: it is recorded and applied later, where deferred columns apply;
+    # None: ProcUpdLazy's default (recorded from 1e7 synapses on)
+    deferred_sweeps: Optional[int] = None
 
     @property
     def total_hcu(self) -> int:
@@ -328,6 +332,8 @@ def prototxt(spec: NetSpec, stim_path: str, conn_path: str, rec_dir: str,
         L.append('  argi { key: "rowcol-wave" val: %d }' % spec.rowcol_wave)
     if spec.deferred_columns is not None:
         L.append('  argi { key: "deferred-columns" val: %d }' % spec.deferred_columns)
+    if spec.deferred_sweeps is not None:
+        L.append('  argi { key: "deferred-sweeps" val: %d }' % spec.deferred_sweeps)
     if spec.pop_wave is not None:
         L.append('  argi { key: "pop-wave" val: %d }' % spec.pop_wave)
     if spec.ovf_keep is not None:

@@ -416,38 +416,27 @@ __device__ __forceinline__ bool replay_kicks(const SynIO<PREC>& io, SynVals& v,
   return n0 <= n1;
 }
 
-/* The same for a ring of K = 8, held in registers: the ring is read with two
- * 16-byte loads that need no earlier result (issued beside the synapse
- * record), the entries are put in spike order by register selects, and the
- * coefficients of each kick are loaded while the previous kick is applied,
- * instead of one dependent load per ring entry and per kick.
- * s[q] is the step of spike number T - 7 + q (q = 0..6: the last K - 1
- * spikes); numbers below 0 hold INT_MIN and are never applied. */
+/* The last seven kicks of a unit in registers: the ring entries are read by
+ * loads that need no earlier result (issued beside the synapse record), and
+ * the coefficients of each kick are loaded while the previous kick is
+ * applied, instead of one dependent load per ring entry and per kick.
+ * s[q] is the step of spike number T - 7 + q (q = 0..6); numbers below 0 hold
+ * INT_MIN and are never applied.  more: number T - 8 (INT_MIN when the ring
+ * holds no such entry); a synapse older than it has more kicks pending than
+ * the seven and takes replay_kicks. */
 struct Ring8 {
-  int s[7];
+  int s[7], more;
 };
 
-__device__ __forceinline__ Ring8 ring8(const int4 lo, const int4 hi, const int T) {
-  const int e[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+__device__ __forceinline__ Ring8 ring8_load(const int32_t* ring, const int T, const int K) {
   Ring8 r;
 #pragma unroll
-  for (int q = 0; q < 7; ++q) {
-    const int n = T - 7 + q;
-    const int idx = n & 7;
-    int v = e[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) v = idx == i ? e[i] : v;
-    r.s[q] = n >= 0 ? v : INT_MIN;
-  }
+  for (int q = 0; q < 7; ++q) r.s[q] = T - 7 + q >= 0 ? ring[(T - 7 + q) & (K - 1)] : INT_MIN;
+  r.more = K > 8 && T - 8 >= 0 ? ring[(T - 8) & (K - 1)] : INT_MIN;
   return r;
 }
 
-__device__ __forceinline__ Ring8 ring8_load(const int32_t* ring, const int T) {
-  const int4* p = reinterpret_cast<const int4*>(ring);
-  return ring8(p[0], p[1], T);
-}
-
-/* replay_kicks for K = 8 from registers: applies the entries with
+/* replay_kicks from registers: applies the entries with
  * v.tij < s <= upto in spike order, each as the reference's column update
  * of step s.  With own != nullptr, also loads (first, beside the first
  * kick's) the coefficients of the gap from the last applied kick (or tij)
@@ -486,6 +475,77 @@ __device__ __forceinline__ bool replay_ring8(const SynIO<PREC>& io, SynVals& v, 
     }
   }
   return any;
+}
+
+/* The pending column kicks of one synapse in step order, for merging with
+ * recorded sweeps: positioned once (scanning back from the newest to the
+ * first past tij), then one ring load per kick, where replay_kicks would scan
+ * the ring again for every sweep. */
+struct Kicks {
+  const int32_t* ring;
+  int K, T, n, next; /* next: the step of kick n, INT_MAX after the last */
+  __device__ __forceinline__ Kicks(const int32_t* r, int T_, int K_, int tij)
+      : ring(r), K(K_), T(T_), n(T_), next(INT_MAX) {
+    const int lo = T - K + 1 > 0 ? T - K + 1 : 0;
+    while (n > lo) {
+      const int s = ring[(n - 1) & (K - 1)];
+      if (s <= tij) break;
+      next = s;
+      --n;
+    }
+  }
+  /* applies the kicks up to `upto`, each as replay_kicks does */
+  template <int PREC>
+  __device__ __forceinline__ void run(const SynIO<PREC>& io, SynVals& v, int upto,
+                                      const float* table, int table_len, float kftj) {
+    while (next <= upto) {
+      gsbn_syn_catchup_k(load_coef(table, table_len, next - v.tij), &v.pij, &v.eij, &v.zi2, &v.zj2);
+      v.zj2 = v.zj2 + kftj;
+      v.tij = next;
+      io.round_traces(v);
+      ++n;
+      next = n < T ? ring[n & (K - 1)] : INT_MAX;
+    }
+  }
+};
+
+/* The recorded sweeps (gsbn_sweep_log) of one synapse: for each of the n
+ * entries past v.tij, the pending column kicks up to its target, then the
+ * catch-up to the target, as all_kernel does them at the sweep (16-bit forms:
+ * rounded as its store rounds).  A sweep with a learning rate also sets the
+ * weight, from the traces of its own time only, and nothing reads the weight
+ * before the next one, so only the last such entry's is computed.  st, the
+ * synapse's row record, passes through the entries past its ti on the way
+ * (its pi enters the weight).  Returns whether the weight changed. */
+template <int PREC, class A>
+__device__ __forceinline__ bool replay_log(const SynIO<PREC>& io, SynVals& v, gsbn_row_rec& st,
+                                           const gsbn_sweep_log* __restrict__ lg, const int n,
+                                           const A& a, const int uj, Kicks& kicks) {
+  int wk = -1;
+  float wp = 0.0f, wpi = 0.0f;
+  for (int k = 0; k < n; ++k) {
+    const gsbn_sweep_entry e = lg->e[k];
+    if (e.target > st.ti) {
+      gsbn_row_catchup(gsbn_coef(e.table, e.table_len, e.target - st.ti), &st.pi, &st.ei, &st.zi);
+      st.ti = e.target;
+    }
+    if (e.target <= v.tij) continue;
+    kicks.run<PREC>(io, v, e.target, e.table, e.table_len, a.kftj);
+    const int D = e.target - v.tij;
+    if (D > 0) {
+      gsbn_syn_catchup_k(load_coef(e.table, e.table_len, D), &v.pij, &v.eij, &v.zi2, &v.zj2);
+      v.tij = e.target;
+      if (e.kp != 0.0f) {
+        wk = k;
+        wp = v.pij;
+        wpi = st.pi;
+      }
+      io.round_traces(v);
+    }
+  }
+  if (wk >= 0)
+    v.wij = gsbn_wij(wp, wpi, lg->pj[(int64_t)wk * a.H * a.M + uj], a.wgain, a.eps, a.eps2);
+  return wk >= 0;
 }
 
 /* per-launch values of a row/column update (taken from the argument struct
@@ -1550,12 +1610,17 @@ __global__ void __launch_bounds__(POP_MAX_THREADS) pop_flush_kernel(gsbn_pop_arg
 
 /* Part `part` of the row/column update of hypercolumn h.  FUSED: the
  * hypercolumn's active rows, spikes and pj come from the population phase
- * of the same workgroup (fl), not from memory. */
-template <int PREC, bool FUSED = false, bool ROWS = true, int NT = RC_THREADS, bool RING8 = false>
+ * of the same workgroup (fl), not from memory.  LOG: the nlog recorded sweeps
+ * of lg are pending (instances of their own, so that the others keep their
+ * registers). */
+template <int PREC, bool FUSED = false, bool ROWS = true, int NT = RC_THREADS, bool RING8 = false,
+          bool LOG = false>
 __device__ __forceinline__ void rowcol_body(const gsbn_rowcol_args& a, const RcStep& q,
                                             const int h, const int part,
                                             const FusedLds* fl = nullptr, const int keep = INT_MAX,
-                                            const int row_first = 0, const bool one_row = false) {
+                                            const int row_first = 0, const bool one_row = false,
+                                            const gsbn_sweep_log* lg = nullptr,
+                                            const int nlog = 0) {
   const SynIO<PREC> io(a);
   const int P = q.P;
   const int M = a.M, C = a.C;
@@ -1600,16 +1665,32 @@ __device__ __forceinline__ void rowcol_body(const gsbn_rowcol_args& a, const RcS
       const int64_t r = (int64_t)h * C + k;
       const int64_t sidx = r * M + j;
       gsbn_row_rec st = a.rowst[r];
-      SynVals s = io.load(sidx, !learn);
+      SynVals s = io.load(sidx, LOG || !learn);
+      bool w_log = false;
+      if constexpr (LOG) {
+        const int uj = h * M + j;
+        Kicks kicks(a.dhist + (int64_t)uj * a.dK, a.dcnt[uj], a.dK, s.tij);
+        w_log = replay_log<PREC>(io, s, st, lg, nlog, a, uj, kicks);
+        kicks.run<PREC>(io, s, t - 1, q.table, q.table_len, a.kftj);
+      }
       /* the synapse's own coefficients (gap to this step from tij after
        * any replayed kicks) */
       gsbn_syn_coef_t cown;
-      if (RING8 && a.dK == 8) {
+      if (LOG) {
+        if (t - s.tij > 0) cown = load_coef(q.table, q.table_len, t - s.tij);
+      } else if (RING8 && a.dK >= 8) {
         /* deferred column updates: this synapse's pending kicks first, from
-         * the unit's ring in registers; the ring is read beside the record */
+         * the unit's last ones in registers; they are read beside the record */
         const int uj = h * M + j;
-        const Ring8 rg = ring8_load(a.dhist + (int64_t)uj * 8, a.dcnt[uj]);
-        replay_ring8<PREC>(io, s, rg, t - 1, q.table, q.table_len, a.kftj, t, &cown);
+        const int T = a.dcnt[uj];
+        const int32_t* ring = a.dhist + (int64_t)uj * a.dK;
+        const Ring8 rg = ring8_load(ring, T, a.dK);
+        if (rg.more > s.tij) {
+          replay_kicks<PREC>(io, s, ring, T, a.dK, t - 1, q.table, q.table_len, a.kftj);
+          if (t - s.tij > 0) cown = load_coef(q.table, q.table_len, t - s.tij);
+        } else {
+          replay_ring8<PREC>(io, s, rg, t - 1, q.table, q.table_len, a.kftj, t, &cown);
+        }
       } else {
         if (a.dK) {
           const int uj = h * M + j;
@@ -1652,7 +1733,7 @@ __device__ __forceinline__ void rowcol_body(const gsbn_rowcol_args& a, const RcS
       /* column increment of a spiking postsynaptic unit after the row
        * update (the reference's col pass sees D == 0 here) */
       if ((FUSED ? fl->sj[j] : a.sj[h * M + j]) > 0) s.zj2 += a.kftj;
-      io.store(sidx, s, w_new);
+      io.store(sidx, s, w_new || w_log);
       a.contrib[((int64_t)h * C + aa) * M + j] = cval;
     }
     __syncthreads();
@@ -1683,6 +1764,22 @@ __device__ __forceinline__ void rowcol_body(const gsbn_rowcol_args& a, const RcS
       const int uj = h * M + j;
       const int32_t* ring = a.dhist + (int64_t)uj * a.dK;
       const int T = a.walk_T[h * M + s_i];
+      if constexpr (LOG) {
+        /* slot by slot: its recorded sweeps, then the kicks since */
+        for (int k = k0 + tid; k < k1; k += NT) {
+          const int r = h * C + k;
+          if (a.ii[r] < 0 || a.act_stamp[r] == q.exec) continue;
+          const int64_t sidx = (int64_t)r * M + j;
+          SynVals v = io.load(sidx, true);
+          gsbn_row_rec st = a.rowst[r];
+          const int tij = v.tij;
+          Kicks kicks(ring, T, a.dK, tij);
+          const bool w = replay_log<PREC>(io, v, st, lg, nlog, a, uj, kicks);
+          kicks.run<PREC>(io, v, t, q.table, q.table_len, a.kftj);
+          if (v.tij != tij) io.store(sidx, v, w);
+        }
+        continue;
+      }
       const int lo = T - a.dK + 1 > 0 ? T - a.dK + 1 : 0;
       const int cnt = T - lo;
       __syncthreads(); /* the previous walk's LDS */
@@ -1820,19 +1917,30 @@ __global__ void __launch_bounds__(RC_THREADS, 5) rowcol_kernel(gsbn_rowcol_args 
   rowcol_body<PREC, false, true, RC_THREADS, true>(a, q, h, blockIdx.x - h * a.parts);
 }
 
+template <int PREC>
+__global__ void __launch_bounds__(RC_THREADS) rowcol_kernel_log(gsbn_rowcol_args a,
+                                                                const gsbn_sweep_log* lg, int nlog) {
+  touch_kernarg_lines<sizeof(gsbn_rowcol_args)>();
+  const int h = blockIdx.x / a.parts;
+  const RcStep q = {a.simstep, a.exec, a.parts, a.table_len, a.kp, a.table};
+  rowcol_body<PREC, false, true, RC_THREADS, false, true>(a, q, h, blockIdx.x - h * a.parts, nullptr,
+                                                          INT_MAX, 0, false, lg, nlog);
+}
+
 /* work item i = (map entry i / parts, part i % parts); workgroup b takes
  * items b, b + gridDim.x, ... (see loop_grid) */
-template <int PREC>
-__global__ void __launch_bounds__(RC_THREADS, RC_WAVES(PREC))
+template <int PREC, bool LOG = false>
+__global__ void __launch_bounds__(RC_THREADS, LOG ? 4 : RC_WAVES(PREC))
     rowcol_kernel_batch(const gsbn_rowcol_args* __restrict__ arr, const int32_t* __restrict__ wg_proj,
                         const int32_t* __restrict__ wg_hcu, int parts, int nitems,
-                        gsbn_step_args st) {
+                        gsbn_step_args st, const gsbn_sweep_log* logs, int nlog) {
   for (int i = blockIdx.x; i < nitems; i += gridDim.x) {
     const int w = i / parts;
     const gsbn_rowcol_args& a = arr[wg_proj[w]];
     const RcStep q = {st.simstep, st.exec, parts, a.table_lens[st.kp_slot], a.taupdt * st.prn,
                       a.tables[st.kp_slot]};
-    rowcol_body<PREC>(a, q, wg_hcu[w], i - w * parts);
+    rowcol_body<PREC, false, true, RC_THREADS, false, LOG>(a, q, wg_hcu[w], i - w * parts, nullptr,
+                                                           INT_MAX, 0, false, logs + wg_proj[w], nlog);
   }
 }
 
@@ -1842,12 +1950,12 @@ __global__ void __launch_bounds__(RC_THREADS, RC_WAVES(PREC))
  * wave each keeps four times as many hypercolumns in flight.  Six waves per
  * SIMD as the other batched forms (FP16 five): 2.5 % faster than the five
  * its register count gives on 512 networks, seven slower. */
-template <int PREC>
-__global__ void __launch_bounds__(64, RC_WAVES(PREC))
+template <int PREC, bool LOG = false>
+__global__ void __launch_bounds__(64, LOG ? 4 : RC_WAVES(PREC))
     rowcol_kernel_batch_wave(const gsbn_rowcol_args* __restrict__ arr,
                              const int32_t* __restrict__ wg_proj,
                              const int32_t* __restrict__ wg_hcu, int nhcu, int nhelp,
-                             gsbn_step_args st) {
+                             gsbn_step_args st, const gsbn_sweep_log* logs, int nlog) {
   /* workgroups below nhelp (a multiple of the sub-queue count) run the
    * queued rows of this step, helper i those of sub-queue i % 64; the others
    * one hypercolumn each, keeping ovf_keep rows unless their sub-queue
@@ -1863,7 +1971,8 @@ __global__ void __launch_bounds__(64, RC_WAVES(PREC))
       const gsbn_rowcol_args& a = arr[tk[0]];
       const RcStep q = {st.simstep, st.exec, 1, a.table_lens[st.kp_slot], a.taupdt * st.prn,
                         a.tables[st.kp_slot]};
-      rowcol_body<PREC, false, true, 64>(a, q, tk[1], 0, nullptr, INT_MAX, tk[2], true);
+      rowcol_body<PREC, false, true, 64, false, LOG>(a, q, tk[1], 0, nullptr, INT_MAX, tk[2], true,
+                                                     logs + tk[0], nlog);
     }
     return;
   }
@@ -1874,7 +1983,8 @@ __global__ void __launch_bounds__(64, RC_WAVES(PREC))
                       a.tables[st.kp_slot]};
     int keep = INT_MAX;
     if (nhelp > 0 && st.ovf_cnt[ovf_counter(st.exec, ovf_queue(pj, h))] <= capq) keep = st.ovf_keep;
-    rowcol_body<PREC, false, true, 64>(a, q, h, 0, nullptr, keep);
+    rowcol_body<PREC, false, true, 64, false, LOG>(a, q, h, 0, nullptr, keep, 0, false, logs + pj,
+                                                   nlog);
   }
 }
 
@@ -1900,17 +2010,19 @@ __global__ void __launch_bounds__(64, RC_WAVES(PREC))
 /* The same with a work split per hypercolumn: workgroup w runs part
  * wg_part[w] & 0xffff of wg_part[w] >> 16 of hypercolumn wg_hcu[w] of
  * projection wg_proj[w] (larger hypercolumns split into more parts). */
-template <int PREC>
-__global__ void __launch_bounds__(RC_THREADS, RC_WAVES(PREC))
+template <int PREC, bool LOG = false>
+__global__ void __launch_bounds__(RC_THREADS, LOG ? 4 : RC_WAVES(PREC))
     rowcol_kernel_graded(const gsbn_rowcol_args* __restrict__ arr,
                          const int32_t* __restrict__ wg_proj, const int32_t* __restrict__ wg_hcu,
-                         const int32_t* __restrict__ wg_part, int nwg, gsbn_step_args st) {
+                         const int32_t* __restrict__ wg_part, int nwg, gsbn_step_args st,
+                         const gsbn_sweep_log* logs, int nlog) {
   for (int w = blockIdx.x; w < nwg; w += gridDim.x) {
     const gsbn_rowcol_args& a = arr[wg_proj[w]];
     const int pp = wg_part[w];
     const RcStep q = {st.simstep, st.exec, pp >> 16, a.table_lens[st.kp_slot], a.taupdt * st.prn,
                       a.tables[st.kp_slot]};
-    rowcol_body<PREC>(a, q, wg_hcu[w], pp & 0xffff);
+    rowcol_body<PREC, false, true, RC_THREADS, false, LOG>(a, q, wg_hcu[w], pp & 0xffff, nullptr,
+                                                           INT_MAX, 0, false, logs + wg_proj[w], nlog);
   }
 }
 
@@ -2057,9 +2169,173 @@ __global__ void __launch_bounds__(ALL_THREADS) materialize_kernel(gsbn_all_args 
   }
 }
 
-__global__ void jxx_kernel(gsbn_jxx_args a) {
+/* gsbn_proj_walk: the units whose kicks since their last column walk reach
+ * `due`, listed per HCU (ascending) with their spike counts; their walk
+ * counts as done.  One wave per HCU. */
+__device__ __forceinline__ void list_due(const gsbn_pop_proj& p, const int h, const int M,
+                                         const int due) {
+  const int lane = threadIdx.x;
+  int base = 0;
+  for (int j0 = 0; j0 < M; j0 += 64) {
+    const int j = j0 + lane, idx = h * M + j;
+    const int n = j < M ? p.dcnt[idx] : 0;
+    const bool is = j < M && n - p.dfl[idx] >= due;
+    const uint64_t bal = __ballot(is);
+    if (is) {
+      const int at = h * M + base + __popcll(bal & ((1ull << lane) - 1ull));
+      p.walk_list[at] = j;
+      p.walk_T[at] = n;
+      p.dfl[idx] = n;
+    }
+    base += __popcll(bal);
+  }
+  if (lane == 0) p.walk_cnt[h] = base;
+}
+
+__global__ void walk_list_kernel(gsbn_pop_proj p, int M, int due) {
+  list_due(p, blockIdx.x, M, due);
+}
+__global__ void walk_list_kernel_batch(const gsbn_pop_args* __restrict__ arr,
+                                       const int32_t* __restrict__ wg_pop,
+                                       const int32_t* __restrict__ wg_hcu, int due) {
+  const gsbn_pop_args& a = arr[wg_pop[blockIdx.x]];
+  list_due(a.proj0, wg_hcu[blockIdx.x], a.M, due);
+}
+
+/* the listed units' columns: rowcol_body's column pass with no active rows
+ * (no row carries the stamp -2); part blockIdx.y of the HCU's slots */
+template <int PREC, bool LOG>
+__global__ void __launch_bounds__(RC_THREADS) walk_kernel(gsbn_rowcol_args a, const gsbn_sweep_log* lg,
+                                                          int nlog) {
+  const RcStep q = {a.simstep, -2, (int)gridDim.y, a.table_len, a.kp, a.table};
+  rowcol_body<PREC, false, false, RC_THREADS, false, LOG>(a, q, blockIdx.x, blockIdx.y, nullptr,
+                                                          INT_MAX, 0, false, lg, nlog);
+}
+template <int PREC, bool LOG>
+__global__ void __launch_bounds__(RC_THREADS)
+    walk_kernel_batch(const gsbn_rowcol_args* __restrict__ arr, const int32_t* __restrict__ wg_proj,
+                      const int32_t* __restrict__ wg_hcu, gsbn_step_args st,
+                      const gsbn_sweep_log* logs, int nlog) {
+  const int pj = wg_proj[blockIdx.x];
+  const gsbn_rowcol_args& a = arr[pj];
+  /* parts of about 512 slots: those beyond the HCU's leave */
+  const int parts = (a.C + 511) / 512 < (int)gridDim.y ? (a.C + 511) / 512 : (int)gridDim.y;
+  if ((int)blockIdx.y >= parts) return;
+  const RcStep q = {st.simstep, -2, parts, a.table_lens[st.kp_slot], a.taupdt * st.prn,
+                    a.tables[st.kp_slot]};
+  rowcol_body<PREC, false, false, RC_THREADS, false, LOG>(a, q, wg_hcu[blockIdx.x], blockIdx.y,
+                                                          nullptr, INT_MAX, 0, false, logs + pj, nlog);
+}
+
+/* gsbn_proj_sweep_log: all_kernel over several recorded sweeps in one pass,
+ * the kicks after the last one included.  One pass moves a synapse once for
+ * up to GSBN_SWEEP_LOG sweeps; the sweeps in between cost arithmetic only (a
+ * coefficient lookup and, with a learning rate, a logarithm each). */
+template <int PREC>
+__global__ void __launch_bounds__(ALL_THREADS) sweep_log_kernel(gsbn_all_args a,
+                                                                const gsbn_sweep_log* lg, int n) {
+  __shared__ float sh_pi[ALL_ROWS][GSBN_SWEEP_LOG + 1];
+  __shared__ int sh_ii[ALL_ROWS];
+  /* the entries' targets, rates and coefficients of the gap from the entry
+   * before: after its first entry a synapse without kicks in between takes
+   * every gap from here */
+  __shared__ __attribute__((aligned(16))) float sh_gap[GSBN_SWEEP_LOG][8];
+  __shared__ int sh_target[GSBN_SWEEP_LOG];
+  __shared__ float sh_kp[GSBN_SWEEP_LOG];
+  if ((int)threadIdx.x < n) {
+    const int k = threadIdx.x;
+    const gsbn_sweep_entry e = lg->e[k];
+    sh_target[k] = e.target;
+    sh_kp[k] = e.kp;
+    if (k > 0) {
+      const gsbn_syn_coef_t c = load_coef(e.table, e.table_len, e.target - lg->e[k - 1].target);
+      float* g = sh_gap[k];
+      g[0] = c.ezi;
+      g[1] = c.ezj;
+      g[2] = c.ee;
+      g[3] = c.ep;
+      g[4] = c.cez;
+      g[5] = c.cpe;
+      g[6] = c.cpz;
+      g[7] = 0.0f;
+    }
+  }
+  const SynIO<PREC> io(a);
+  const int64_t R = (int64_t)a.H * a.C, N = (int64_t)a.H * a.M;
+  const int M = a.M;
+  const int tid = threadIdx.x;
+  const int64_t nchunks = (R + ALL_ROWS - 1) / ALL_ROWS;
+  for (int64_t ch = blockIdx.x; ch < nchunks; ch += gridDim.x) {
+    const int64_t r0 = ch * ALL_ROWS;
+    const int nr = (R - r0 < ALL_ROWS) ? (int)(R - r0) : ALL_ROWS;
+    if (tid < nr) {
+      const int64_t r = r0 + tid;
+      gsbn_row_rec st = a.rowst[r];
+      const int ti = st.ti;
+      for (int k = 0; k < n; ++k) {
+        const gsbn_sweep_entry e = lg->e[k];
+        if (e.target > st.ti) {
+          gsbn_row_catchup(gsbn_coef(e.table, e.table_len, e.target - st.ti), &st.pi, &st.ei, &st.zi);
+          st.ti = e.target;
+        }
+        sh_pi[tid][k] = st.pi;
+      }
+      if (st.ti != ti) a.rowst[r] = st;
+      sh_ii[tid] = a.ii[r];
+    }
+    __syncthreads();
+    for (int f = tid; f < nr * M; f += ALL_THREADS) {
+      const int rr = f / M;
+      const int j = f - rr * M;
+      const int64_t r = r0 + rr;
+      const int64_t sidx = r * M + j;
+      const int uj = (int)(r / a.C) * M + j;
+      SynVals s = io.load(sidx, true);
+      const int tij = s.tij;
+      const bool conn = sh_ii[rr] >= 0;
+      const int T = conn ? a.dcnt[uj] : 0;
+      const int32_t* ring = a.dhist + (int64_t)uj * a.dK;
+      Kicks kicks(ring, T, a.dK, tij);
+      int wk = -1;
+      float wp = 0.0f;
+      for (int k = 0; k < n; ++k) {
+        const int target = sh_target[k];
+        if (target <= s.tij) continue;
+        if (kicks.next <= target)
+          kicks.run<PREC>(io, s, target, lg->e[k].table, lg->e[k].table_len, a.kftj);
+        const int D = target - s.tij;
+        if (D > 0) {
+          gsbn_syn_coef_t c;
+          if (k > 0 && s.tij == sh_target[k - 1]) {
+            const float4 x = *reinterpret_cast<const float4*>(sh_gap[k]);
+            const float4 y = *reinterpret_cast<const float4*>(sh_gap[k] + 4);
+            c = {x.x, x.y, x.z, x.w, y.x, y.y, y.z};
+          } else {
+            c = load_coef(lg->e[k].table, lg->e[k].table_len, D);
+          }
+          gsbn_syn_catchup_k(c, &s.pij, &s.eij, &s.zi2, &s.zj2);
+          s.tij = target;
+          if (sh_kp[k] != 0.0f) {
+            wk = k;
+            wp = s.pij;
+          }
+          io.round_traces(s);
+        }
+      }
+      /* the last learning sweep's weight (see replay_log) */
+      if (wk >= 0) s.wij = gsbn_wij(wp, sh_pi[rr][wk], lg->pj[wk * N + uj], a.wgain, a.eps, a.eps2);
+      const bool w_new = wk >= 0;
+      kicks.run<PREC>(io, s, a.target, a.table, a.table_len, a.kftj);
+      if (s.tij != tij) io.store(sidx, s, w_new);
+    }
+    __syncthreads();
+  }
+}
+
+__global__ void jxx_kernel(gsbn_jxx_args a, float* pj_before) {
   for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < a.N; idx += gridDim.x * blockDim.x) {
     float pj = a.pj[idx], ej = a.ej[idx], zj = a.zj[idx];
+    if (pj_before) pj_before[idx] = pj;
     const int sj = a.sj[idx];
     a.epsc[idx] *= (1 - a.kepsc);
     pj += (ej - pj) * a.kp;
@@ -2070,6 +2346,32 @@ __global__ void jxx_kernel(gsbn_jxx_args a) {
     a.pj[idx] = pj;
     a.ej[idx] = ej;
     a.zj[idx] = zj;
+  }
+}
+
+/* jxx_kernel for every population of a batch, one workgroup per HCU */
+__global__ void jxx_mark_kernel_batch(const gsbn_pop_args* __restrict__ arr, gsbn_sweep_log* logs,
+                                      int slot, const int32_t* __restrict__ wg_pop,
+                                      const int32_t* __restrict__ wg_hcu, gsbn_step_args st) {
+  const gsbn_pop_args& a = arr[wg_pop[blockIdx.x]];
+  const gsbn_pop_proj& p = a.proj0;
+  const int h = wg_hcu[blockIdx.x], M = a.M;
+  float* before = logs[p.bidx].pj + (int64_t)slot * a.H * M;
+  const float kp = p.taupdt * st.prn;
+  for (int j = threadIdx.x; j < M; j += blockDim.x) {
+    const int idx = h * M + j;
+    float pj = p.pj[idx], ej = p.ej[idx], zj = p.zj[idx];
+    const int sj = a.spike[idx];
+    before[idx] = pj;
+    a.epsc[idx] *= (1 - p.kepsc);
+    pj += (ej - pj) * kp;
+    ej += (zj - ej) * p.ke;
+    zj *= (1 - p.kzj);
+    if (sj > 0) zj += p.kftj;
+    if (kp != 0.0f) a.bj[idx] = p.bgain * gsbn_logf(pj + p.eps);
+    p.pj[idx] = pj;
+    p.ej[idx] = ej;
+    p.zj[idx] = zj;
   }
 }
 
@@ -2430,8 +2732,44 @@ int gsbn_proj_all(const gsbn_all_args* a, void* stream) {
 int gsbn_proj_jxx(const gsbn_jxx_args* a, void* stream) {
   if (!a || a->N < 0) return GSBN_ERR_ARG;
   if (a->N == 0) return 0;
-  launch_timed(jxx_kernel, dim3(grid_for(a->N, 256, 4096)), dim3(256), 0,
-                     (hipStream_t)stream, *a);
+  launch_timed(jxx_kernel, dim3(grid_for(a->N, 256, 4096)), dim3(256), 0, (hipStream_t)stream, *a,
+               (float*)nullptr);
+  return launch_status();
+}
+
+int gsbn_proj_jxx_mark(const gsbn_jxx_args* a, float* pj_before, void* stream) {
+  if (!a || a->N < 0 || !pj_before) return GSBN_ERR_ARG;
+  if (a->N == 0) return 0;
+  launch_timed(jxx_kernel, dim3(grid_for(a->N, 256, 4096)), dim3(256), 0, (hipStream_t)stream, *a,
+               pj_before);
+  return launch_status();
+}
+
+int gsbn_proj_jxx_mark_batch(const gsbn_pop_args* pops_dev, gsbn_sweep_log* logs, int32_t slot,
+                             const int32_t* wg_pop, const int32_t* wg_hcu, int32_t nwg,
+                             const gsbn_step_args* step, void* stream) {
+  if (!pops_dev || !logs || slot < 0 || slot >= GSBN_SWEEP_LOG || !wg_pop || !wg_hcu || nwg <= 0 ||
+      !step)
+    return GSBN_ERR_ARG;
+  launch_timed(jxx_mark_kernel_batch, dim3(nwg), dim3(64), 0, (hipStream_t)stream, pops_dev, logs,
+               slot, wg_pop, wg_hcu, *step);
+  return launch_status();
+}
+
+int gsbn_proj_sweep_log(const gsbn_all_args* a, const gsbn_sweep_log* log, int32_t n, void* stream) {
+  if (!a || a->H <= 0 || a->M <= 0 || a->C < 0 || !a->table || a->table_len < 2 ||
+      !trace_form_ok(*a) || a->dK <= 0 || !deferred_ok(a->dK, a->ii, a->dhist, a->dcnt) ||
+      !a->rowst || !log || n < 0 || n > GSBN_SWEEP_LOG)
+    return GSBN_ERR_ARG;
+  const int64_t R = (int64_t)a->H * a->C;
+  if (R == 0) return 0;
+  const dim3 grid(grid_for((R + ALL_ROWS - 1) / ALL_ROWS, 1, 8192)), b(ALL_THREADS);
+  hipStream_t s = (hipStream_t)stream;
+  switch (a->prec) {
+    case GSBN_PREC_F32: launch_timed(sweep_log_kernel<GSBN_PREC_F32>, grid, b, 0, s, *a, log, n); break;
+    case GSBN_PREC_BF16: launch_timed(sweep_log_kernel<GSBN_PREC_BF16>, grid, b, 0, s, *a, log, n); break;
+    default: launch_timed(sweep_log_kernel<GSBN_PREC_F16>, grid, b, 0, s, *a, log, n); break;
+  }
   return launch_status();
 }
 
@@ -2458,7 +2796,8 @@ int gsbn_rowcol_resident(int32_t prec, int32_t* out) {
   return 0;
 }
 
-int gsbn_proj_rowcol(const gsbn_rowcol_args* a, void* stream) {
+static int launch_rowcol(const gsbn_rowcol_args* a, const gsbn_sweep_log* lg, int nlog,
+                         void* stream) {
   if (!a || a->H <= 0 || a->M <= 0 || a->C < 0 || !a->table || a->table_len < 2 || a->parts < 0 ||
       !trace_form_ok(*a) || !deferred_ok(a->dK, a->ii, a->dhist, a->dcnt) ||
       (a->dK && !a->walk_T))
@@ -2474,17 +2813,93 @@ int gsbn_proj_rowcol(const gsbn_rowcol_args* a, void* stream) {
   const int64_t grid = (int64_t)b.H * b.parts;
   if (grid > 0x7fffffff) return GSBN_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
+  const dim3 g((unsigned)grid), t(RC_THREADS);
+#define RC_SINGLE(P)                                              \
+  if (lg)                                                         \
+    launch_timed(rowcol_kernel_log<P>, g, t, 0, s, b, lg, nlog);  \
+  else                                                            \
+    launch_timed(rowcol_kernel<P>, g, t, 0, s, b);                \
+  break
   switch (b.prec) {
-    case GSBN_PREC_F32:
-      launch_timed(rowcol_kernel<GSBN_PREC_F32>, dim3((unsigned)grid), dim3(RC_THREADS), 0, s, b);
-      break;
-    case GSBN_PREC_BF16:
-      launch_timed(rowcol_kernel<GSBN_PREC_BF16>, dim3((unsigned)grid), dim3(RC_THREADS), 0, s, b);
-      break;
-    default:
-      launch_timed(rowcol_kernel<GSBN_PREC_F16>, dim3((unsigned)grid), dim3(RC_THREADS), 0, s, b);
-      break;
+    case GSBN_PREC_F32: RC_SINGLE(GSBN_PREC_F32);
+    case GSBN_PREC_BF16: RC_SINGLE(GSBN_PREC_BF16);
+    default: RC_SINGLE(GSBN_PREC_F16);
   }
+#undef RC_SINGLE
+  return launch_status();
+}
+
+static bool batch_step_ok(const gsbn_step_args* st) {
+  return st && st->kp_slot >= 0 && st->kp_slot < GSBN_KP_SLOTS && st->prec >= GSBN_PREC_F32 &&
+         st->prec <= GSBN_PREC_F16;
+}
+
+/* recorded sweeps of a row/column launch: deferred column updates on */
+static bool log_ok(const gsbn_sweep_log* lg, int n) {
+  return lg && n > 0 && n <= GSBN_SWEEP_LOG;
+}
+
+int gsbn_proj_rowcol(const gsbn_rowcol_args* a, void* stream) {
+  return launch_rowcol(a, nullptr, 0, stream);
+}
+
+int gsbn_proj_rowcol_log(const gsbn_rowcol_args* a, const gsbn_sweep_log* log, int32_t n,
+                         void* stream) {
+  if (!log_ok(log, n) || !a || a->dK <= 0) return GSBN_ERR_ARG;
+  return launch_rowcol(a, log, n, stream);
+}
+
+int gsbn_proj_walk(const gsbn_pop_proj* p, const gsbn_rowcol_args* a, int32_t due,
+                   const gsbn_sweep_log* log, int32_t n, void* stream) {
+  if (!p || !a || a->H <= 0 || a->M <= 0 || a->C < 0 || !a->table || a->table_len < 2 ||
+      !trace_form_ok(*a) || a->dK <= 0 || !deferred_ok(a->dK, a->ii, a->dhist, a->dcnt) ||
+      due <= 0 || !p->dcnt || !p->dfl || !p->walk_list || !p->walk_cnt || !p->walk_T ||
+      a->spk_list != p->walk_list || a->spk_cnt != p->walk_cnt || a->walk_T != p->walk_T ||
+      (n && !log_ok(log, n)) || a->H > 0x7fffffff / 64)
+    return GSBN_ERR_ARG;
+  if (a->C == 0) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(walk_list_kernel, dim3(a->H), dim3(64), 0, s, *p, a->M, due);
+  const int parts = (a->C + 511) / 512 < 64 ? (a->C + 511) / 512 : 64;
+  const dim3 g(a->H, parts), t(RC_THREADS);
+#define WALK(P)                                                                         \
+  if (n) hipLaunchKernelGGL((walk_kernel<P, true>), g, t, 0, s, *a, log, n);            \
+  else hipLaunchKernelGGL((walk_kernel<P, false>), g, t, 0, s, *a, log, n);             \
+  break
+  switch (a->prec) {
+    case GSBN_PREC_F32: WALK(GSBN_PREC_F32);
+    case GSBN_PREC_BF16: WALK(GSBN_PREC_BF16);
+    default: WALK(GSBN_PREC_F16);
+  }
+#undef WALK
+  return launch_status();
+}
+
+int gsbn_proj_walk_batch(const gsbn_pop_args* pops_dev, const int32_t* wg_pop,
+                         const int32_t* wg_pop_hcu, int32_t nwg, const gsbn_rowcol_args* projs_dev,
+                         const int32_t* wg_proj, const int32_t* wg_proj_hcu, int32_t nhcu,
+                         int32_t max_slots, int32_t due, const gsbn_sweep_log* logs, int32_t n,
+                         const gsbn_step_args* step, void* stream) {
+  if (!pops_dev || !wg_pop || !wg_pop_hcu || nwg <= 0 || !projs_dev || !wg_proj || !wg_proj_hcu ||
+      nhcu <= 0 || max_slots <= 0 || due <= 0 || (n && !log_ok(logs, n)) || !batch_step_ok(step))
+    return GSBN_ERR_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(walk_list_kernel_batch, dim3(nwg), dim3(64), 0, s, pops_dev, wg_pop, wg_pop_hcu,
+                     due);
+  const int parts = (max_slots + 511) / 512 < 64 ? (max_slots + 511) / 512 : 64;
+  const dim3 g(nhcu, parts), t(RC_THREADS);
+#define WALK(P)                                                                                   \
+  if (n) hipLaunchKernelGGL((walk_kernel_batch<P, true>), g, t, 0, s, projs_dev, wg_proj,         \
+                            wg_proj_hcu, *step, logs, n);                                         \
+  else hipLaunchKernelGGL((walk_kernel_batch<P, false>), g, t, 0, s, projs_dev, wg_proj,          \
+                          wg_proj_hcu, *step, logs, n);                                           \
+  break
+  switch (step->prec) {
+    case GSBN_PREC_F32: WALK(GSBN_PREC_F32);
+    case GSBN_PREC_BF16: WALK(GSBN_PREC_BF16);
+    default: WALK(GSBN_PREC_F16);
+  }
+#undef WALK
   return launch_status();
 }
 
@@ -2525,96 +2940,104 @@ int gsbn_pop_update_batch_wave(const gsbn_pop_args* pops_dev, const int32_t* wg_
   return launch_status();
 }
 
-int gsbn_proj_rowcol_batch(const gsbn_rowcol_args* projs_dev, const int32_t* wg_proj,
-                           const int32_t* wg_hcu, int32_t nhcu, int32_t parts,
-                           const gsbn_step_args* step, void* stream) {
-  if (!projs_dev || !wg_proj || !wg_hcu || !step || nhcu <= 0 || parts <= 0 ||
-      step->kp_slot < 0 || step->kp_slot >= GSBN_KP_SLOTS || step->prec < GSBN_PREC_F32 ||
-      step->prec > GSBN_PREC_F16)
+/* the instance of a batched row/column kernel for a trace form, with or
+ * without recorded sweeps */
+#define RC_BATCH(K, grid, block, ...)                                                             \
+  switch (step->prec) {                                                                           \
+    case GSBN_PREC_F32:                                                                           \
+      if (logs) launch_timed(K<GSBN_PREC_F32, true>, grid, block, 0, s, __VA_ARGS__, logs, nlog); \
+      else launch_timed(K<GSBN_PREC_F32, false>, grid, block, 0, s, __VA_ARGS__, logs, nlog);     \
+      break;                                                                                      \
+    case GSBN_PREC_BF16:                                                                          \
+      if (logs) launch_timed(K<GSBN_PREC_BF16, true>, grid, block, 0, s, __VA_ARGS__, logs, nlog);\
+      else launch_timed(K<GSBN_PREC_BF16, false>, grid, block, 0, s, __VA_ARGS__, logs, nlog);    \
+      break;                                                                                      \
+    default:                                                                                      \
+      if (logs) launch_timed(K<GSBN_PREC_F16, true>, grid, block, 0, s, __VA_ARGS__, logs, nlog); \
+      else launch_timed(K<GSBN_PREC_F16, false>, grid, block, 0, s, __VA_ARGS__, logs, nlog);     \
+      break;                                                                                      \
+  }
+
+static int launch_batch(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs, int nlog,
+                        const int32_t* wg_proj, const int32_t* wg_hcu, int32_t nhcu, int32_t parts,
+                        const gsbn_step_args* step, void* stream) {
+  if (!projs_dev || !wg_proj || !wg_hcu || nhcu <= 0 || parts <= 0 || !batch_step_ok(step))
     return GSBN_ERR_ARG;
   const int64_t items = (int64_t)nhcu * parts;
   if (items > 0x7fffffff) return GSBN_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 b(RC_THREADS);
   const int n = (int)items;
-  switch (step->prec) {
-    case GSBN_PREC_F32:
-      launch_timed(rowcol_kernel_batch<GSBN_PREC_F32>,
-                   dim3(loop_grid(rowcol_kernel_batch<GSBN_PREC_F32>, RC_THREADS, 0, n)), b, 0, s,
-                   projs_dev, wg_proj, wg_hcu, parts, n, *step);
-      break;
-    case GSBN_PREC_BF16:
-      launch_timed(rowcol_kernel_batch<GSBN_PREC_BF16>,
-                   dim3(loop_grid(rowcol_kernel_batch<GSBN_PREC_BF16>, RC_THREADS, 0, n)), b, 0,
-                   s, projs_dev, wg_proj, wg_hcu, parts, n, *step);
-      break;
-    default:
-      launch_timed(rowcol_kernel_batch<GSBN_PREC_F16>,
-                   dim3(loop_grid(rowcol_kernel_batch<GSBN_PREC_F16>, RC_THREADS, 0, n)), b, 0,
-                   s, projs_dev, wg_proj, wg_hcu, parts, n, *step);
-      break;
-  }
+  RC_BATCH(rowcol_kernel_batch, dim3((unsigned)n), dim3(RC_THREADS), projs_dev, wg_proj, wg_hcu,
+           parts, n, *step)
   return launch_status();
 }
 
+int gsbn_proj_rowcol_batch(const gsbn_rowcol_args* projs_dev, const int32_t* wg_proj,
+                           const int32_t* wg_hcu, int32_t nhcu, int32_t parts,
+                           const gsbn_step_args* step, void* stream) {
+  return launch_batch(projs_dev, nullptr, 0, wg_proj, wg_hcu, nhcu, parts, step, stream);
+}
 
+int gsbn_proj_rowcol_batch_log(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs,
+                               int32_t n, const int32_t* wg_proj, const int32_t* wg_hcu,
+                               int32_t nhcu, int32_t parts, const gsbn_step_args* step,
+                               void* stream) {
+  if (!log_ok(logs, n)) return GSBN_ERR_ARG;
+  return launch_batch(projs_dev, logs, n, wg_proj, wg_hcu, nhcu, parts, step, stream);
+}
+
+static int launch_wave(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs, int nlog,
+                       const int32_t* wg_proj, const int32_t* wg_hcu, int32_t nhcu,
+                       const gsbn_step_args* step, void* stream) {
+  if (!projs_dev || !wg_proj || !wg_hcu || nhcu <= 0 || !batch_step_ok(step) ||
+      (step->ovf_keep > 0 && (!step->ovf_cnt || !step->ovf_task || step->ovf_cap < 0)))
+    return GSBN_ERR_ARG;
+  hipStream_t s = (hipStream_t)stream;
+  /* helper waves for the queued rows: enough to run a busy step's queue in
+   * about one pass of the device */
+  const int nhelp = step->ovf_keep > 0 ? GSBN_OVF_HELPERS : 0;
+  RC_BATCH(rowcol_kernel_batch_wave, dim3((unsigned)(nhcu + nhelp)), dim3(64), projs_dev, wg_proj,
+           wg_hcu, nhcu, nhelp, *step)
+  return launch_status();
+}
 
 int gsbn_proj_rowcol_batch_wave(const gsbn_rowcol_args* projs_dev, const int32_t* wg_proj,
                                 const int32_t* wg_hcu, int32_t nhcu, const gsbn_step_args* step,
                                 void* stream) {
-  if (!projs_dev || !wg_proj || !wg_hcu || !step || nhcu <= 0 || step->kp_slot < 0 ||
-      step->kp_slot >= GSBN_KP_SLOTS || step->prec < GSBN_PREC_F32 || step->prec > GSBN_PREC_F16 ||
-      (step->ovf_keep > 0 && (!step->ovf_cnt || !step->ovf_task || step->ovf_cap < 0)))
+  return launch_wave(projs_dev, nullptr, 0, wg_proj, wg_hcu, nhcu, step, stream);
+}
+
+int gsbn_proj_rowcol_batch_wave_log(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs,
+                                    int32_t n, const int32_t* wg_proj, const int32_t* wg_hcu,
+                                    int32_t nhcu, const gsbn_step_args* step, void* stream) {
+  if (!log_ok(logs, n)) return GSBN_ERR_ARG;
+  return launch_wave(projs_dev, logs, n, wg_proj, wg_hcu, nhcu, step, stream);
+}
+
+static int launch_graded(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs, int nlog,
+                         const int32_t* wg_proj, const int32_t* wg_hcu, const int32_t* wg_part,
+                         int32_t nwg, const gsbn_step_args* step, void* stream) {
+  if (!projs_dev || !wg_proj || !wg_hcu || !wg_part || nwg <= 0 || !batch_step_ok(step))
     return GSBN_ERR_ARG;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 b(64);
-  /* helper waves for the queued rows: enough to run a busy step's queue in
-   * about one pass of the device */
-  const int nhelp = step->ovf_keep > 0 ? GSBN_OVF_HELPERS : 0;
-  const unsigned g = (unsigned)(nhcu + nhelp);
-  switch (step->prec) {
-    case GSBN_PREC_F32:
-      launch_timed(rowcol_kernel_batch_wave<GSBN_PREC_F32>, dim3(g), b, 0, s, projs_dev, wg_proj,
-                   wg_hcu, nhcu, nhelp, *step);
-      break;
-    case GSBN_PREC_BF16:
-      launch_timed(rowcol_kernel_batch_wave<GSBN_PREC_BF16>, dim3(g), b, 0, s, projs_dev, wg_proj,
-                   wg_hcu, nhcu, nhelp, *step);
-      break;
-    default:
-      launch_timed(rowcol_kernel_batch_wave<GSBN_PREC_F16>, dim3(g), b, 0, s, projs_dev, wg_proj,
-                   wg_hcu, nhcu, nhelp, *step);
-      break;
-  }
+  RC_BATCH(rowcol_kernel_graded, dim3((unsigned)nwg), dim3(RC_THREADS), projs_dev, wg_proj, wg_hcu,
+           wg_part, nwg, *step)
   return launch_status();
 }
+#undef RC_BATCH
 
 int gsbn_proj_rowcol_graded(const gsbn_rowcol_args* projs_dev, const int32_t* wg_proj,
                             const int32_t* wg_hcu, const int32_t* wg_part, int32_t nwg,
                             const gsbn_step_args* step, void* stream) {
-  if (!projs_dev || !wg_proj || !wg_hcu || !wg_part || !step || nwg <= 0 || step->kp_slot < 0 ||
-      step->kp_slot >= GSBN_KP_SLOTS || step->prec < GSBN_PREC_F32 || step->prec > GSBN_PREC_F16)
-    return GSBN_ERR_ARG;
-  hipStream_t s = (hipStream_t)stream;
-  const dim3 b(RC_THREADS);
-  switch (step->prec) {
-    case GSBN_PREC_F32:
-      launch_timed(rowcol_kernel_graded<GSBN_PREC_F32>,
-                   dim3(loop_grid(rowcol_kernel_graded<GSBN_PREC_F32>, RC_THREADS, 0, nwg)), b, 0,
-                   s, projs_dev, wg_proj, wg_hcu, wg_part, nwg, *step);
-      break;
-    case GSBN_PREC_BF16:
-      launch_timed(rowcol_kernel_graded<GSBN_PREC_BF16>,
-                   dim3(loop_grid(rowcol_kernel_graded<GSBN_PREC_BF16>, RC_THREADS, 0, nwg)), b,
-                   0, s, projs_dev, wg_proj, wg_hcu, wg_part, nwg, *step);
-      break;
-    default:
-      launch_timed(rowcol_kernel_graded<GSBN_PREC_F16>,
-                   dim3(loop_grid(rowcol_kernel_graded<GSBN_PREC_F16>, RC_THREADS, 0, nwg)), b,
-                   0, s, projs_dev, wg_proj, wg_hcu, wg_part, nwg, *step);
-      break;
-  }
-  return launch_status();
+  return launch_graded(projs_dev, nullptr, 0, wg_proj, wg_hcu, wg_part, nwg, step, stream);
+}
+
+int gsbn_proj_rowcol_graded_log(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs,
+                                int32_t n, const int32_t* wg_proj, const int32_t* wg_hcu,
+                                const int32_t* wg_part, int32_t nwg, const gsbn_step_args* step,
+                                void* stream) {
+  if (!log_ok(logs, n)) return GSBN_ERR_ARG;
+  return launch_graded(projs_dev, logs, n, wg_proj, wg_hcu, wg_part, nwg, step, stream);
 }
 
 int gsbn_proj_rowcol_graded_wave(const gsbn_rowcol_args* projs_dev, const int32_t* wg_proj,

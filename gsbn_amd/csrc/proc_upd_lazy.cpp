@@ -93,6 +93,7 @@ struct CoefTable {
 struct TableCache {
   std::map<std::array<uint32_t, 4>, std::unique_ptr<CoefTable>> m;
   uint64_t version = 0;
+  uint64_t log_version = 0; /* changes with any projection's recorded sweeps */
   int sim_end = 0;
   const CoefTable& get(float kzi, float kzj, float ke, float kp, int64_t need) {
     std::array<uint32_t, 4> key;
@@ -219,6 +220,22 @@ class Proj : public ProjRowOps {
     }
   }
   void materialize_kicks();
+  /* Deferred sweeps (see gsbn_sweep_log): the recorded sweeps' targets and
+   * learning rates, oldest first; their pj rows are in log_pj.  Every row and
+   * synapse is at floor_t or later, so a sweep to a target up to it changes
+   * nothing.  log_hook brings the device's log up to date (set by
+   * ProcUpdLazy). */
+  struct Sweep {
+    int target;
+    float kp;
+  };
+  vector<Sweep> log;
+  DevBuf<float> log_pj;
+  int floor_t = 0;
+  std::function<const gsbn_sweep_log*()> log_hook;
+  void apply_log(const gsbn_sweep_log* logs, int upto, float kp);
+  gsbn_all_args all_args(int target, float kp);
+  gsbn_jxx_args jxx_args(float prn);
   /* deferral ends (the kicks pending are applied first): structural changes
    * of the rows are not replayed; set by ProcUpdLazy */
   std::function<void()> eager_hook;
@@ -304,6 +321,7 @@ struct RowField : VecView {
   RowField(Proj* q, int f) : p(q), field(f) {}
   void pull(VecBase* v) override {
     p->flush_deferred();
+    if (!p->log.empty()) p->materialize_kicks(); /* recorded sweeps reach the rows */
     const size_t n = p->rowst.n;
     DevBuf<uint32_t> tmp;
     tmp.alloc(n);
@@ -810,6 +828,7 @@ void Proj::init_new(ProcParam proc_param, ProjParam proj_param, Database& db,
     views.push_back(e.v);
   }
   if (copy) {
+    floor_t = INT32_MIN;
     /* a snapshot without siq_ (written by the reference) resumes with no
      * row active at the first step, as the reference's resume does */
     resume_qi.resize((size_t)R, 0);
@@ -889,6 +908,7 @@ void Proj::prepare(int simstep) {
     if (v->status == VecBase::HOST_NEWER && v->view) {
       v->view->push(v);
       v->status = VecBase::SYNCED;
+      if (v == _ti || v == _tij) floor_t = INT32_MIN;
     }
   }
   if (_ii->host_version != ii_version || _di->host_version != di_version) {
@@ -901,9 +921,9 @@ void Proj::prepare(int simstep) {
   (void)simstep;
 }
 
-void Proj::update_all(int simstep, float old_prn) {
-  const float kp = _taupdt * old_prn;
-  const int target = simstep - 1;
+/* the arguments of a pass over every row and synapse to `target` with the
+ * table of learning rate kp */
+gsbn_all_args Proj::all_args(int target, float kp) {
   const CoefTable& t = table(kp, (int64_t)std::max(target, 0) + 2);
   gsbn_all_args a;
   memset(&a, 0, sizeof(a));
@@ -919,7 +939,6 @@ void Proj::update_all(int simstep, float old_prn) {
   a.table_len = (int32_t)t.len;
   a.syn = syn.p;
   a.rowst = rowst.p;
-  a.pj = _pj->gpu_data();
   a.prec = prec;
   a.syn16 = syn16.p;
   a.wij = wij16.p;
@@ -927,46 +946,52 @@ void Proj::update_all(int simstep, float old_prn) {
   a.e_scale = e_scale();
   if (dK) {
     a.dK = dK;
-    a.ii = _ii->gpu_data();
+    a.ii = ii_dev;
     a.dhist = dhist.p;
     a.dcnt = dcnt.p;
     a.kftj = _kftj;
   }
+  return a;
+}
+
+void Proj::update_all(int simstep, float old_prn) {
+  gsbn_all_args a = all_args(simstep - 1, _taupdt * old_prn);
+  a.pj = _pj->gpu_data();
+  if (dK) a.ii = _ii->gpu_data();
   Timing::get().begin(2, active_stream());
   op_check(gsbn_proj_all(&a, active_stream()), "gsbn_proj_all");
   Timing::get().end(2, active_stream());
+  floor_t = simstep - 1;
 }
 
-/* every pending column kick, applied (the state the reference's eager
- * column updates leave); the learning rate has not changed since the kicks
- * (a change sweeps them up) */
+/* the recorded sweeps, applied to every row and synapse, and the column
+ * kicks up to `upto`, whose learning rate since the last sweep is kp */
+void Proj::apply_log(const gsbn_sweep_log* logs, int upto, float kp) {
+  const int n = (int)log.size();
+  const gsbn_all_args a = all_args(upto, kp);
+  Timing::get().begin(2, active_stream());
+  op_check(gsbn_proj_sweep_log(&a, logs + _id, n, active_stream()), "gsbn_proj_sweep_log");
+  Timing::get().end(2, active_stream());
+  floor_t = log.back().target;
+  log.clear();
+  ++tcache->log_version;
+}
+
+/* every pending column kick and recorded sweep, applied (the state the
+ * reference's eager updates leave); kick_kp is the learning rate since the
+ * last recorded sweep */
 void Proj::materialize_kicks() {
-  if (!dK || !kicks_pending) return;
+  if (!dK || !(kicks_pending || !log.empty())) return;
   kicks_pending = false;
-  const CoefTable& t = table(kick_kp, (int64_t)std::max(kick_t, 0) + 2);
-  gsbn_all_args a;
-  memset(&a, 0, sizeof(a));
-  a.H = _dim_hcu;
-  a.M = _dim_mcu;
-  a.C = _dim_conn;
-  a.target = kick_t;
-  a.table = t.dev.p;
-  a.table_len = (int32_t)t.len;
-  a.syn = syn.p;
-  a.prec = prec;
-  a.syn16 = syn16.p;
-  a.wij = wij16.p;
-  a.p_scale = p_scale();
-  a.e_scale = e_scale();
-  a.dK = dK;
-  a.ii = ii_dev;
-  a.dhist = dhist.p;
-  a.dcnt = dcnt.p;
-  a.kftj = _kftj;
+  if (!log.empty()) {
+    apply_log(log_hook(), kick_t, kick_kp);
+    return;
+  }
+  const gsbn_all_args a = all_args(kick_t, kick_kp);
   op_check(gsbn_proj_materialize(&a, active_stream()), "gsbn_proj_materialize");
 }
 
-void Proj::update_jxx(float prn) {
+gsbn_jxx_args Proj::jxx_args(float prn) {
   Pop* dp = _ptr_dest_pop;
   gsbn_jxx_args a;
   memset(&a, 0, sizeof(a));
@@ -985,6 +1010,11 @@ void Proj::update_jxx(float prn) {
   a.kftj = _kftj;
   a.bgain = _bgain;
   a.eps = _eps;
+  return a;
+}
+
+void Proj::update_jxx(float prn) {
+  const gsbn_jxx_args a = jxx_args(prn);
   Timing::get().begin(3, active_stream());
   op_check(gsbn_proj_jxx(&a, active_stream()), "gsbn_proj_jxx");
   Timing::get().end(3, active_stream());
@@ -1271,13 +1301,39 @@ class ProcUpdLazy : public ProcedureBase {
    * g = 1, 2, 3 (plans -21, -22, -23) */
   int _wave_fixed = 0;
   /* deferred-columns K: column updates deferred through rings of K spike
-   * steps per unit (0: eager); see Proj::dK.  Same results for every K, a
-   * fraction of the column traffic.  Default where it applies: 8 for one
-   * network (its row update replays a ring of 8 from registers), 16 for a
-   * batch, whose one-wave-per-hypercolumn row/column launch is dominated by
-   * column walks at 8 (measured on 512 networks: 50.8 us at 8, 38.9 us at
-   * 16, 39.1 us at 32 and 64). */
+   * steps per unit (0: eager); see Proj::dK.  Same results for every K.
+   * GlobalVar deferred-columns reports K, 8 for one network and 16 for a
+   * batch when it is not given; the rings then hold kRing steps (GlobalVar
+   * deferred-ring) and are walked between the steps. */
   static constexpr int kDeferDefault = 8, kDeferBatch = 16;
+  /* Without the argument, every kWalkEvery steps the units with kWalkDue or
+   * more spikes since their last walk are walked by a launch of its own over
+   * the whole device; at most kWalkDue - 1 + kWalkEvery < 63 spikes are then
+   * ever pending, so no step walks a column itself (a walk inside a step holds
+   * the step: 9900 slots by the few workgroups of one hypercolumn) */
+  static constexpr int kRing = 64, kWalkEvery = 32, kWalkDue = 30;
+  int _walk_age = 0; /* steps since the last walk launch */
+  /* deferred-sweeps 1 (with deferred column updates, not with a forced
+   * chained step): learning-rate changes are recorded instead of sweeping
+   * every synapse, up to GSBN_SWEEP_LOG of them, and applied by the row and
+   * column updates that next touch a synapse, by one pass when the log is
+   * full, when the state is read or written from the host, or at the end of
+   * the schedule.  The log is the same length for every projection.
+   * Default: from kSweepDefer synapses.  A step with recorded sweeps costs 2
+   * to 4 us more (its row updates look through them), about 100 to 200 us per
+   * sweep of the recall schedules, and a sweep moves 36-64 bytes per synapse
+   * at 4.7 TB/s: 3.7e6 synapses in fp16 (29 us a sweep) ran 33.4 ms with
+   * sweeps and 36.5 recorded, 3e7 in fp32 (1.3 ms) 99 and 75, 1e8 in bf16
+   * (1.4 ms) 178 and 115, 6.6e8 in fp32 (10 ms) 290 and 164. */
+  static constexpr int64_t kSweepDefer = 10000000;
+  int _sweep_defer = -1;
+  DevBuf<gsbn_sweep_log> _logs_dev; /* per projection */
+  uint64_t _logs_tables = ~0ull, _logs_seen = ~0ull; /* what the device's logs hold */
+  int _best_split = 0;
+  size_t nlog() const { return _list_proj.empty() ? 0 : _list_proj[0]->log.size(); }
+  const gsbn_sweep_log* logs();
+  void apply_logs(int upto, float prn);
+  void record_sweep(int simstep, float old_prn, float prn, const gsbn_step_args& st);
   int _defer_arg = -1; /* the argument, -1 when not given */
   int _defer_k = kDeferDefault;
   void end_deferral();
@@ -1313,6 +1369,80 @@ void ProcUpdLazy::flush_deferred() {
   Timing::get().end(1, s);
 }
 
+/* the projections' recorded sweeps on the device (log entries hold table
+ * pointers, so a rebuilt table refreshes them) */
+const gsbn_sweep_log* ProcUpdLazy::logs() {
+  for (auto* q : _list_proj)
+    for (auto& e : q->log) (void)q->table(e.kp, (int64_t)std::max(e.target, 0) + 2);
+  if (_logs_dev.p && _logs_seen == _tables.log_version && _logs_tables == _tables.version)
+    return _logs_dev.p;
+  vector<gsbn_sweep_log> h(_list_proj.size());
+  memset(h.data(), 0, h.size() * sizeof(h[0]));
+  for (size_t i = 0; i < h.size(); ++i) {
+    Proj* q = _list_proj[i];
+    h[i].pj = q->log_pj.p;
+    for (size_t k = 0; k < q->log.size(); ++k) {
+      const CoefTable& t = q->table(q->log[k].kp, (int64_t)std::max(q->log[k].target, 0) + 2);
+      h[i].e[k].table = t.dev.p;
+      h[i].e[k].table_len = (int32_t)t.len;
+      h[i].e[k].target = q->log[k].target;
+      h[i].e[k].kp = q->log[k].kp;
+    }
+  }
+  _logs_dev.upload(h.data(), h.size());
+  _logs_seen = _tables.log_version;
+  _logs_tables = _tables.version;
+  return _logs_dev.p;
+}
+
+/* every projection's recorded sweeps applied (some may be already, by a read
+ * of their state: their logs are empty), so that all logs are empty */
+void ProcUpdLazy::apply_logs(int upto, float prn) {
+  const gsbn_sweep_log* lg = logs(); /* every log, before any is cleared */
+  for (auto* q : _list_proj)
+    if (!q->log.empty()) q->apply_log(lg, upto, q->_taupdt * prn);
+}
+
+/* a learning-rate change at simstep, recorded: the sweep to simstep - 1 with
+ * the old rate, and the postsynaptic update of the step */
+void ProcUpdLazy::record_sweep(int simstep, float old_prn, float prn, const gsbn_step_args& st) {
+  const int target = simstep - 1;
+  /* logs of one length: a projection whose log was applied on its own (its
+   * state was read) brings the others along */
+  for (auto* q : _list_proj)
+    if (q->log.size() != nlog() || nlog() == GSBN_SWEEP_LOG) {
+      apply_logs(target, old_prn);
+      break;
+    }
+  bool need = false;
+  for (auto* q : _list_proj) need = need || target > q->floor_t;
+  const int slot = (int)nlog();
+  hipStream_t s = active_stream();
+  if (need)
+    for (auto* q : _list_proj) {
+      if (!q->log_pj.p) q->log_pj.alloc((size_t)GSBN_SWEEP_LOG * q->_dim_hcu * q->_dim_mcu);
+      q->log.push_back({target, q->_taupdt * old_prn});
+      ++_tables.log_version;
+    }
+  Timing::get().begin(3, s);
+  if (_batch && need) {
+    /* the log's pj rows are written here, so it has to be on the device */
+    (void)logs();
+    op_check(gsbn_proj_jxx_mark_batch(_pop_dev.p, _logs_dev.p, slot, _wg_pop.p, _wg_pop_hcu.p,
+                                      _nwg_pop, &st, s),
+             "gsbn_proj_jxx_mark_batch");
+  } else {
+    for (auto* q : _list_proj) {
+      const gsbn_jxx_args a = q->jxx_args(prn);
+      if (need)
+        op_check(gsbn_proj_jxx_mark(&a, q->log_pj.p + (size_t)slot * a.N, s), "gsbn_proj_jxx_mark");
+      else
+        op_check(gsbn_proj_jxx(&a, s), "gsbn_proj_jxx");
+    }
+  }
+  Timing::get().end(3, s);
+}
+
 /* column updates become eager again (a structural change of the rows is
  * coming, which the replay of pending kicks cannot follow): the pending
  * row/column work and every pending kick are applied first */
@@ -1324,8 +1454,10 @@ void ProcUpdLazy::end_deferral() {
     q->dK = 0;
   }
   _defer_k = 0;
+  _sweep_defer = 0;
   _args_dirty = true;
   _glv.puti("deferred-columns", 0);
+  _glv.puti("deferred-sweeps", 0);
 }
 
 /* the plan of this step; *timed while tuning (the step belongs to run
@@ -1382,7 +1514,7 @@ int ProcUpdLazy::rowcol_parts(hipStream_t s, bool* timed) {
 void ProcUpdLazy::finish_tuning() {
   const size_t nc = _cand.size();
   hip_check(hipEventSynchronize(_tev.back()), "hipEventSynchronize");
-  float best = 0.0f;
+  float best = 0.0f, best_split = 0.0f;
   for (size_t c = 0; c < nc; ++c) {
     vector<float> t;
     for (int k = 0; k < kTuneSamples; ++k) {
@@ -1398,6 +1530,10 @@ void ProcUpdLazy::finish_tuning() {
     if (c == 0 || med < best) {
       best = med;
       _parts = _cand[c];
+    }
+    if (_cand[c] > 0 && (_best_split == 0 || med < best_split)) {
+      best_split = med;
+      _best_split = _cand[c];
     }
   }
   _tuned = true;
@@ -1430,6 +1566,7 @@ void ProcUpdLazy::init(SolverParam solver_param, Database& db, bool copy) {
     throw Error(-2, "ProcUpdLazy: ovf-keep and ovf-cap must be >= 0");
   if (_wave_fixed < 0 || _wave_fixed > 4)
     throw Error(-2, "ProcUpdLazy: rowcol-wave must be in [0, 4]");
+  par.argi("deferred-sweeps", _sweep_defer);
   par.argi("deferred-columns", _defer_arg);
   if (_defer_arg != -1 &&
       (_defer_arg < 0 || _defer_arg == 1 || _defer_arg > 64 || (_defer_arg & (_defer_arg - 1))))
@@ -1617,6 +1754,16 @@ void ProcUpdLazy::refresh_args(int simstep) {
 void ProcUpdLazy::update_gpu() {
   int cycle_flag = 0;
   GSBN_CHECK(_glv.geti("cycle-flag", cycle_flag), "cycle-flag");
+  if (cycle_flag < 0) {
+    /* the schedule is over: no sweep stays behind */
+    const gsbn_sweep_log* lg = nullptr;
+    for (auto* q : _list_proj)
+      if (!q->log.empty()) {
+        if (!lg) lg = logs();
+        q->kicks_pending = false;
+        q->apply_log(lg, q->kick_t, q->kick_kp);
+      }
+  }
   if (cycle_flag != 1) return;
   int simstep = 0, lginp_idx = 0, wmask_idx = 0;
   float prn = 0, old_prn = 0;
@@ -1708,11 +1855,20 @@ void ProcUpdLazy::update_gpu() {
     if (_defer_k) {
       _fusable = false;
       for (auto* q : _list_proj) {
-        q->enable_deferred(_defer_k);
+        q->enable_deferred(_defer_arg >= 0 ? _defer_k : kRing);
         q->eager_hook = [this]() { end_deferral(); };
+        q->log_hook = [this]() { return logs(); };
       }
     }
+    if (_sweep_defer < 0) {
+      int64_t synapses = 0;
+      for (auto* q : _list_proj) synapses += q->nsyn;
+      _sweep_defer = synapses >= kSweepDefer ? 1 : 0;
+    }
+    if (!_defer_k || _chain_fixed > 0) _sweep_defer = 0;
+    _glv.puti("deferred-sweeps", _sweep_defer ? 1 : 0);
     _glv.puti("deferred-columns", _defer_k);
+    _glv.puti("deferred-ring", _defer_k ? _list_proj[0]->dK : 0);
     /* GlobalVar pop-wave: units per lane of the one-wave population launch
      * of a batch (0: the block kernel, or no batch) */
     _glv.puti("pop-wave", _batch ? _pop_upl : 0);
@@ -1779,6 +1935,12 @@ void ProcUpdLazy::update_gpu() {
     timed = false;
     _chain_warm = 0;
     if (plan == -1) plan = _parts0;
+  }
+  /* a chained launch has no form for recorded sweeps: the best of the
+   * splits runs while there are any */
+  if (_sweep_defer && plan == -2 && (sweep || nlog())) {
+    plan = _best_split ? _best_split : _parts0;
+    timed = false;
   }
   if (plan != -2 && _pending) flush_deferred();
   /* the row overflow queue: passed to every one-wave population launch (it
@@ -1891,13 +2053,46 @@ void ProcUpdLazy::update_gpu() {
     for (auto* p : _list_pop) p->flush_pending = true;
     if (sweep) {
       for (auto* q : _list_proj) {
-        q->update_all(simstep, old_prn);
+        if (!_sweep_defer) q->update_all(simstep, old_prn);
         sweep_synapses += (int64_t)q->_dim_hcu * q->_dim_conn * q->_dim_mcu;
       }
       sweeps++;
-      for (auto* q : _list_proj) q->update_jxx(prn);
+      if (_sweep_defer)
+        record_sweep(simstep, old_prn, prn, st);
+      else
+        for (auto* q : _list_proj) q->update_jxx(prn);
     }
-    if (!_list_proj.empty()) {
+    /* one length for all logs: see record_sweep */
+    const int nl = (int)nlog();
+    for (auto* q : _list_proj)
+      if ((int)q->log.size() != nl) {
+        apply_logs(simstep - 1, prn);
+        break;
+      }
+    if (!_list_proj.empty() && nlog()) {
+      const int n = (int)nlog();
+      const gsbn_sweep_log* lg = logs();
+      Timing::get().begin(1, stream);
+      if (_batch && plan == -20) {
+        op_check(gsbn_proj_rowcol_batch_wave_log(_proj_dev.p, lg, n, _wg_proj.p, _wg_proj_hcu.p,
+                                                 _nhcu_proj, &st, stream),
+                 "gsbn_proj_rowcol_batch_wave_log");
+      } else if (_batch && plan <= -10) {
+        /* (the graded one-wave plans take the workgroup form's map) */
+        const int g = plan <= -20 ? -20 - plan : -10 - plan;
+        if (!_gmap_n[g]) build_graded_map(g);
+        op_check(gsbn_proj_rowcol_graded_log(_proj_dev.p, lg, n, _gmap_proj[g].p, _gmap_hcu[g].p,
+                                             _gmap_part[g].p, _gmap_n[g], &st, stream),
+                 "gsbn_proj_rowcol_graded_log");
+      } else if (_batch) {
+        op_check(gsbn_proj_rowcol_batch_log(_proj_dev.p, lg, n, _wg_proj.p, _wg_proj_hcu.p,
+                                            _nhcu_proj, plan, &st, stream),
+                 "gsbn_proj_rowcol_batch_log");
+      } else {
+        op_check(gsbn_proj_rowcol_log(&ra, lg, n, stream), "gsbn_proj_rowcol_log");
+      }
+      Timing::get().end(1, stream);
+    } else if (!_list_proj.empty()) {
       Timing::get().begin(1, stream);
       if (_batch && plan <= -21 && plan >= -23) {
         const int g = -20 - plan;
@@ -1922,6 +2117,21 @@ void ProcUpdLazy::update_gpu() {
       else
         op_check(gsbn_proj_rowcol(&ra, stream), "gsbn_proj_rowcol");
       Timing::get().end(1, stream);
+    }
+  }
+  /* (a chained step's row updates come with the next launch: its walks stay
+   * inside the steps, as its column workgroups run them in parallel) */
+  if (_defer_k && _defer_arg < 0 && plan != -2 && ++_walk_age >= kWalkEvery) {
+    _walk_age = 0;
+    const int n = (int)nlog();
+    const gsbn_sweep_log* lg = n ? logs() : nullptr;
+    if (_batch) {
+      op_check(gsbn_proj_walk_batch(_pop_dev.p, _wg_pop.p, _wg_pop_hcu.p, _nwg_pop, _proj_dev.p,
+                                    _wg_proj.p, _wg_proj_hcu.p, _nhcu_proj, _max_slots, kWalkDue,
+                                    lg, n, &st, stream),
+               "gsbn_proj_walk_batch");
+    } else {
+      op_check(gsbn_proj_walk(&pa.proj0, &ra, kWalkDue, lg, n, stream), "gsbn_proj_walk");
     }
   }
   for (auto* q : _list_proj) q->update_que(_exec);

@@ -245,6 +245,30 @@ int gsbn_proj_all(const gsbn_all_args* a, void* stream);
  * pj and rowst are not used. */
 int gsbn_proj_materialize(const gsbn_all_args* a, void* stream);
 
+/* Deferred sweeps: a full catch-up (gsbn_proj_all) of a learning-rate change
+ * touches every synapse.  Instead it can be recorded: `target` (simstep - 1),
+ * the learning rate until then (kp) with its table, and the postsynaptic pj at
+ * that time.  A row or column update of a synapse (gsbn_proj_rowcol_log and
+ * its batched forms) first applies the recorded sweeps past its tij, oldest
+ * first, between the pending column kicks in step order, each as the sweep
+ * would have; gsbn_proj_sweep_log applies them to every row and synapse.  The
+ * results are those of the sweeps.  Needs deferred column updates (dK > 0). */
+#define GSBN_SWEEP_LOG 16
+typedef struct {
+  const float* table;
+  int32_t table_len, target;
+  float kp;
+  int32_t pad;
+} gsbn_sweep_entry;
+typedef struct {
+  gsbn_sweep_entry e[GSBN_SWEEP_LOG]; /* ascending targets */
+  float* pj;                          /* [GSBN_SWEEP_LOG][H * M] */
+} gsbn_sweep_log;
+/* apply the first n recorded sweeps of log (device memory) to every row and
+ * synapse, then the pending column kicks up to a->target (table: the current
+ * learning rate's); kp and pj of `a` are not used */
+int gsbn_proj_sweep_log(const gsbn_all_args* a, const gsbn_sweep_log* log, int32_t n, void* stream);
+
 /* Postsynaptic Euler update and bias (Proj.cpp:310-363), standalone form. */
 typedef struct {
   int32_t N;
@@ -253,6 +277,13 @@ typedef struct {
   float kp, ke, kzj, kepsc, kftj, bgain, eps;
 } gsbn_jxx_args;
 int gsbn_proj_jxx(const gsbn_jxx_args* a, void* stream);
+/* the same, keeping pj as it was in pj_before[N] (a recorded sweep's pj) */
+int gsbn_proj_jxx_mark(const gsbn_jxx_args* a, float* pj_before, void* stream);
+/* the same for every population of a batch (one incoming projection each,
+ * logs[proj0.bidx].pj row `slot` receives pj), one workgroup per HCU */
+int gsbn_proj_jxx_mark_batch(const gsbn_pop_args* pops_dev, gsbn_sweep_log* logs, int32_t slot,
+                             const int32_t* wg_pop, const int32_t* wg_hcu, int32_t nwg,
+                             const gsbn_step_args* step, void* stream);
 
 /* Row and column lazy updates of one step (Proj.cpp:365-536, 667-760).
  * Grid: `parts` workgroups per destination HCU; part q of HCU h takes the
@@ -303,6 +334,27 @@ typedef struct {
   int32_t dK, dpad;
 } gsbn_rowcol_args;
 int gsbn_proj_rowcol(const gsbn_rowcol_args* a, void* stream);
+
+/* gsbn_proj_rowcol with the first n recorded sweeps of log (device memory,
+ * 0 < n <= GSBN_SWEEP_LOG) pending */
+int gsbn_proj_rowcol_log(const gsbn_rowcol_args* a, const gsbn_sweep_log* log, int32_t n,
+                         void* stream);
+
+/* Column walks between steps: every unit of p's projection whose spikes since
+ * its last walk number `due` or more has its pending column kicks (of steps
+ * up to a->simstep) applied in every slot with ii >= 0, so that a ring of dK
+ * steps with walks every dK / 2 steps never lists a unit within a step.  `a`:
+ * that projection's arguments with p's walk lists; log, n: its recorded
+ * sweeps (n = 0: none).  After the row/column update of step a->simstep. */
+int gsbn_proj_walk(const gsbn_pop_proj* p, const gsbn_rowcol_args* a, int32_t due,
+                   const gsbn_sweep_log* log, int32_t n, void* stream);
+/* the same for every projection of a batch (proj0 of each population);
+ * max_slots: the largest slot count */
+int gsbn_proj_walk_batch(const gsbn_pop_args* pops_dev, const int32_t* wg_pop,
+                         const int32_t* wg_pop_hcu, int32_t nwg, const gsbn_rowcol_args* projs_dev,
+                         const int32_t* wg_proj, const int32_t* wg_proj_hcu, int32_t nhcu,
+                         int32_t max_slots, int32_t due, const gsbn_sweep_log* logs, int32_t n,
+                         const gsbn_step_args* step, void* stream);
 
 /* Row/column workgroups of trace form `prec` that the current device holds
  * at once (resident workgroups per CU times CUs): a split whose grid
@@ -359,6 +411,20 @@ int gsbn_proj_rowcol_graded(const gsbn_rowcol_args* projs_dev, const int32_t* wg
 int gsbn_proj_rowcol_graded_wave(const gsbn_rowcol_args* projs_dev, const int32_t* wg_proj,
                                  const int32_t* wg_hcu, const int32_t* wg_part, int32_t nwg,
                                  const gsbn_step_args* step, void* stream);
+
+/* gsbn_proj_rowcol_batch, _batch_wave and _graded with the first n recorded
+ * sweeps of every projection pending: logs[p] for projs_dev[p] */
+int gsbn_proj_rowcol_batch_log(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs,
+                               int32_t n, const int32_t* wg_proj, const int32_t* wg_hcu,
+                               int32_t nhcu, int32_t parts, const gsbn_step_args* step,
+                               void* stream);
+int gsbn_proj_rowcol_batch_wave_log(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs,
+                                    int32_t n, const int32_t* wg_proj, const int32_t* wg_hcu,
+                                    int32_t nhcu, const gsbn_step_args* step, void* stream);
+int gsbn_proj_rowcol_graded_log(const gsbn_rowcol_args* projs_dev, const gsbn_sweep_log* logs,
+                                int32_t n, const int32_t* wg_proj, const int32_t* wg_hcu,
+                                const int32_t* wg_part, int32_t nwg, const gsbn_step_args* step,
+                                void* stream);
 
 /* One launch per executed step without a sweep (ProcUpdLazy.cpp:112-123
  * and 153-165 in one kernel), for populations with one incoming projection

@@ -105,6 +105,8 @@ def apply_plan(spec, plan: str):
         spec.fused_step = 1
     elif plan == "chained":
         spec.chained_step = 1
+    elif plan == "block":
+        spec.block_step = 1
     elif plan == "wave":
         spec.rowcol_wave = 1
         spec.chained_step = -1
@@ -208,7 +210,8 @@ def cpu_only(args):
                                    args.warmup + args.steps, dt)}))
 
 
-PLAN_NAMES = {-1: "fused", -2: "chained", -20: "wave"}
+BLOCK = -3
+PLAN_NAMES = {-1: "fused", -2: "chained", BLOCK: "block", -20: "wave"}
 
 
 def plan_name(parts: int) -> str:
@@ -221,7 +224,7 @@ def plan_name(parts: int) -> str:
 
 def fixed_plan(spec) -> bool:
     return bool(spec.fused_step or spec.chained_step > 0 or spec.rowcol_parts or
-                spec.rowcol_graded or spec.rowcol_wave)
+                spec.rowcol_graded or spec.rowcol_wave or spec.block_step)
 
 
 def fix_plan(spec, parts: int):
@@ -230,6 +233,8 @@ def fix_plan(spec, parts: int):
         spec.fused_step = 1
     elif parts == -2:
         spec.chained_step = 1
+    elif parts == BLOCK:
+        spec.block_step = 1
     elif parts <= -20:
         spec.rowcol_wave = -19 - parts
         spec.chained_step = -1
@@ -255,10 +260,12 @@ def settle_plan(spec, max_steps: int = 5000):
             if s.step(1) == 0:
                 break
             n += 1
-            if s.glob("plan-tuned"):
+            if s.glob("plan-tuned") or s.glob("block-step"):
                 break
         parts = s.glob("rowcol-parts")
         tuned = s.glob("plan-tuned")
+        if s.glob("block-step"):  # calls of several steps, as the timed ones
+            parts, tuned = BLOCK, 1
         s.close()
     if not tuned:
         raise SystemExit("bench: the plan tuner did not finish within %d steps" % n)
@@ -304,7 +311,7 @@ def measure(spec, steps, warmup, step_times=0):
             raise SystemExit("bench: needs --warmup >= 1 and --steps >= 1")
         _steps(s, warmup)
         s.sync()
-        parts = s.glob("rowcol-parts")
+        parts = BLOCK if spec.block_step else s.glob("rowcol-parts")
         deferred = s.glob("deferred-columns")
         pop_wave = s.glob("pop-wave")
         t0 = time.perf_counter()
@@ -342,18 +349,21 @@ def measure(spec, steps, warmup, step_times=0):
     cols = int(k1[1] - k0[1])
     sweep = int(k1[2] - k0[2])
     bpu = BYTES_PER_SYN_UPDATE[spec.trace_precision]
-    # one launch per step (the fused plan, -1, or the chained plan, -2) is
-    # timed as kind 6; split plans time the population launches (kind 0) and
-    # the row/column launches (kind 1)
-    one_launch = parts in (-1, -2)
+    # one launch per step (the fused plan, -1, or the chained plan, -2) or per
+    # several (block steps) is timed as kind 6; split plans time the population
+    # launches (kind 0) and the row/column launches (kind 1)
+    one_launch = parts in (-1, -2, BLOCK)
     batch = len(spec.pops) > 1
-    rc_name = (("chained_kernel" if parts == -2 else "step_kernel_batch" if batch else "step_kernel")
+    rc_name = (("block_kernel" if parts == BLOCK else "chained_kernel" if parts == -2
+                else "step_kernel_batch" if batch else "step_kernel")
                if one_launch else "rowcol_kernel_batch_wave" if parts == -20
                else "rowcol_kernel_graded_wave" if parts <= -21
                else "rowcol_kernel_graded" if parts <= -10
                else "rowcol_kernel_batch" if batch else "rowcol_kernel")
     kind = 6 if one_launch else 1
     other = int(launches[1]) if one_launch else int(launches[6])
+    if parts == BLOCK:
+        other -= int(k1[4] - k0[4])  # a sweep step has launches of its own
     if other:
         raise SystemExit("bench: %d launches of another plan in the kernel window" % other)
     kernels = {}
@@ -628,7 +638,7 @@ def main():
                          "(reference point for rocprofv3 FETCH_SIZE / WRITE_SIZE)")
     ap.add_argument("--plan", default="auto",
                     help="step plan: auto (tuned online), split:N (N row/column workgroups "
-                         "per HCU), fused, chained, or for batches wave (one wave per HCU), "
+                         "per HCU), fused, chained, block, or for batches wave (one wave per HCU), "
                          "graded:G (parts per size bucket, G = 1-3) or graded-wave:G (the "
                          "same with one wave per part)")
     ap.add_argument("--deferred", type=int, default=None, metavar="K",

@@ -159,6 +159,10 @@ class NetSpec:
     # through rings of K spike steps per postsynaptic unit; 0: eager; None:
     # ProcUpdLazy's default (where it applies: 8 for one network, 16 for a batch)
     deferred_columns: Optional[int] = None
+    # block_step 0: steps are never run several per launch; 1: every step is
+    # run that way; None: ProcUpdLazy's default (in calls of several steps,
+    # where it applies)
+    block_step: Optional[int] = None
     # deferred_sweeps 0: every learning-rate change sweeps all synapses at
     # once; 1: it is recorded and applied later, where deferred columns apply;
     # None: ProcUpdLazy's default (recorded from 1e7 synapses on)
@@ -332,6 +336,8 @@ def prototxt(spec: NetSpec, stim_path: str, conn_path: str, rec_dir: str,
         L.append('  argi { key: "rowcol-wave" val: %d }' % spec.rowcol_wave)
     if spec.deferred_columns is not None:
         L.append('  argi { key: "deferred-columns" val: %d }' % spec.deferred_columns)
+    if spec.block_step is not None:
+        L.append('  argi { key: "block-step" val: %d }' % spec.block_step)
     if spec.deferred_sweeps is not None:
         L.append('  argi { key: "deferred-sweeps" val: %d }' % spec.deferred_sweeps)
     if spec.pop_wave is not None:

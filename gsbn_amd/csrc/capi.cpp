@@ -181,10 +181,12 @@ int64_t gsbn_solver_step(gsbn_solver* s, int64_t nsteps) {
     gsbn::GlobalVar glv;
     int f = 0;
     glv.geti("cycle-flag", f);
+    s->s->begin_steps(nsteps);
     while (n < nsteps && f >= 0) {
       f = s->s->step();
       ++n;
     }
+    s->s->flush();
     return n;
   } catch (const std::exception& e) {
     return fail(e);
@@ -196,6 +198,7 @@ int64_t gsbn_solver_run(gsbn_solver* s) { return gsbn_solver_step(s, INT64_MAX);
 int gsbn_solver_sync(gsbn_solver* s) {
   return guard([&] {
     if (!s || !s->s) throw Error(GSBN_ERR_ARG, "null solver");
+    s->s->flush();
     gsbn::hip_check(hipStreamSynchronize(s->s->stream()), "hipStreamSynchronize");
     return 0;
   });
@@ -281,6 +284,7 @@ int gsbn_solver_check(gsbn_solver* s, int32_t* correct, int32_t* total, int32_t*
 int gsbn_solver_work(gsbn_solver* s, int64_t* out5) {
   return guard([&] {
     if (!s || !s->s || !out5) throw Error(GSBN_ERR_ARG, "null argument");
+    s->s->flush();
     if (!gsbn::updlazy_work(s->s->upd(), out5)) throw Error(GSBN_ERR_STATE, "no ProcUpdLazy");
     return 0;
   });

@@ -404,7 +404,9 @@ int Solver::step() {
 void Solver::run() {
   int f = 0;
   _glv.geti("cycle-flag", f);
+  begin_steps(INT64_MAX);
   while (f >= 0) f = step();
+  flush();
 }
 
 /* ------------------------------------------------------------------ */

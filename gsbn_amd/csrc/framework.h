@@ -75,6 +75,18 @@ class SolverMemory : public std::enable_shared_from_this<SolverMemory> {
   /* device -> host after the work queued on s; dst is complete on return */
   void download(void* dst, const void* src, size_t bytes, hipStream_t s);
 
+  /* Set by a procedure that holds executed steps back to run several in one
+   * launch: run_held launches them (before any vector moves to or from the
+   * host, and at the end of every solver call), and count_spikes adds the
+   * spikes of the step executed last to counts[all units] when it is held
+   * (false: it is not, the spike vectors are this step's). */
+  std::function<void()> run_held;
+  std::function<bool(int32_t* counts)> count_spikes;
+  int64_t call_steps = 1; /* steps the solver call being served was asked for */
+  void run_held_steps() {
+    if (run_held) run_held();
+  }
+
  private:
   struct Chunk {
     char* base;
@@ -270,6 +282,7 @@ class SyncVector : public VecBase {
   /* the device copy was modified by a kernel */
   void mark_device() { status = DEVICE_NEWER; }
   void mark_host() {
+    run_held_steps();
     status = HOST_NEWER;
     ++host_version;
     ++host_epoch();
@@ -288,9 +301,13 @@ class SyncVector : public VecBase {
   void resize_raw(size_t n) override { resize(n); }
 
   static hipStream_t stream() { return active_stream(); }
+  static void run_held_steps() {
+    if (active_memory()) active_memory()->run_held_steps();
+  }
 
   void to_host() {
     if (status != DEVICE_NEWER) return;
+    run_held_steps();
     ++host_epoch();
     if (before_host_read) before_host_read();
     if (view) {
@@ -304,6 +321,7 @@ class SyncVector : public VecBase {
   }
   bool read_device(void* out) override {
     if (status != DEVICE_NEWER || !n_) return false;
+    run_held_steps();
     if (before_host_read) before_host_read();
     if (view) return view->pull_to(out, n_);
     mem_->download(out, d_, n_ * sizeof(T), stream());
@@ -592,6 +610,13 @@ class Solver {
   Database& db() { return _database; }
   Upd& upd() { return _upd; }
   hipStream_t stream() const { return _stream; }
+  /* the number of steps the caller is about to ask for */
+  void begin_steps(int64_t n) { _mem->call_steps = n; }
+  /* steps held back by a procedure are launched */
+  void flush() {
+    activate();
+    _mem->run_held_steps();
+  }
   /* this solver's stream and memory become the calling thread's */
   void activate() {
     active_stream() = _stream;

@@ -137,6 +137,13 @@ unsigned loop_grid(K kernel, int threads, size_t lds, int64_t n) {
   return (unsigned)n;
 }
 
+/* LDS operations of a wave are processed in order; this only keeps the
+ * compiler from moving them across */
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 /* exclusive prefix sum across the workgroup (blockDim multiple of 64);
  * sh needs blockDim/64 + 1 ints */
 __device__ int block_excl_scan(int v, int* sh, int* total) {
@@ -381,6 +388,13 @@ struct SynIO {
       s.pij = gsbn_unpack_trace(PREC, (uint16_t)gsbn_pack_trace(PREC, s.pij, ps), pinv);
       s.eij = gsbn_unpack_trace(PREC, (uint16_t)gsbn_pack_trace(PREC, s.eij, es), einv);
     }
+  }
+  /* a column increment on its own */
+  __device__ __forceinline__ void add_zj2(int64_t i, float k) const {
+    if constexpr (PREC == GSBN_PREC_F32)
+      syn[i].zj2 += k;
+    else
+      syn16[i].zj2 += k;
   }
   __device__ __forceinline__ void store_tij(int64_t i, int t) const {
     if constexpr (PREC == GSBN_PREC_F32)
@@ -2081,6 +2095,445 @@ __global__ void __launch_bounds__(RC_THREADS) chained_kernel(gsbn_pop_args a, gs
   rowcol_body<PREC, false, false>(b, q, h, w - h * b.parts);
 }
 
+/* ---- block step: several executed steps of a hypercolumn in one launch ----
+ *
+ * A spike of step s activates rows at step s + di + 2 at the earliest, so
+ * during dmin + 2 steps a hypercolumn depends on nothing that happens in the
+ * same steps elsewhere: its active rows are in the ring already.  One workgroup
+ * runs them all, its units' state and traces in registers, support
+ * contributions and newest kicks in LDS.
+ *
+ * What bounds it: a chain of dependent latencies per step, so the work is
+ * spread over waves by role and meets at two barriers per step:
+ *   wave 0       support, WTA, soft-max, spikes (UPL units per lane, wave
+ *                scans and reductions, no barriers of its own);
+ *   UPL waves    the next step's draws and the traces (pj, bj, which the next
+ *                step needs, do not depend on this step's spikes); after the
+ *                spikes, the queue push;
+ *   the others   this step's active rows (they need the step's spikes only
+ *                for zj2's increment, added after the first barrier), and the
+ *                next step's ring words.
+ * Rows past RCAP (a busier step than the LDS holds) are run after the first
+ * barrier by the row waves in passes, their contributions through memory.
+ * Outputs that only the last step leaves (act, draws, spike lists, active
+ * rows) are stored once.
+ * Measured, launches of 3 steps (delay 1): 10 HCUs x 10 units 13.6 us, where
+ * the split plan's six launches took 31 us; 100 x 100 24.3 us (45); 24 networks
+ * of 16 to 128 units, 860 HCUs, 38 us (54). */
+#define BLK_LIST 512 /* active rows of a step held in LDS; the rest through rows2 / rows_list */
+
+struct BlockArgs {
+  int nlog, simstep, exec, nsteps, kp_slot;
+  float prn;
+  int64_t lg_off, wm_off;
+  uint32_t count_mask;      /* bit s: step s's spikes are counted in check */
+  int32_t* check;           /* [all units], NULL when count_mask is 0 */
+  const float* lginp_base;  /* the first population's lginp (units before a population) */
+};
+
+template <int PREC, bool LOG, int UPL, int T, int RCAP>
+__global__ void __launch_bounds__(T)
+    block_kernel(const gsbn_pop_args* __restrict__ pops, const gsbn_rowcol_args* __restrict__ projs,
+                 const int32_t* __restrict__ wg_pop, const int32_t* __restrict__ wg_hcu,
+                 int32_t* const* __restrict__ rows2, const gsbn_sweep_log* __restrict__ logs,
+                 const BlockArgs g) {
+  constexpr int MX = 64 * UPL, NW = T / 64, RW0 = 1 + UPL, RT = T - 64 * RW0, NRW = NW - RW0;
+  static_assert(NRW > 0 && RT >= RCAP, "row waves");
+  __shared__ float sh_u[2][MX], sh_xi[2][MX], sh_pj[2][MX], sh_bj[2][MX];
+  __shared__ __attribute__((aligned(16))) float sh_act[MX];
+  __shared__ float sh_con[RCAP][MX];
+  __shared__ gsbn_row_rec sh_row[RCAP];
+  __shared__ int sh_sj[MX], sh_dcnt[MX], sh_k8[8][MX], sh_spk[MX];
+  __shared__ int sh_list[2][BLK_LIST];
+  __shared__ int sh_wsum[4][NRW];
+  __shared__ int sh_nspk;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rt = tid - 64 * RW0; /* row thread */
+  const gsbn_pop_args& a = pops[wg_pop[blockIdx.x]];
+  const gsbn_pop_proj& p0 = a.proj0;
+  const gsbn_rowcol_args& b = projs[p0.bidx];
+  touch_lines<sizeof(gsbn_pop_args)>(&a);
+  touch_lines<sizeof(gsbn_rowcol_args)>(&b);
+  const int h = wg_hcu[blockIdx.x];
+  const int M = a.M, C = p0.C, W = p0.W, K = p0.dK;
+  const int64_t hC = (int64_t)h * C;
+  const SynIO<PREC> io(b);
+  const float* table = b.tables[g.kp_slot];
+  const int table_len = b.table_lens[g.kp_slot];
+  const float kp = p0.taupdt * g.prn;
+  const bool learn = kp != 0.0f;
+  int32_t* const list_mem[2] = {p0.rows_list + hC, rows2[p0.bidx] + hC};
+  const gsbn_sweep_log* lg = LOG ? logs + p0.bidx : nullptr; /* rows2: the second list of rows past BLK_LIST */
+
+  /* the ring words of exec step x into registers, cleared, with their counts
+   * per band and wave (row waves) */
+  uint32_t wd[4] = {0u, 0u, 0u, 0u};
+  int wpre[4];
+  auto take_words = [&](int x) {
+    uint32_t* words = p0.fut + ((int64_t)(x % GSBN_FUT) * a.H + h) * W;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int w = rt + i * RT;
+      wd[i] = w < W ? words[w] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int w = rt + i * RT;
+      if (wd[i]) words[w] = 0u;
+      const int c = __popc(wd[i]);
+      const int incl = (int)wave_incl_scan((uint32_t)c);
+      wpre[i] = incl - c;
+      if (lane == 63) sh_wsum[i][wave - RW0] = incl;
+    }
+  };
+  /* places the rows of those words, ascending, in list `to` */
+  auto place_rows = [&](int to) {
+    int base = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i * RT >= W) break;
+      int mine = base;
+      for (int w = 0; w < NRW; ++w) {
+        const int c = sh_wsum[i][w];
+        if (w < wave - RW0) mine += c;
+        base += c;
+      }
+      uint32_t bits = wd[i];
+      int pos = mine + wpre[i];
+      while (bits) {
+        const int k = ((rt + i * RT) << 5) + __ffs(bits) - 1;
+        bits &= bits - 1;
+        if (pos < BLK_LIST) sh_list[to][pos] = k;
+        else list_mem[to][pos] = k;
+        ++pos;
+      }
+    }
+  };
+  auto count_rows = [&]() {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i * RT >= W) break;
+      for (int w = 0; w < NRW; ++w) n += sh_wsum[i][w];
+    }
+    return n;
+  };
+
+  /* the update of synapse (row list[aa], j) at step t: row record to sh_row
+   * (aa < RCAP), the record stored, returns the contribution.  `kick`: the
+   * unit's spike of this step is known and applied. */
+  auto row_update = [&](int k, int j, int t, float pjv, bool kick, gsbn_row_rec* row_out) -> float {
+    const int64_t r = hC + k, sidx = r * M + j;
+    const int uj = h * M + j;
+    gsbn_row_rec st = b.rowst[r];
+    SynVals s = io.load(sidx, LOG || !learn);
+    const int T0 = sh_dcnt[j];
+    const int32_t* ring = b.dhist + (int64_t)uj * K;
+    bool w_log = false;
+    gsbn_syn_coef_t cown;
+    if constexpr (LOG) {
+      Kicks kicks(ring, T0, K, s.tij);
+      w_log = replay_log<PREC>(io, s, st, lg, g.nlog, b, uj, kicks);
+      kicks.run<PREC>(io, s, t - 1, table, table_len, b.kftj);
+      if (t - s.tij > 0) cown = load_coef(table, table_len, t - s.tij);
+    } else {
+      const int more = T0 - 8 >= 0 ? sh_k8[T0 & 7][j] : INT_MIN;
+      if (more > s.tij) {
+        replay_kicks<PREC>(io, s, ring, T0, K, t - 1, table, table_len, b.kftj);
+        if (t - s.tij > 0) cown = load_coef(table, table_len, t - s.tij);
+      } else {
+        Ring8 rg;
+#pragma unroll
+        for (int q = 0; q < 7; ++q) rg.s[q] = T0 - 7 + q >= 0 ? sh_k8[(T0 + 1 + q) & 7][j] : INT_MIN;
+        replay_ring8<PREC>(io, s, rg, t - 1, table, table_len, b.kftj, t, &cown);
+      }
+    }
+    const int Dr = t - st.ti;
+    if (Dr > 0) gsbn_row_catchup(gsbn_coef(table, table_len, Dr), &st.pi, &st.ei, &st.zi);
+    st.zi += b.kfti;
+    st.ti = t;
+    if (j == 0) *row_out = st;
+    float cval;
+    bool w_new = w_log;
+    if (t - s.tij <= 0) {
+      s.zi2 += b.kfti;
+      s.tij = t;
+      cval = gsbn_bitsf(GSBN_NO_CONTRIB_BITS);
+    } else {
+      gsbn_syn_catchup_k(cown, &s.pij, &s.eij, &s.zi2, &s.zj2);
+      s.zi2 = s.zi2 + b.kfti;
+      s.tij = t;
+      if (learn) {
+        s.wij = gsbn_wij(s.pij, st.pi, pjv, b.wgain, b.eps, b.eps2);
+        w_new = true;
+      }
+      cval = s.wij;
+    }
+    if (kick) s.zj2 += b.kftj;
+    io.store(sidx, s, w_new);
+    return cval;
+  };
+
+  /* --- state --- */
+  float dsup[UPL], lgv[UPL], e[UPL], act[UPL];
+  int counter[UPL], chk[UPL], spk[UPL];
+  float wmv = 0.0f;
+  float pj = 0.0f, ej = 0.0f, zj = 0.0f, bj = 0.0f, pj_n = 0.0f;
+  const int jj = (wave - 1) * 64 + lane; /* the trace waves' unit */
+  const bool jlive = wave >= 1 && wave < RW0 && jj < M;
+  if (wave == 0) {
+    wmv = a.wmask[g.wm_off + h];
+    const int pend = p0.pend_cnt[h];
+#pragma unroll
+    for (int u = 0; u < UPL; ++u) {
+      const int j = lane + 64 * u, idx = h * M + j;
+      dsup[u] = lgv[u] = e[u] = act[u] = 0.0f;
+      counter[u] = chk[u] = spk[u] = 0;
+      if (j < M) {
+        dsup[u] = a.dsup[idx];
+        lgv[u] = a.lginp[g.lg_off + idx];
+        counter[u] = a.counter[idx];
+        e[u] = a.epsc[idx];
+        const float* c = p0.contrib + hC * M + j;
+        for (int k = 0; k < pend; ++k) {
+          const float v = c[(int64_t)k * M];
+          if (gsbn_fbits(v) != GSBN_NO_CONTRIB_BITS) e[u] = e[u] + v;
+        }
+      }
+    }
+  } else if (wave < RW0) {
+    if (jlive) {
+      const int idx = h * M + jj;
+      pj = p0.pj[idx];
+      ej = p0.ej[idx];
+      zj = p0.zj[idx];
+      bj = a.bj[idx];
+      const int n = p0.dcnt[idx];
+      sh_dcnt[jj] = n;
+#pragma unroll
+      for (int q = 1; q <= 8; ++q)
+        if (n - q >= 0) sh_k8[(n - q) & 7][jj] = p0.dhist[(int64_t)idx * K + ((n - q) & (K - 1))];
+      float u01, z;
+      gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)g.simstep, (uint32_t)idx, &u01, &z);
+      sh_u[0][jj] = u01;
+      sh_xi[0][jj] = a.snoise * z;
+      pj_n = pj + (ej - pj) * kp;
+      sh_pj[0][jj] = pj_n;
+      sh_bj[1][jj] = bj;
+    }
+  } else {
+    take_words(g.exec);
+  }
+  __syncthreads();
+  if (wave >= RW0) place_rows(0);
+  int nrows = count_rows(), rows_sum = 0, spk_sum = 0;
+  __syncthreads();
+
+  for (int s = 0; s < g.nsteps; ++s) {
+    const int t = g.simstep + s, x = g.exec + s, par = s & 1;
+    const int nlds = nrows < RCAP ? nrows : RCAP;
+    const bool more_steps = s + 1 < g.nsteps;
+    if (wave == 0) {
+      /* support, dsup (Pop.cpp:229-261) */
+      float maxdsup = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < UPL; ++u) {
+        const int j = lane + 64 * u;
+        if (j < M) {
+          float wsup = 0.0f;
+          wsup += sh_bj[par ^ 1][j] + e[u];
+          float sup = a.lgbias + a.igain * lgv[u] + sh_xi[par][j];
+          sup += (a.wgain * wmv) * wsup;
+          dsup[u] = dsup[u] + (sup - dsup[u]) * a.taumdt;
+        }
+        const float o = wave_max_left(j < M ? dsup[u] : -INFINITY);
+        if (u == 0 || o > maxdsup) maxdsup = o;
+      }
+      /* soft-max (Pop.cpp:280-302); the maximum's exponential from a lane that
+       * holds the maximum, whose own is 1 (see recall_wave_kernel) */
+      const float xmax = a.wtagain * maxdsup;
+      float maxact = 0.0f;
+      bool have = false;
+#pragma unroll
+      for (int u = 0; u < UPL; ++u) {
+        const float diff = dsup[u] - maxdsup;
+        const bool top = lane + 64 * u < M && diff == 0.0f && a.wtagain * diff == 0.0f;
+        const float ex = gsbn_expf_guarded(top ? xmax : a.wtagain * diff);
+        act[u] = top ? 1.0f : ex;
+        const uint64_t tb = __ballot(top);
+        if (tb && !have) {
+          maxact = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ex), __builtin_ctzll(tb)));
+          have = true;
+        }
+      }
+      if (!have) maxact = gsbn_expf_guarded(xmax);
+#pragma unroll
+      for (int u = 0; u < UPL; ++u) {
+        if (maxact < 1.0f) act[u] *= maxact;
+        sh_act[lane + 64 * u] = act[u];
+      }
+      wave_order();
+      float vsum = 0.0f;
+      if (lane == 0) vsum = ordered_sum_lds(sh_act, M);
+      vsum = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(vsum)));
+      /* spikes and counters (Pop.cpp:305-323), epsc's decay */
+      int ns = 0;
+#pragma unroll
+      for (int u = 0; u < UPL; ++u) {
+        const int j = lane + 64 * u;
+        if (vsum > 1.0f) act[u] /= vsum;
+        spk[u] = (j < M && sh_u[par][j] < act[u] * a.maxfqdt) ? 1 : 0;
+        counter[u] += spk[u];
+        if ((g.count_mask >> s) & 1u) chk[u] += spk[u];
+        sh_sj[j] = spk[u];
+        const uint64_t bal = __ballot(spk[u]);
+        if (spk[u]) sh_spk[ns + __popcll(bal & ((1ull << lane) - 1ull))] = j;
+        ns += __popcll(bal);
+        e[u] = e[u] * (1 - p0.kepsc);
+      }
+      if (lane == 0) sh_nspk = ns;
+    } else if (wave < RW0) {
+      /* the next step's draws; this step's traces (Proj.cpp:310-363), whose
+       * spike increment follows, and with them the next step's pj */
+      if (jlive) {
+        const int idx = h * M + jj;
+        if (more_steps) {
+          float u01, z;
+          gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)(t + 1), (uint32_t)idx, &u01, &z);
+          sh_u[par ^ 1][jj] = u01;
+          sh_xi[par ^ 1][jj] = a.snoise * z;
+        }
+        pj = pj_n;
+        ej = ej + (zj - ej) * p0.ke;
+        zj = zj * (1 - p0.kzj);
+        if (learn) bj = p0.bgain * gsbn_logf_guarded(pj + p0.eps);
+        sh_bj[par][jj] = bj;
+        pj_n = pj + (ej - pj) * kp;
+        sh_pj[par ^ 1][jj] = pj_n;
+      }
+    } else {
+      /* this step's first rows */
+      for (int f = rt; f < nlds * M; f += RT) {
+        const int rr = f / M, j = f - rr * M;
+        sh_con[rr][j] = row_update(sh_list[par][rr], j, t, sh_pj[par][j], false, &sh_row[rr]);
+      }
+      if (more_steps) take_words(x + 1);
+    }
+    __syncthreads();
+    const int ns = sh_nspk;
+    rows_sum += nrows;
+    spk_sum += ns;
+    if (wave >= RW0) {
+      if (rt < nlds) b.rowst[hC + sh_list[par][rt]] = sh_row[rt];
+      /* the column increment of the spiking units on this step's rows */
+      for (int i = 0; i < ns; ++i) {
+        const int j = sh_spk[i];
+        for (int rr = rt; rr < nlds; rr += RT) io.add_zj2((hC + sh_list[par][rr]) * M + j, b.kftj);
+      }
+    }
+    /* rows past the LDS, in passes of RCAP */
+    for (int base = RCAP; base < nrows; base += RCAP) {
+      const int nr = nrows - base < RCAP ? nrows - base : RCAP;
+      __syncthreads(); /* sh_row, and sh_dcnt is not yet advanced */
+      if (wave >= RW0) {
+        for (int f = rt; f < nr * M; f += RT) {
+          const int rr = f / M, j = f - rr * M, aa = base + rr;
+          const int k = aa < BLK_LIST ? sh_list[par][aa] : list_mem[par][aa];
+          b.contrib[(hC + aa) * M + j] =
+              row_update(k, j, t, sh_pj[par][j], sh_sj[j] > 0, &sh_row[rr]);
+        }
+      }
+      __syncthreads();
+      if (wave >= RW0 && rt < nr) {
+        const int aa = base + rt;
+        b.rowst[hC + (aa < BLK_LIST ? sh_list[par][aa] : list_mem[par][aa])] = sh_row[rt];
+      }
+    }
+    if (nrows > RCAP) __syncthreads();
+    if (wave == 0) {
+      /* the spikes into the units' rings of pending column kicks */
+#pragma unroll
+      for (int u = 0; u < UPL; ++u) {
+        if (spk[u]) {
+          const int j = lane + 64 * u, idx = h * M + j, n = sh_dcnt[j];
+          sh_k8[n & 7][j] = t;
+          sh_dcnt[j] = n + 1;
+          p0.dhist[(int64_t)idx * K + (n & (K - 1))] = t;
+          p0.dcnt[idx] = n + 1;
+        }
+      }
+    } else if (wave < RW0) {
+      if (jlive && sh_sj[jj] > 0) zj += p0.kftj;
+      if (a.nproj_out > 0)
+        for (int i = 0; i < ns; ++i) push_unit(a.out0, h * M + sh_spk[i], x, tid - 64, 64 * UPL);
+    } else if (more_steps) {
+      place_rows(par ^ 1);
+    }
+    const int next = more_steps ? count_rows() : 0;
+    if (!more_steps) {
+      /* the last step's lists (.ssi, .ssj) */
+      for (int i = tid; i < nrows; i += T)
+        p0.rows_list[hC + i] = i < BLK_LIST ? sh_list[par][i] : list_mem[par][i];
+      for (int i = tid; i < ns; i += T) a.spk_list[h * M + i] = sh_spk[i];
+      if (tid == 0) {
+        a.spk_cnt[h] = ns;
+        p0.rows_cnt[h] = nrows;
+        p0.pend_cnt[h] = 0;
+        if (a.work) {
+          atomicAdd(reinterpret_cast<unsigned long long*>(&a.work[0]),
+                    (unsigned long long)rows_sum * (unsigned long long)M);
+          atomicAdd(reinterpret_cast<unsigned long long*>(&a.work[1]),
+                    (unsigned long long)spk_sum * (unsigned long long)C);
+        }
+      }
+    }
+    __syncthreads();
+    if (wave == 0) {
+      /* this step's support contributions, ascending row order */
+#pragma unroll
+      for (int u = 0; u < UPL; ++u) {
+        const int j = lane + 64 * u;
+        if (j < M) {
+          for (int rr = 0; rr < nlds; ++rr) {
+            const float v = sh_con[rr][j];
+            if (gsbn_fbits(v) != GSBN_NO_CONTRIB_BITS) e[u] = e[u] + v;
+          }
+          for (int aa = RCAP; aa < nrows; ++aa) {
+            const float v = p0.contrib[(hC + aa) * M + j];
+            if (gsbn_fbits(v) != GSBN_NO_CONTRIB_BITS) e[u] = e[u] + v;
+          }
+        }
+      }
+    }
+    nrows = next;
+  }
+
+  const int last = (g.nsteps - 1) & 1;
+  if (wave == 0) {
+#pragma unroll
+    for (int u = 0; u < UPL; ++u) {
+      const int j = lane + 64 * u, idx = h * M + j;
+      if (j >= M) continue;
+      a.dsup[idx] = dsup[u];
+      a.rnd_u[idx] = sh_u[last][j];
+      a.rnd_n[idx] = sh_xi[last][j];
+      a.act[idx] = act[u];
+      a.counter[idx] = counter[u];
+      a.spike[idx] = (int8_t)spk[u];
+      a.epsc[idx] = e[u];
+      if (g.count_mask) g.check[(a.lginp - g.lginp_base) + idx] += chk[u];
+    }
+  } else if (jlive) {
+    const int idx = h * M + jj;
+    p0.pj[idx] = pj;
+    p0.ej[idx] = ej;
+    p0.zj[idx] = zj;
+    if (learn) a.bj[idx] = bj;
+  }
+}
+
 template <int PREC>
 __global__ void __launch_bounds__(ALL_THREADS) all_kernel(gsbn_all_args a) {
   __shared__ float sh_pi[ALL_ROWS];
@@ -3192,6 +3645,55 @@ int gsbn_step_fused_batch(const gsbn_pop_args* pops_dev, int32_t npop,
                    wg_hcu, in_proj, *step);
       break;
   }
+  return launch_status();
+}
+
+int gsbn_step_block(const gsbn_block_args* k, const gsbn_step_args* step, void* stream) {
+  if (!k || !batch_step_ok(step) || !k->pops_dev || !k->projs_dev || !k->wg_pop || !k->wg_hcu ||
+      !k->rows2 || k->nwg <= 0 || k->nsteps <= 0 || k->nsteps > GSBN_BLOCK_MAX || k->max_m <= 0 ||
+      k->max_m > 128 || k->max_slots <= 0 || (k->nlog && !log_ok(k->logs, k->nlog)) ||
+      (k->count_mask && !k->check) || !k->lginp_base)
+    return GSBN_ERR_ARG;
+  const int upl = k->max_m <= 64 ? 1 : 2;
+  const int threads = k->threads;
+  if (threads != 256 && threads != 1024) return GSBN_ERR_ARG;
+  /* the ring words of a step in four words per row thread */
+  if ((k->max_slots + 31) / 32 > 4 * (threads - 64 * (1 + upl))) return GSBN_ERR_UNSUPPORTED;
+  BlockArgs g;
+  g.nlog = k->nlog;
+  g.simstep = step->simstep;
+  g.exec = step->exec;
+  g.nsteps = k->nsteps;
+  g.kp_slot = step->kp_slot;
+  g.prn = step->prn;
+  g.lg_off = step->lginp_offset;
+  g.wm_off = step->wmask_offset;
+  g.count_mask = k->count_mask;
+  g.check = k->check;
+  g.lginp_base = k->lginp_base;
+  const dim3 grid(k->nwg), t(threads);
+  hipStream_t s = (hipStream_t)stream;
+#define BLK2(P, L, U)                                                                \
+  if (threads == 1024) launch_timed(block_kernel<P, L, U, 1024, 32>, grid, t, 0, s, k->pops_dev, k->projs_dev, \
+                                    k->wg_pop, k->wg_hcu, k->rows2, k->logs, g);          \
+  else launch_timed(block_kernel<P, L, U, 256, 8>, grid, t, 0, s, k->pops_dev, k->projs_dev, \
+                    k->wg_pop, k->wg_hcu, k->rows2, k->logs, g)
+#define BLK(P)                          \
+  if (k->nlog) {                        \
+    if (upl == 1) BLK2(P, true, 1);     \
+    else BLK2(P, true, 2);              \
+  } else {                              \
+    if (upl == 1) BLK2(P, false, 1);    \
+    else BLK2(P, false, 2);             \
+  }                                     \
+  break
+  switch (step->prec) {
+    case GSBN_PREC_F32: BLK(GSBN_PREC_F32);
+    case GSBN_PREC_BF16: BLK(GSBN_PREC_BF16);
+    default: BLK(GSBN_PREC_F16);
+  }
+#undef BLK
+#undef BLK2
   return launch_status();
 }
 

@@ -259,6 +259,8 @@ class Proj : public ProjRowOps {
     f.W = W;
     return f;
   }
+  int delay_min = 31; /* smallest delay of its rows */
+  DevBuf<int32_t> rows_list1; /* block step: second list of a step's rows */
   uint64_t ii_version = ~0ull, di_version = ~0ull;
   int last_exec = -1;
   bool direct_que = false; /* the source population's kernel pushes this step's spikes */
@@ -878,12 +880,14 @@ void Proj::rebuild_fanout() {
   const int* ii = _ii->cpu_data();
   const int* di = _di->cpu_data();
   vector<int32_t> off((size_t)_nsrc + 1, 0);
+  delay_min = 31;
   for (int64_t r = 0; r < R; ++r) {
     const int n = ii[r];
     if (n < 0) continue;
     if (n >= _nsrc) throw Error(-2, "ii_" + std::to_string(_id) + ": source unit out of range");
     const int d = di[r];
     if (d < 1 || d > 31) throw Error(-2, "di_" + std::to_string(_id) + ": delay must be in [1, 31]");
+    delay_min = std::min(delay_min, d);
     off[(size_t)n + 1]++;
   }
   for (int n = 0; n < _nsrc; ++n) off[(size_t)n + 1] += off[(size_t)n];
@@ -1277,6 +1281,37 @@ class ProcUpdLazy : public ProcedureBase {
   DevBuf<int32_t> _gmap_proj[4], _gmap_hcu[4], _gmap_part[4];
   int _gmap_n[4] = {0, 0, 0, 0};
   void build_graded_map(int g);
+  /* Block step: in a solver call of more than one step, steps are held back
+   * and up to the smallest delay plus 2 of them run in one launch
+   * (gsbn_step_block), when the next step does not fit, when anything reads
+   * or writes a vector, and at the end of the call.  Calls of one step, which
+   * leave nothing to hold, run the plans above.  Applies to populations of at
+   * most 128 MCUs with one incoming and at most one outgoing projection whose
+   * spikes the population kernel pushes itself, deferred columns by default,
+   * no external spikes, no wta-pop-max, and no plan asked for.
+   * argi block-step 0: never; 1: every step, an error where it does not
+   * apply.  GlobalVar block-step: 1 where it applies.
+   * By default up to kBlockHcus hypercolumns: what the device holds at once
+   * (256 CUs, four workgroups of 256 each).  Per step, blocks of 3 against the
+   * best split: 10 HCUs x 10 units 4.5 us (10.3), 100 x 100 8.1 us (15), 24
+   * networks (860 HCUs) 12.8 us (18); 128 networks (4600 HCUs) 51 us (34-42). */
+  static constexpr int kBlockHcus = 1024;
+  int _block_arg = -1;
+  bool _block = false;
+  int _block_threads = 1024;
+  struct Held {
+    int n = 0, simstep = 0, exec = 0, slot = 0;
+    float prn = 0.0f;
+    int64_t lg_off = 0, wm_off = 0;
+    uint32_t count_mask = 0;
+    int32_t* check = nullptr;
+  } _held;
+  DevBuf<int32_t*> _rows2;
+  std::shared_ptr<SolverMemory> _held_mem; /* where run_held and count_spikes are set */
+  int block_max() const;
+  bool block_applies() const;
+  void run_held();
+  bool count_held(int32_t* counts);
   bool _chainable = false, _pending = false;
   int _chain_fixed = 0, _chain_parts = 1, _chain_warm = 0;
   gsbn_rowcol_args _pend_ra;
@@ -1347,6 +1382,10 @@ class ProcUpdLazy : public ProcedureBase {
 REGISTERIMPL(ProcUpdLazy);
 
 ProcUpdLazy::~ProcUpdLazy() {
+  if (_held_mem) {
+    _held_mem->run_held = nullptr;
+    _held_mem->count_spikes = nullptr;
+  }
   for (hipEvent_t e : _tev) (void)hipEventDestroy(e);
   for (auto* p : _list_proj) delete p;
   for (auto* p : _list_pop) delete p;
@@ -1355,6 +1394,7 @@ ProcUpdLazy::~ProcUpdLazy() {
 /* the row and column updates a chained step left pending, as a row/column
  * launch of that step */
 void ProcUpdLazy::flush_deferred() {
+  run_held();
   if (!_pending) return;
   _pending = false;
   Proj* q = _list_proj[0];
@@ -1443,12 +1483,107 @@ void ProcUpdLazy::record_sweep(int simstep, float old_prn, float prn, const gsbn
   Timing::get().end(3, s);
 }
 
+bool ProcUpdLazy::block_applies() const {
+  if (_fused_fixed || _chain_fixed > 0 || _graded_fixed || _wave_fixed || _parts_fixed ||
+      _wta_pop_max || !_defer_k || _defer_arg >= 0 || _list_proj.empty())
+    return false;
+  for (auto* q : _list_proj)
+    if (!q->direct_que) return false;
+  for (auto* p : _list_pop)
+    if (p->_dim_mcu > 128 || p->_in.size() != 1 || p->_out.size() > 1 || p->has_ext) return false;
+  return true;
+}
+
+/* steps a block may hold: a spike's rows are active delay + 2 steps later */
+int ProcUpdLazy::block_max() const {
+  int n = GSBN_BLOCK_MAX;
+  for (auto* q : _list_proj) n = std::min(n, q->delay_min + 2);
+  return n;
+}
+
+/* the steps held back, in one launch, and the walks that are due */
+void ProcUpdLazy::run_held() {
+  if (!_held.n) return;
+  const Held k = _held;
+  _held.n = 0;
+  _held.count_mask = 0;
+  hipStream_t s = active_stream();
+  gsbn_step_args st;
+  memset(&st, 0, sizeof(st));
+  st.simstep = k.simstep;
+  st.exec = k.exec;
+  st.do_jxx = 1;
+  st.kp_slot = k.slot;
+  st.prn = k.prn;
+  st.prec = _list_proj[0]->prec;
+  st.lginp_offset = k.lg_off;
+  st.wmask_offset = k.wm_off;
+  const int nl = (int)nlog();
+  for (auto* q : _list_proj)
+    if ((int)q->log.size() != nl) { /* one length for all logs: see record_sweep */
+      apply_logs(k.simstep - 1, k.prn);
+      break;
+    }
+  gsbn_block_args b;
+  memset(&b, 0, sizeof(b));
+  b.pops_dev = _pop_dev.p;
+  b.projs_dev = _proj_dev.p;
+  b.wg_pop = _wg_pop.p;
+  b.wg_hcu = _wg_pop_hcu.p;
+  b.rows2 = _rows2.p;
+  b.nlog = (int)nlog();
+  b.logs = b.nlog ? logs() : nullptr;
+  b.nwg = _nwg_pop;
+  b.nsteps = k.n;
+  b.threads = _block_threads;
+  b.max_m = _max_m;
+  b.max_slots = _max_slots;
+  b.count_mask = k.count_mask;
+  b.check = k.check;
+  b.lginp_base = _pop_args[0].lginp;
+  /* chained steps walk at full rings only */
+  auto walk = [&](int simstep, int exec) {
+    _walk_age = 0;
+    gsbn_step_args w = st;
+    w.simstep = simstep;
+    w.exec = exec;
+    op_check(gsbn_proj_walk_batch(_pop_dev.p, _wg_pop.p, _wg_pop_hcu.p, _nwg_pop, _proj_dev.p,
+                                  _wg_proj.p, _wg_proj_hcu.p, _nhcu_proj, _max_slots, kWalkDue,
+                                  b.logs, b.nlog, &w, s),
+             "gsbn_proj_walk_batch");
+  };
+  if (_walk_age >= kWalkEvery) walk(k.simstep - 1, k.exec - 1);
+  Timing::get().begin(6, s);
+  op_check(gsbn_step_block(&b, &st, s), "gsbn_step_block");
+  Timing::get().end(6, s);
+  _walk_age += k.n;
+  /* the next block may be GSBN_BLOCK_MAX steps long */
+  if (_walk_age + GSBN_BLOCK_MAX > kWalkEvery) walk(k.simstep + k.n - 1, k.exec + k.n - 1);
+}
+
+/* SolverMemory::count_spikes */
+bool ProcUpdLazy::count_held(int32_t* counts) {
+  if (!_held.n) return false;
+  const uint32_t bit = 1u << (_held.n - 1);
+  if ((_held.count_mask && _held.check != counts) || (_held.count_mask & bit)) {
+    run_held(); /* another counter, or one step counted twice */
+    return false;
+  }
+  _held.check = counts;
+  _held.count_mask |= bit;
+  return true;
+}
+
 /* column updates become eager again (a structural change of the rows is
  * coming, which the replay of pending kicks cannot follow): the pending
  * row/column work and every pending kick are applied first */
 void ProcUpdLazy::end_deferral() {
   if (!_defer_k) return;
   flush_deferred();
+  if (_block) { /* the tuned plans from here on */
+    _block = false;
+    _glv.puti("block-step", 0);
+  }
   for (auto* q : _list_proj) {
     q->materialize_kicks();
     q->dK = 0;
@@ -1566,6 +1701,7 @@ void ProcUpdLazy::init(SolverParam solver_param, Database& db, bool copy) {
     throw Error(-2, "ProcUpdLazy: ovf-keep and ovf-cap must be >= 0");
   if (_wave_fixed < 0 || _wave_fixed > 4)
     throw Error(-2, "ProcUpdLazy: rowcol-wave must be in [0, 4]");
+  par.argi("block-step", _block_arg);
   par.argi("deferred-sweeps", _sweep_defer);
   par.argi("deferred-columns", _defer_arg);
   if (_defer_arg != -1 &&
@@ -1690,7 +1826,7 @@ void ProcUpdLazy::build_batch_maps() {
                                                       p->_in[0]) - _list_proj.begin()));
   _in_proj.upload(in.data(), in.size());
   _in_proj_host = in;
-  if (_pop_upl && _ovf_keep > 0) {
+  if (_batch && _pop_upl && _ovf_keep > 0) {
     _ovf_cnt.alloc(kOvfCounters);
     _ovf_task.alloc((size_t)3 * std::max(_ovf_cap, 1));
     op_check(gsbn_i32_fill(_ovf_cnt.p, kOvfCounters, 0, active_stream()), "fill");
@@ -1726,14 +1862,14 @@ void ProcUpdLazy::refresh_args(int simstep) {
   for (auto* p : _list_pop) _pop_args.push_back(p->args(0, 0, 0.0f, 0, 0, true, _seed, _wta_pop_max));
   /* the incoming projection's index in the batch's row/column argument
    * array, which the overflow queue's tasks name */
-  if (_batch)
+  if (_batch || _block)
     for (size_t i = 0; i < _pop_args.size() && i < _in_proj_host.size(); ++i)
       _pop_args[i].proj0.bidx = _in_proj_host[i];
   _proj_args.clear();
   for (auto* q : _list_proj) _proj_args.push_back(q->static_args(_slot_prn, _nslots, (int64_t)simstep + 2));
   /* a host write (a new stimulus row, say) leaves these unchanged: the
    * upload, which waits for the queued steps, is skipped then */
-  if (_batch) {
+  if (_batch || _block) {
     const size_t pb = _pop_args.size() * sizeof(gsbn_pop_args);
     if (_pop_sent.size() != pb || memcmp(_pop_sent.data(), _pop_args.data(), pb)) {
       _pop_dev.upload(_pop_args.data(), _pop_args.size());
@@ -1755,6 +1891,7 @@ void ProcUpdLazy::update_gpu() {
   int cycle_flag = 0;
   GSBN_CHECK(_glv.geti("cycle-flag", cycle_flag), "cycle-flag");
   if (cycle_flag < 0) {
+    run_held();
     /* the schedule is over: no sweep stays behind */
     const gsbn_sweep_log* lg = nullptr;
     for (auto* q : _list_proj)
@@ -1785,7 +1922,7 @@ void ProcUpdLazy::update_gpu() {
       if (q->direct_que) q->_ptr_src_pop->push_direct = true;
     }
     _batch = _list_pop.size() > 1 || _list_proj.size() > 1;
-    if (_batch) build_batch_maps();
+    build_batch_maps();
     _nhcu_proj = 0;
     for (auto* q : _list_proj) _nhcu_proj += q->_dim_hcu;
     _max_m = 0;
@@ -1867,6 +2004,31 @@ void ProcUpdLazy::update_gpu() {
     }
     if (!_defer_k || _chain_fixed > 0) _sweep_defer = 0;
     _glv.puti("deferred-sweeps", _sweep_defer ? 1 : 0);
+    _block = _block_arg != 0 && block_applies() && (_block_arg > 0 || _nwg_pop <= kBlockHcus);
+    if (_block) {
+      /* one workgroup per HCU: large ones while every HCU has a CU of its own
+       * (a step's rows in parallel), small ones beyond (more HCUs in flight);
+       * a step's ring words are held four per row thread */
+      const int words = (_max_slots + 31) / 32, role = 64 * (1 + (_max_m <= 64 ? 1 : 2));
+      _block_threads = _nwg_pop <= 256 || words > 4 * (256 - role) ? 1024 : 256;
+      if (words > 4 * (_block_threads - role)) _block = false;
+    }
+    if (_block_arg > 0 && !_block)
+      throw Error(-2, "ProcUpdLazy: block-step needs populations of at most 128 MCUs with one "
+                      "incoming projection and at most one outgoing, the population kernel's queue "
+                      "push, default deferred columns, no wta-pop-max, external spikes or other plan");
+    if (_block) {
+      vector<int32_t*> r2;
+      for (auto* q : _list_proj) {
+        q->rows_list1.alloc((size_t)q->_dim_hcu * q->_dim_conn);
+        r2.push_back(q->rows_list1.p);
+        q->flush_hook = [this]() { flush_deferred(); };
+      }
+      _rows2.upload(r2.data(), r2.size());
+      _held_mem = active_memory()->shared_from_this();
+      _held_mem->run_held = [this]() { run_held(); };
+      _held_mem->count_spikes = [this](int32_t* c) { return count_held(c); };
+    }
     _glv.puti("deferred-columns", _defer_k);
     _glv.puti("deferred-ring", _defer_k ? _list_proj[0]->dK : 0);
     /* GlobalVar pop-wave: units per lane of the one-wave population launch
@@ -1877,6 +2039,7 @@ void ProcUpdLazy::update_gpu() {
     if (_wave_fixed > 0 && !_batch)
       throw Error(-2, "ProcUpdLazy: rowcol-wave needs a batch of populations or projections");
     _parts = _fused_fixed ? -1 : (_chain_fixed > 0 ? -2 : _parts0);
+    _glv.puti("block-step", _block ? 1 : 0);
     _glv.puti("rowcol-parts", _fused_fixed ? -1
                               : _chain_fixed > 0 ? -2
                               : _graded_fixed > 0 ? -10 - _graded_fixed
@@ -1887,6 +2050,27 @@ void ProcUpdLazy::update_gpu() {
                              _wave_fixed > 0 || _parts_fixed > 0 || _list_proj.empty()) ? 1 : 0);
     _configured = true;
     _args_dirty = true;
+  }
+  const bool sweep = old_prn != prn;
+  Pop* p0 = _list_pop.front();
+  const int64_t lg_off = p0->_lginp->ld() <= 0 ? (int64_t)lginp_idx : (int64_t)lginp_idx * p0->_lginp->ld();
+  const int64_t wm_off = p0->_wmask->ld() <= 0 ? (int64_t)wmask_idx : (int64_t)wmask_idx * p0->_wmask->ld();
+  if (_held.n) {
+    /* one more step of the block being held, if it goes on as before */
+    if (!sweep && _held.n < block_max() && simstep == _held.simstep + _held.n &&
+        !memcmp(&prn, &_held.prn, 4) && lg_off == _held.lg_off && wm_off == _held.wm_off &&
+        VecBase::host_epoch() == _epoch_seen && VecBase::host_write_epoch() == _write_epoch_seen &&
+        !_args_dirty && _tables.version == _tables_seen && simstep <= _tables.sim_end) {
+      ++_held.n;
+      for (auto* q : _list_proj) {
+        q->last_exec = _exec;
+        q->kick_t = simstep;
+      }
+      _exec++;
+      execs++;
+      return;
+    }
+    run_held();
   }
   const int slot = kp_slot(prn);
   for (auto* q : _list_proj) (void)q->table(q->_taupdt * prn, (int64_t)simstep + 2);
@@ -1906,15 +2090,39 @@ void ProcUpdLazy::update_gpu() {
   if (touched || _args_dirty || _tables.version != _tables_seen) refresh_args(simstep);
 
   /* current .lginp / .wmask rows (Pop.cpp:331-332) */
-  Pop* p0 = _list_pop.front();
-  const int64_t lg_off = p0->_lginp->ld() <= 0 ? (int64_t)lginp_idx : (int64_t)lginp_idx * p0->_lginp->ld();
-  const int64_t wm_off = p0->_wmask->ld() <= 0 ? (int64_t)wmask_idx : (int64_t)wmask_idx * p0->_wmask->ld();
   if (lginp_idx < 0 || lg_off + _total_units > (int64_t)p0->_lginp->size())
     throw Error(-2, "lginp-idx out of range");
   if (wmask_idx < 0 || wm_off + _total_hcus > (int64_t)p0->_wmask->size())
     throw Error(-2, "wmask-idx " + std::to_string(wmask_idx) + " out of range");
 
-  const bool sweep = old_prn != prn;
+  const bool blocks = _block && (_block_arg > 0 || active_memory()->call_steps > 1);
+  if (blocks) _run_len = 0; /* a tuning run restarts after the blocks */
+  if (blocks && !sweep) {
+    /* the first step of a block */
+    flush_deferred();
+    _held.n = 1;
+    _held.simstep = simstep;
+    _held.exec = _exec;
+    _held.slot = slot;
+    _held.prn = prn;
+    _held.lg_off = lg_off;
+    _held.wm_off = wm_off;
+    _held.count_mask = 0;
+    for (auto* p : _list_pop) p->spk_side = 0;
+    for (auto* q : _list_proj) {
+      q->last_exec = _exec;
+      q->kick_t = simstep;
+      q->kick_kp = q->_taupdt * prn;
+      q->kicks_pending = true;
+    }
+    if (touched)
+      for (auto* q : _list_proj) q->mark_views_device();
+    _epoch_seen = VecBase::host_epoch();
+    _tables_seen = _tables.version;
+    _exec++;
+    execs++;
+    return;
+  }
   gsbn_step_args st;
   memset(&st, 0, sizeof(st));
   st.simstep = simstep;
@@ -1929,7 +2137,7 @@ void ProcUpdLazy::update_gpu() {
   /* the step plan (row/column parts, or -1: the fused launch); sweep steps
    * run the sweep between the two launches and are not tuning samples */
   bool timed = false;
-  int plan = _list_proj.empty() ? 1 : rowcol_parts(stream, &timed);
+  int plan = _list_proj.empty() ? 1 : blocks ? _parts0 : rowcol_parts(stream, &timed);
   if (sweep) {
     if (timed) _run_len = 0; /* the run restarts after the sweep */
     timed = false;
@@ -2003,6 +2211,7 @@ void ProcUpdLazy::update_gpu() {
     Timing::get().end(6, stream);
     dp->flush_pending = true;
     dp->spk_side = side;
+    if (_block) _walk_age = kWalkEvery; /* a walk before the next block */
     ra.spk_list = pa.spk_list;
     ra.spk_cnt = pa.spk_cnt;
     if (q->dK) {
@@ -2121,7 +2330,8 @@ void ProcUpdLazy::update_gpu() {
   }
   /* (a chained step's row updates come with the next launch: its walks stay
    * inside the steps, as its column workgroups run them in parallel) */
-  if (_defer_k && _defer_arg < 0 && plan != -2 && ++_walk_age >= kWalkEvery) {
+  if (_defer_k && _defer_arg < 0 && plan != -2 &&
+      ++_walk_age + (_block ? GSBN_BLOCK_MAX - 1 : 0) >= kWalkEvery) {
     _walk_age = 0;
     const int n = (int)nlog();
     const gsbn_sweep_log* lg = n ? logs() : nullptr;

@@ -549,6 +549,7 @@ class ProcCheck : public ProcedureBase {
     int32_t* count; /* its part of _counts */
   };
   void report(bool final_line);
+  void make_items();
   GlobalVar _glv;
   vector<mode_t> _list_mode;
   SyncVector<int32_t>* _lgidx = nullptr;
@@ -634,6 +635,23 @@ void ProcCheck::init_new(SolverParam solver_param, Database& db) {
   _updated_flag = false;
 }
 
+/* the items of the launches over several populations */
+void ProcCheck::make_items() {
+  if (!_items.empty()) return;
+  int hoff = 0;
+  for (auto& p : _pops) {
+    gsbn_check_item c;
+    c.spike = p.spike->gpu_data();
+    c.count = p.count;
+    c.H = p.H;
+    c.M = p.M;
+    c.out_offset = hoff;
+    hoff += p.H;
+    _items.push_back(c);
+  }
+  _items_dev.upload(_items.data(), _items.size());
+}
+
 void ProcCheck::update_gpu() {
   int cycle_flag = 0;
   GSBN_CHECK(_glv.geti("cycle-flag", cycle_flag), "cycle-flag");
@@ -648,6 +666,11 @@ void ProcCheck::update_gpu() {
   const mode_t& m = _list_mode[_cursor];
   if (timestep <= m.begin_step) return;
   if (timestep < m.end_step) {
+    SolverMemory* mem = active_memory();
+    if (mem && mem->count_spikes && mem->count_spikes(_counts.p)) {
+      _updated_flag = true;
+      return;
+    }
     bool multi = _pops.size() > 1;
     for (auto& p : _pops)
       if (p.H > 1024) multi = false; /* gsbn_check_argmax_multi covers 1024 HCUs */
@@ -656,22 +679,7 @@ void ProcCheck::update_gpu() {
         op_check(gsbn_check_count(p.H * p.M, p.spike->gpu_data(), p.count, active_stream()),
                  "gsbn_check_count");
     } else {
-      if (_items.empty()) {
-        vector<gsbn_check_item> it;
-        int hoff = 0;
-        for (auto& p : _pops) {
-          gsbn_check_item c;
-          c.spike = p.spike->gpu_data();
-          c.count = p.count;
-          c.H = p.H;
-          c.M = p.M;
-          c.out_offset = hoff;
-          hoff += p.H;
-          it.push_back(c);
-        }
-        _items = it;
-        _items_dev.upload(it.data(), it.size());
-      }
+      make_items();
       op_check(gsbn_check_count_multi(_items_dev.p, (int32_t)_items.size(), active_stream()),
                "gsbn_check_count_multi");
     }
@@ -683,6 +691,11 @@ void ProcCheck::update_gpu() {
     return;
   }
   const int w = (int)_window_mode.size();
+  if (active_memory()) active_memory()->run_held_steps();
+  bool multi = _pops.size() > 1;
+  for (auto& p : _pops)
+    if (p.H > 1024) multi = false; /* gsbn_check_argmax_multi covers 1024 HCUs */
+  if (multi) make_items();
   if (_items_dev.p) {
     op_check(gsbn_check_argmax_multi(_items_dev.p, (int32_t)_items.size(),
                                      _res_idx.p + (int64_t)w * _total_hcu,

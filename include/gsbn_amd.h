@@ -464,6 +464,34 @@ int gsbn_step_fused_batch(const gsbn_pop_args* pops_dev, int32_t npop,
                           int32_t max_m, int32_t max_slots, int32_t any_wta_pop_max,
                           const gsbn_step_args* step, void* stream);
 
+/* Block step: `nsteps` consecutive executed steps (simsteps step->simstep ..,
+ * one stimulus and mask row, one learning rate, none of them a sweep step) of
+ * every population in one launch, one workgroup per HCU: the population
+ * updates (gsbn_pop_update) and row updates (gsbn_proj_rowcol) of those steps,
+ * with deferred column updates whose walks run between launches
+ * (gsbn_proj_walk).  Every population has M <= 128, one incoming projection
+ * with a ring of at least 8 kicks, at most one outgoing, no external spikes
+ * and no wta_pop_max; nsteps is at most the smallest delay of any projection
+ * plus 2, and no ring reaches its capacity during them (the caller checks).
+ * Leaves the state of the last step; epsc is final (pend_cnt 0).  No
+ * counterpart in the reference, whose steps are separate passes. */
+#define GSBN_BLOCK_MAX 8
+typedef struct {
+  const gsbn_pop_args* pops_dev;    /* proj0.bidx names the projection in projs_dev */
+  const gsbn_rowcol_args* projs_dev;
+  const int32_t* wg_pop;
+  const int32_t* wg_hcu;
+  int32_t* const* rows2;            /* per projection, [H * C] (device) */
+  const gsbn_sweep_log* logs;       /* per projection, when nlog > 0 */
+  int32_t nlog, nwg, nsteps, threads; /* threads: 256, or 1024 for few HCUs */
+  int32_t max_m, max_slots;
+  uint32_t count_mask; /* bit s: the spikes of step s are added to check */
+  int32_t pad;
+  int32_t* check;            /* [all units] */
+  const float* lginp_base;   /* lginp of the first population */
+} gsbn_block_args;
+int gsbn_step_block(const gsbn_block_args* k, const gsbn_step_args* step, void* stream);
+
 /* Delay-queue push (Proj.cpp:645-664) from si: si holds the spikes of exec
  * step exec - 1 (ProcExchangeSpike's copy), each source unit with si > 0
  * pushes its rows.  Grid: one workgroup per source HCU. */

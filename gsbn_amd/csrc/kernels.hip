@@ -2103,25 +2103,28 @@ __global__ void __launch_bounds__(RC_THREADS) chained_kernel(gsbn_pop_args a, gs
  * runs them all, its units' state and traces in registers, support
  * contributions and newest kicks in LDS.
  *
- * What bounds it: a chain of dependent latencies per step, so the work is
- * spread over waves by role and meets at two barriers per step:
+ * What bounds it: chains of dependent latencies, first touches above all (a
+ * launch starts with cold caches).  What depends on no earlier step is done
+ * before the first, a task per wave: the row lists of all steps from the ring
+ * and all draws.  Then per step two barriers and waves by role:
  *   wave 0       support, WTA, soft-max, spikes (UPL units per lane, wave
  *                scans and reductions, no barriers of its own);
- *   UPL waves    the next step's draws and the traces (pj, bj, which the next
- *                step needs, do not depend on this step's spikes); after the
- *                spikes, the queue push;
- *   the others   this step's active rows (they need the step's spikes only
- *                for zj2's increment, added after the first barrier), and the
- *                next step's ring words.
- * Rows past RCAP (a busier step than the LDS holds) are run after the first
- * barrier by the row waves in passes, their contributions through memory.
- * Outputs that only the last step leaves (act, draws, spike lists, active
- * rows) are stored once.
- * Measured, launches of 3 steps (delay 1): 10 HCUs x 10 units 13.6 us, where
- * the split plan's six launches took 31 us; 100 x 100 24.3 us (45); 24 networks
- * of 16 to 128 units, 860 HCUs, 38 us (54). */
-#define BLK_LIST 512 /* active rows of a step held in LDS; the rest through rows2 / rows_list */
-
+ *   UPL waves    the traces (pj, bj, which the next step needs, do not depend
+ *                on this step's spikes);
+ *   one wave     the queue push of the step before;
+ *   all waves    when done with these, this step's active rows, 64 synapses at
+ *                a time from a shared counter (they need the step's spikes only
+ *                for zj2's increment, added after the first barrier).
+ * Contributions of rows past RCAP (a busier step than the LDS holds) go
+ * through memory.  Outputs that only the last step leaves (act, draws, spike
+ * lists, active rows) are stored once.
+ * Measured, launches of 3 steps (delay 1): 10 HCUs x 10 units 10.2 us, 100 x 100
+ * 18.9 us (13.6 and 24.3 with draws and lists made inside the steps and rows
+ * bound to the waves without another role), where the split plan's six
+ * launches took 31 and 45 us; 24 networks of 16 to 128 units, 860 HCUs, 20 us
+ * (38; 54).  Of the 18.9 us the prologue takes 2.5, support to spikes 1.5 per
+ * step (exponentials 0.5, the ordered sum 0.5).  Touching the next steps' rows
+ * ahead from idle waves cost more at the barrier than it gave (+3 %). */
 struct BlockArgs {
   int nlog, simstep, exec, nsteps, kp_slot;
   float prn;
@@ -2131,32 +2134,33 @@ struct BlockArgs {
   const float* lginp_base;  /* the first population's lginp (units before a population) */
 };
 
-template <int PREC, bool LOG, int UPL, int T, int RCAP>
-__global__ void __launch_bounds__(T)
+/* T threads; RCAP: rows of a step whose contributions are held on chip; BL:
+ * entries of a step's row list held on chip (the rest through lists) */
+template <int PREC, bool LOG, int UPL, int T, int RCAP, int BL>
+__global__ void __launch_bounds__(T, T >= 512 ? 0 : 4)
     block_kernel(const gsbn_pop_args* __restrict__ pops, const gsbn_rowcol_args* __restrict__ projs,
-                 const int32_t* __restrict__ wg_pop, const int32_t* __restrict__ wg_hcu,
-                 int32_t* const* __restrict__ rows2, const gsbn_sweep_log* __restrict__ logs,
-                 const BlockArgs g) {
-  constexpr int MX = 64 * UPL, NW = T / 64, RW0 = 1 + UPL, RT = T - 64 * RW0, NRW = NW - RW0;
-  static_assert(NRW > 0 && RT >= RCAP, "row waves");
-  __shared__ float sh_u[2][MX], sh_xi[2][MX], sh_pj[2][MX], sh_bj[2][MX];
+                 const gsbn_block_wg* __restrict__ wgs, int32_t* const* __restrict__ lists,
+                 const gsbn_sweep_log* __restrict__ logs, const BlockArgs g) {
+  constexpr int MX = 64 * UPL, NW = T / 64, RW0 = 1 + UPL, NS = GSBN_BLOCK_MAX;
+  constexpr int PW = T >= 512 ? NW - 1 : 1; /* the wave that pushes */
+  static_assert(NW > RW0 && T >= RCAP, "waves");
+  __shared__ float sh_u[NS][MX], sh_xi[NS][MX], sh_pj[2][MX], sh_bj[2][MX];
   __shared__ __attribute__((aligned(16))) float sh_act[MX];
   __shared__ float sh_con[RCAP][MX];
   __shared__ gsbn_row_rec sh_row[RCAP];
-  __shared__ int sh_sj[MX], sh_dcnt[MX], sh_k8[8][MX], sh_spk[MX];
-  __shared__ int sh_list[2][BLK_LIST];
-  __shared__ int sh_wsum[4][NRW];
-  __shared__ int sh_nspk;
+  __shared__ int sh_sj[MX], sh_dcnt[MX], sh_k8[8][MX], sh_spk[2][MX];
+  __shared__ int sh_list[NS][BL], sh_nrows[NS];
+  __shared__ int sh_nspk[2], sh_next[2];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rt = tid - 64 * RW0; /* row thread */
-  const gsbn_pop_args& a = pops[wg_pop[blockIdx.x]];
+  const gsbn_block_wg wg = wgs[blockIdx.x];
+  const gsbn_pop_args& a = pops[wg.pop];
   const gsbn_pop_proj& p0 = a.proj0;
-  const gsbn_rowcol_args& b = projs[p0.bidx];
+  const gsbn_rowcol_args& b = projs[wg.proj];
   touch_lines<sizeof(gsbn_pop_args)>(&a);
   touch_lines<sizeof(gsbn_rowcol_args)>(&b);
-  const int h = wg_hcu[blockIdx.x];
+  const int h = wg.hcu;
   const int M = a.M, C = p0.C, W = p0.W, K = p0.dK;
   const int64_t hC = (int64_t)h * C;
   const SynIO<PREC> io(b);
@@ -2164,67 +2168,53 @@ __global__ void __launch_bounds__(T)
   const int table_len = b.table_lens[g.kp_slot];
   const float kp = p0.taupdt * g.prn;
   const bool learn = kp != 0.0f;
-  int32_t* const list_mem[2] = {p0.rows_list + hC, rows2[p0.bidx] + hC};
-  const gsbn_sweep_log* lg = LOG ? logs + p0.bidx : nullptr; /* rows2: the second list of rows past BLK_LIST */
+  const gsbn_sweep_log* lg = LOG ? logs + wg.proj : nullptr;
+  /* rows of step s past the LDS list */
+  auto list_mem = [&](int s) { return lists[wg.proj] + (int64_t)s * a.H * C + hC; };
+  auto row_at = [&](int s, int i) { return i < BL ? sh_list[s][i] : list_mem(s)[i]; };
 
-  /* the ring words of exec step x into registers, cleared, with their counts
-   * per band and wave (row waves) */
-  uint32_t wd[4] = {0u, 0u, 0u, 0u};
-  int wpre[4];
-  auto take_words = [&](int x) {
-    uint32_t* words = p0.fut + ((int64_t)(x % GSBN_FUT) * a.H + h) * W;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int w = rt + i * RT;
-      wd[i] = w < W ? words[w] : 0u;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int w = rt + i * RT;
-      if (wd[i]) words[w] = 0u;
-      const int c = __popc(wd[i]);
-      const int incl = (int)wave_incl_scan((uint32_t)c);
-      wpre[i] = incl - c;
-      if (lane == 63) sh_wsum[i][wave - RW0] = incl;
-    }
-  };
-  /* places the rows of those words, ascending, in list `to` */
-  auto place_rows = [&](int to) {
+  /* the active rows of step s, ascending, from its ring words (cleared): one
+   * wave, eight loads in flight */
+  auto make_list = [&](int s) {
+    uint32_t* words = p0.fut + ((int64_t)((g.exec + s) % GSBN_FUT) * a.H + h) * W;
     int base = 0;
+    for (int w0 = lane; w0 - lane < W; w0 += 8 * 64) {
+      uint32_t wd[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i * RT >= W) break;
-      int mine = base;
-      for (int w = 0; w < NRW; ++w) {
-        const int c = sh_wsum[i][w];
-        if (w < wave - RW0) mine += c;
-        base += c;
-      }
-      uint32_t bits = wd[i];
-      int pos = mine + wpre[i];
-      while (bits) {
-        const int k = ((rt + i * RT) << 5) + __ffs(bits) - 1;
-        bits &= bits - 1;
-        if (pos < BLK_LIST) sh_list[to][pos] = k;
-        else list_mem[to][pos] = k;
-        ++pos;
+      for (int i = 0; i < 8; ++i) wd[i] = w0 + 64 * i < W ? words[w0 + 64 * i] : 0u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        uint32_t bits = wd[i];
+        if (!__ballot(bits != 0u)) continue;
+        if (bits) words[w0 + 64 * i] = 0u;
+        const int c = __popc(bits);
+        const int incl = (int)wave_incl_scan((uint32_t)c);
+        int pos = base + incl - c;
+        base += __builtin_amdgcn_readlane(incl, 63);
+        while (bits) {
+          const int k = ((w0 + 64 * i) << 5) + __ffs(bits) - 1;
+          bits &= bits - 1;
+          if (pos < BL) sh_list[s][pos] = k;
+          else list_mem(s)[pos] = k;
+          ++pos;
+        }
       }
     }
+    if (lane == 0) sh_nrows[s] = base;
   };
-  auto count_rows = [&]() {
-    int n = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i * RT >= W) break;
-      for (int w = 0; w < NRW; ++w) n += sh_wsum[i][w];
-    }
-    return n;
+  auto make_draws = [&](int s, int u) {
+    const int j = 64 * u + lane;
+    if (j >= M) return;
+    float u01, z;
+    gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)(g.simstep + s),
+                           (uint32_t)(h * M + j), &u01, &z);
+    sh_u[s][j] = u01;
+    sh_xi[s][j] = a.snoise * z;
   };
 
-  /* the update of synapse (row list[aa], j) at step t: row record to sh_row
-   * (aa < RCAP), the record stored, returns the contribution.  `kick`: the
-   * unit's spike of this step is known and applied. */
-  auto row_update = [&](int k, int j, int t, float pjv, bool kick, gsbn_row_rec* row_out) -> float {
+  /* the update of synapse (row k, unit j) at step t: the record stored,
+   * returns the contribution; the row's record of this step in *row */
+  auto row_update = [&](int k, int j, int t, float pjv, gsbn_row_rec* row) -> float {
     const int64_t r = hC + k, sidx = r * M + j;
     const int uj = h * M + j;
     gsbn_row_rec st = b.rowst[r];
@@ -2254,7 +2244,7 @@ __global__ void __launch_bounds__(T)
     if (Dr > 0) gsbn_row_catchup(gsbn_coef(table, table_len, Dr), &st.pi, &st.ei, &st.zi);
     st.zi += b.kfti;
     st.ti = t;
-    if (j == 0) *row_out = st;
+    *row = st;
     float cval;
     bool w_new = w_log;
     if (t - s.tij <= 0) {
@@ -2271,12 +2261,11 @@ __global__ void __launch_bounds__(T)
       }
       cval = s.wij;
     }
-    if (kick) s.zj2 += b.kftj;
     io.store(sidx, s, w_new);
     return cval;
   };
 
-  /* --- state --- */
+  /* --- state, row lists and draws --- */
   float dsup[UPL], lgv[UPL], e[UPL], act[UPL];
   int counter[UPL], chk[UPL], spk[UPL];
   float wmv = 0.0f;
@@ -2296,6 +2285,12 @@ __global__ void __launch_bounds__(T)
         lgv[u] = a.lginp[g.lg_off + idx];
         counter[u] = a.counter[idx];
         e[u] = a.epsc[idx];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < UPL; ++u) {
+      const int j = lane + 64 * u;
+      if (j < M) {
         const float* c = p0.contrib + hC * M + j;
         for (int k = 0; k < pend; ++k) {
           const float v = c[(int64_t)k * M];
@@ -2303,38 +2298,33 @@ __global__ void __launch_bounds__(T)
         }
       }
     }
-  } else if (wave < RW0) {
-    if (jlive) {
-      const int idx = h * M + jj;
-      pj = p0.pj[idx];
-      ej = p0.ej[idx];
-      zj = p0.zj[idx];
-      bj = a.bj[idx];
-      const int n = p0.dcnt[idx];
-      sh_dcnt[jj] = n;
+    if (lane == 0) sh_next[0] = sh_next[1] = 0;
+  } else if (jlive) {
+    const int idx = h * M + jj;
+    pj = p0.pj[idx];
+    ej = p0.ej[idx];
+    zj = p0.zj[idx];
+    bj = a.bj[idx];
+    const int n = p0.dcnt[idx];
+    sh_dcnt[jj] = n;
 #pragma unroll
-      for (int q = 1; q <= 8; ++q)
-        if (n - q >= 0) sh_k8[(n - q) & 7][jj] = p0.dhist[(int64_t)idx * K + ((n - q) & (K - 1))];
-      float u01, z;
-      gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)g.simstep, (uint32_t)idx, &u01, &z);
-      sh_u[0][jj] = u01;
-      sh_xi[0][jj] = a.snoise * z;
-      pj_n = pj + (ej - pj) * kp;
-      sh_pj[0][jj] = pj_n;
-      sh_bj[1][jj] = bj;
-    }
-  } else {
-    take_words(g.exec);
+    for (int q = 1; q <= 8; ++q)
+      if (n - q >= 0) sh_k8[(n - q) & 7][jj] = p0.dhist[(int64_t)idx * K + ((n - q) & (K - 1))];
+    pj_n = pj + (ej - pj) * kp;
+    sh_pj[0][jj] = pj_n;
+    sh_bj[1][jj] = bj;
+  }
+  /* the waves without state to load first */
+  for (int task = NW - 1 - wave; task < g.nsteps * (1 + UPL); task += NW) {
+    if (task < g.nsteps) make_list(task);
+    else make_draws((task - g.nsteps) / UPL, (task - g.nsteps) % UPL);
   }
   __syncthreads();
-  if (wave >= RW0) place_rows(0);
-  int nrows = count_rows(), rows_sum = 0, spk_sum = 0;
-  __syncthreads();
 
+  int rows_sum = 0, spk_sum = 0;
   for (int s = 0; s < g.nsteps; ++s) {
-    const int t = g.simstep + s, x = g.exec + s, par = s & 1;
-    const int nlds = nrows < RCAP ? nrows : RCAP;
-    const bool more_steps = s + 1 < g.nsteps;
+    const int t = g.simstep + s, par = s & 1;
+    const int nrows = sh_nrows[s], nlds = nrows < RCAP ? nrows : RCAP;
     if (wave == 0) {
       /* support, dsup (Pop.cpp:229-261) */
       float maxdsup = -INFINITY;
@@ -2344,7 +2334,7 @@ __global__ void __launch_bounds__(T)
         if (j < M) {
           float wsup = 0.0f;
           wsup += sh_bj[par ^ 1][j] + e[u];
-          float sup = a.lgbias + a.igain * lgv[u] + sh_xi[par][j];
+          float sup = a.lgbias + a.igain * lgv[u] + sh_xi[s][j];
           sup += (a.wgain * wmv) * wsup;
           dsup[u] = dsup[u] + (sup - dsup[u]) * a.taumdt;
         }
@@ -2384,74 +2374,55 @@ __global__ void __launch_bounds__(T)
       for (int u = 0; u < UPL; ++u) {
         const int j = lane + 64 * u;
         if (vsum > 1.0f) act[u] /= vsum;
-        spk[u] = (j < M && sh_u[par][j] < act[u] * a.maxfqdt) ? 1 : 0;
+        spk[u] = (j < M && sh_u[s][j] < act[u] * a.maxfqdt) ? 1 : 0;
         counter[u] += spk[u];
         if ((g.count_mask >> s) & 1u) chk[u] += spk[u];
         sh_sj[j] = spk[u];
         const uint64_t bal = __ballot(spk[u]);
-        if (spk[u]) sh_spk[ns + __popcll(bal & ((1ull << lane) - 1ull))] = j;
+        if (spk[u]) sh_spk[par][ns + __popcll(bal & ((1ull << lane) - 1ull))] = j;
         ns += __popcll(bal);
         e[u] = e[u] * (1 - p0.kepsc);
       }
-      if (lane == 0) sh_nspk = ns;
-    } else if (wave < RW0) {
-      /* the next step's draws; this step's traces (Proj.cpp:310-363), whose
-       * spike increment follows, and with them the next step's pj */
-      if (jlive) {
-        const int idx = h * M + jj;
-        if (more_steps) {
-          float u01, z;
-          gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)(t + 1), (uint32_t)idx, &u01, &z);
-          sh_u[par ^ 1][jj] = u01;
-          sh_xi[par ^ 1][jj] = a.snoise * z;
+      if (lane == 0) sh_nspk[par] = ns;
+    } else if (jlive) {
+      /* the traces (Proj.cpp:310-363), whose spike increment follows, and with
+       * them the next step's pj */
+      pj = pj_n;
+      ej = ej + (zj - ej) * p0.ke;
+      zj = zj * (1 - p0.kzj);
+      if (learn) bj = p0.bgain * gsbn_logf_guarded(pj + p0.eps);
+      sh_bj[par][jj] = bj;
+      pj_n = pj + (ej - pj) * kp;
+      sh_pj[par ^ 1][jj] = pj_n;
+    }
+    if (wave == PW && s > 0 && a.nproj_out > 0) {
+      const int np = sh_nspk[par ^ 1];
+      for (int i = 0; i < np; ++i)
+        push_unit(a.out0, h * M + sh_spk[par ^ 1][i], g.exec + s - 1, lane, 64);
+    }
+    /* this step's rows */
+    for (const int nf = nrows * M;;) {
+      int f = 0;
+      if (lane == 0) f = atomicAdd(&sh_next[par], 64);
+      f = __builtin_amdgcn_readfirstlane(f);
+      if (f >= nf) break;
+      f += lane;
+      if (f < nf) {
+        const int rr = (int)((unsigned)f / (unsigned)M), j = f - rr * M;
+        gsbn_row_rec st;
+        const float cv = row_update(row_at(s, rr), j, t, sh_pj[par][j], &st);
+        if (rr < RCAP) {
+          sh_con[rr][j] = cv;
+          if (j == 0) sh_row[rr] = st;
+        } else {
+          b.contrib[(hC + rr) * M + j] = cv;
         }
-        pj = pj_n;
-        ej = ej + (zj - ej) * p0.ke;
-        zj = zj * (1 - p0.kzj);
-        if (learn) bj = p0.bgain * gsbn_logf_guarded(pj + p0.eps);
-        sh_bj[par][jj] = bj;
-        pj_n = pj + (ej - pj) * kp;
-        sh_pj[par ^ 1][jj] = pj_n;
       }
-    } else {
-      /* this step's first rows */
-      for (int f = rt; f < nlds * M; f += RT) {
-        const int rr = f / M, j = f - rr * M;
-        sh_con[rr][j] = row_update(sh_list[par][rr], j, t, sh_pj[par][j], false, &sh_row[rr]);
-      }
-      if (more_steps) take_words(x + 1);
     }
     __syncthreads();
-    const int ns = sh_nspk;
+    const int ns = sh_nspk[par];
     rows_sum += nrows;
     spk_sum += ns;
-    if (wave >= RW0) {
-      if (rt < nlds) b.rowst[hC + sh_list[par][rt]] = sh_row[rt];
-      /* the column increment of the spiking units on this step's rows */
-      for (int i = 0; i < ns; ++i) {
-        const int j = sh_spk[i];
-        for (int rr = rt; rr < nlds; rr += RT) io.add_zj2((hC + sh_list[par][rr]) * M + j, b.kftj);
-      }
-    }
-    /* rows past the LDS, in passes of RCAP */
-    for (int base = RCAP; base < nrows; base += RCAP) {
-      const int nr = nrows - base < RCAP ? nrows - base : RCAP;
-      __syncthreads(); /* sh_row, and sh_dcnt is not yet advanced */
-      if (wave >= RW0) {
-        for (int f = rt; f < nr * M; f += RT) {
-          const int rr = f / M, j = f - rr * M, aa = base + rr;
-          const int k = aa < BLK_LIST ? sh_list[par][aa] : list_mem[par][aa];
-          b.contrib[(hC + aa) * M + j] =
-              row_update(k, j, t, sh_pj[par][j], sh_sj[j] > 0, &sh_row[rr]);
-        }
-      }
-      __syncthreads();
-      if (wave >= RW0 && rt < nr) {
-        const int aa = base + rt;
-        b.rowst[hC + (aa < BLK_LIST ? sh_list[par][aa] : list_mem[par][aa])] = sh_row[rt];
-      }
-    }
-    if (nrows > RCAP) __syncthreads();
     if (wave == 0) {
       /* the spikes into the units' rings of pending column kicks */
 #pragma unroll
@@ -2464,19 +2435,45 @@ __global__ void __launch_bounds__(T)
           p0.dcnt[idx] = n + 1;
         }
       }
+      if (lane == 0) sh_next[par] = 0;
     } else if (wave < RW0) {
       if (jlive && sh_sj[jj] > 0) zj += p0.kftj;
-      if (a.nproj_out > 0)
-        for (int i = 0; i < ns; ++i) push_unit(a.out0, h * M + sh_spk[i], x, tid - 64, 64 * UPL);
-    } else if (more_steps) {
-      place_rows(par ^ 1);
+    } else {
+      const int rt = tid - 64 * RW0;
+      constexpr int RT = T - 64 * RW0;
+      for (int i = rt; i < nrows; i += RT) {
+        const int64_t r = hC + row_at(s, i);
+        gsbn_row_rec st;
+        if (i < RCAP) {
+          st = sh_row[i];
+        } else {
+          st = b.rowst[r];
+          if constexpr (LOG)
+            for (int q = 0; q < g.nlog; ++q) {
+              const gsbn_sweep_entry en = lg->e[q];
+              if (en.target > st.ti) {
+                gsbn_row_catchup(gsbn_coef(en.table, en.table_len, en.target - st.ti), &st.pi, &st.ei,
+                                 &st.zi);
+                st.ti = en.target;
+              }
+            }
+          const int Dr = t - st.ti;
+          if (Dr > 0) gsbn_row_catchup(gsbn_coef(table, table_len, Dr), &st.pi, &st.ei, &st.zi);
+          st.zi += b.kfti;
+          st.ti = t;
+        }
+        b.rowst[r] = st;
+        /* the column increment of the spiking units on this step's rows */
+        for (int q = 0; q < ns; ++q) io.add_zj2(r * M + sh_spk[par][q], b.kftj);
+      }
     }
-    const int next = more_steps ? count_rows() : 0;
-    if (!more_steps) {
-      /* the last step's lists (.ssi, .ssj) */
-      for (int i = tid; i < nrows; i += T)
-        p0.rows_list[hC + i] = i < BLK_LIST ? sh_list[par][i] : list_mem[par][i];
-      for (int i = tid; i < ns; i += T) a.spk_list[h * M + i] = sh_spk[i];
+    if (s + 1 == g.nsteps) {
+      /* the last step's lists (.ssi, .ssj) and its push */
+      for (int i = tid; i < nrows; i += T) p0.rows_list[hC + i] = row_at(s, i);
+      for (int i = tid; i < ns; i += T) a.spk_list[h * M + i] = sh_spk[par][i];
+      if (wave == PW && a.nproj_out > 0)
+        for (int i = 0; i < ns; ++i)
+          push_unit(a.out0, h * M + sh_spk[par][i], g.exec + s, lane, 64);
       if (tid == 0) {
         a.spk_cnt[h] = ns;
         p0.rows_cnt[h] = nrows;
@@ -2489,7 +2486,6 @@ __global__ void __launch_bounds__(T)
         }
       }
     }
-    __syncthreads();
     if (wave == 0) {
       /* this step's support contributions, ascending row order */
 #pragma unroll
@@ -2507,18 +2503,17 @@ __global__ void __launch_bounds__(T)
         }
       }
     }
-    nrows = next;
+    __syncthreads();
   }
 
-  const int last = (g.nsteps - 1) & 1;
   if (wave == 0) {
 #pragma unroll
     for (int u = 0; u < UPL; ++u) {
       const int j = lane + 64 * u, idx = h * M + j;
       if (j >= M) continue;
       a.dsup[idx] = dsup[u];
-      a.rnd_u[idx] = sh_u[last][j];
-      a.rnd_n[idx] = sh_xi[last][j];
+      a.rnd_u[idx] = sh_u[g.nsteps - 1][j];
+      a.rnd_n[idx] = sh_xi[g.nsteps - 1][j];
       a.act[idx] = act[u];
       a.counter[idx] = counter[u];
       a.spike[idx] = (int8_t)spk[u];
@@ -3649,16 +3644,11 @@ int gsbn_step_fused_batch(const gsbn_pop_args* pops_dev, int32_t npop,
 }
 
 int gsbn_step_block(const gsbn_block_args* k, const gsbn_step_args* step, void* stream) {
-  if (!k || !batch_step_ok(step) || !k->pops_dev || !k->projs_dev || !k->wg_pop || !k->wg_hcu ||
-      !k->rows2 || k->nwg <= 0 || k->nsteps <= 0 || k->nsteps > GSBN_BLOCK_MAX || k->max_m <= 0 ||
-      k->max_m > 128 || k->max_slots <= 0 || (k->nlog && !log_ok(k->logs, k->nlog)) ||
-      (k->count_mask && !k->check) || !k->lginp_base)
+  if (!k || !batch_step_ok(step) || !k->pops_dev || !k->projs_dev || !k->wgs || !k->lists ||
+      k->nwg <= 0 || k->nsteps <= 0 || k->nsteps > GSBN_BLOCK_MAX || k->max_m <= 0 ||
+      k->max_m > 128 || (k->nlog && !log_ok(k->logs, k->nlog)) || (k->count_mask && !k->check) ||
+      !k->lginp_base || (k->threads != 256 && k->threads != 1024))
     return GSBN_ERR_ARG;
-  const int upl = k->max_m <= 64 ? 1 : 2;
-  const int threads = k->threads;
-  if (threads != 256 && threads != 1024) return GSBN_ERR_ARG;
-  /* the ring words of a step in four words per row thread */
-  if ((k->max_slots + 31) / 32 > 4 * (threads - 64 * (1 + upl))) return GSBN_ERR_UNSUPPORTED;
   BlockArgs g;
   g.nlog = k->nlog;
   g.simstep = step->simstep;
@@ -3671,21 +3661,23 @@ int gsbn_step_block(const gsbn_block_args* k, const gsbn_step_args* step, void* 
   g.count_mask = k->count_mask;
   g.check = k->check;
   g.lginp_base = k->lginp_base;
-  const dim3 grid(k->nwg), t(threads);
+  const dim3 grid(k->nwg), t(k->threads);
   hipStream_t s = (hipStream_t)stream;
-#define BLK2(P, L, U)                                                                \
-  if (threads == 1024) launch_timed(block_kernel<P, L, U, 1024, 32>, grid, t, 0, s, k->pops_dev, k->projs_dev, \
-                                    k->wg_pop, k->wg_hcu, k->rows2, k->logs, g);          \
-  else launch_timed(block_kernel<P, L, U, 256, 8>, grid, t, 0, s, k->pops_dev, k->projs_dev, \
-                    k->wg_pop, k->wg_hcu, k->rows2, k->logs, g)
-#define BLK(P)                          \
-  if (k->nlog) {                        \
-    if (upl == 1) BLK2(P, true, 1);     \
-    else BLK2(P, true, 2);              \
-  } else {                              \
-    if (upl == 1) BLK2(P, false, 1);    \
-    else BLK2(P, false, 2);             \
-  }                                     \
+#define BLK2(P, L, U)                                                                             \
+  if (k->threads == 1024)                                                                         \
+    launch_timed(block_kernel<P, L, U, 1024, 32, 512>, grid, t, 0, s, k->pops_dev, k->projs_dev,  \
+                 k->wgs, k->lists, k->logs, g);                                                   \
+  else                                                                                            \
+    launch_timed(block_kernel<P, L, U, 256, 8, 128>, grid, t, 0, s, k->pops_dev, k->projs_dev,    \
+                 k->wgs, k->lists, k->logs, g)
+#define BLK(P)                             \
+  if (k->nlog) {                           \
+    if (k->max_m <= 64) BLK2(P, true, 1);  \
+    else BLK2(P, true, 2);                 \
+  } else {                                 \
+    if (k->max_m <= 64) BLK2(P, false, 1); \
+    else BLK2(P, false, 2);                \
+  }                                        \
   break
   switch (step->prec) {
     case GSBN_PREC_F32: BLK(GSBN_PREC_F32);

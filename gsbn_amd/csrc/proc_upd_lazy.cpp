@@ -260,7 +260,7 @@ class Proj : public ProjRowOps {
     return f;
   }
   int delay_min = 31; /* smallest delay of its rows */
-  DevBuf<int32_t> rows_list1; /* block step: second list of a step's rows */
+  DevBuf<int32_t> block_lists; /* block step: rows of its steps past the on-chip lists */
   uint64_t ii_version = ~0ull, di_version = ~0ull;
   int last_exec = -1;
   bool direct_que = false; /* the source population's kernel pushes this step's spikes */
@@ -1291,11 +1291,10 @@ class ProcUpdLazy : public ProcedureBase {
    * no external spikes, no wta-pop-max, and no plan asked for.
    * argi block-step 0: never; 1: every step, an error where it does not
    * apply.  GlobalVar block-step: 1 where it applies.
-   * By default up to kBlockHcus hypercolumns: what the device holds at once
-   * (256 CUs, four workgroups of 256 each).  Per step, blocks of 3 against the
-   * best split: 10 HCUs x 10 units 4.5 us (10.3), 100 x 100 8.1 us (15), 24
-   * networks (860 HCUs) 12.8 us (18); 128 networks (4600 HCUs) 51 us (34-42). */
-  static constexpr int kBlockHcus = 1024;
+   * Per step, blocks of 3 against the best split: 10 HCUs x 10 units 3.4 us
+   * (10.3), 100 x 100 6.3 us (15); batches of networks of 8-64 HCUs x 16-128
+   * units: 48 networks (1784 HCUs) 12.5 us (21.5), 128 26.7 us (36.9), 256
+   * 47.6 us (60.9), 512 (18438 HCUs) 93.4 us (93.0): no upper line. */
   int _block_arg = -1;
   bool _block = false;
   int _block_threads = 1024;
@@ -1306,7 +1305,9 @@ class ProcUpdLazy : public ProcedureBase {
     uint32_t count_mask = 0;
     int32_t* check = nullptr;
   } _held;
-  DevBuf<int32_t*> _rows2;
+  int _block_len = GSBN_BLOCK_MAX; /* steps the lists are sized for, at the first block */
+  DevBuf<int32_t*> _block_lists;
+  DevBuf<gsbn_block_wg> _block_wgs;
   std::shared_ptr<SolverMemory> _held_mem; /* where run_held and count_spikes are set */
   int block_max() const;
   bool block_applies() const;
@@ -1496,7 +1497,7 @@ bool ProcUpdLazy::block_applies() const {
 
 /* steps a block may hold: a spike's rows are active delay + 2 steps later */
 int ProcUpdLazy::block_max() const {
-  int n = GSBN_BLOCK_MAX;
+  int n = _block_len;
   for (auto* q : _list_proj) n = std::min(n, q->delay_min + 2);
   return n;
 }
@@ -1524,20 +1525,27 @@ void ProcUpdLazy::run_held() {
       apply_logs(k.simstep - 1, k.prn);
       break;
     }
+  if (!_block_lists.p) {
+    _block_len = block_max();
+    vector<int32_t*> lists;
+    for (auto* q : _list_proj) {
+      q->block_lists.alloc((size_t)_block_len * q->_dim_hcu * q->_dim_conn);
+      lists.push_back(q->block_lists.p);
+    }
+    _block_lists.upload(lists.data(), lists.size());
+  }
   gsbn_block_args b;
   memset(&b, 0, sizeof(b));
   b.pops_dev = _pop_dev.p;
   b.projs_dev = _proj_dev.p;
-  b.wg_pop = _wg_pop.p;
-  b.wg_hcu = _wg_pop_hcu.p;
-  b.rows2 = _rows2.p;
+  b.wgs = _block_wgs.p;
+  b.lists = _block_lists.p;
   b.nlog = (int)nlog();
   b.logs = b.nlog ? logs() : nullptr;
   b.nwg = _nwg_pop;
   b.nsteps = k.n;
   b.threads = _block_threads;
   b.max_m = _max_m;
-  b.max_slots = _max_slots;
   b.count_mask = k.count_mask;
   b.check = k.check;
   b.lginp_base = _pop_args[0].lginp;
@@ -2004,27 +2012,25 @@ void ProcUpdLazy::update_gpu() {
     }
     if (!_defer_k || _chain_fixed > 0) _sweep_defer = 0;
     _glv.puti("deferred-sweeps", _sweep_defer ? 1 : 0);
-    _block = _block_arg != 0 && block_applies() && (_block_arg > 0 || _nwg_pop <= kBlockHcus);
+    _block = _block_arg != 0 && block_applies();
     if (_block) {
       /* one workgroup per HCU: large ones while every HCU has a CU of its own
-       * (a step's rows in parallel), small ones beyond (more HCUs in flight);
-       * a step's ring words are held four per row thread */
-      const int words = (_max_slots + 31) / 32, role = 64 * (1 + (_max_m <= 64 ? 1 : 2));
-      _block_threads = _nwg_pop <= 256 || words > 4 * (256 - role) ? 1024 : 256;
-      if (words > 4 * (_block_threads - role)) _block = false;
+       * (a step's rows in parallel), small ones beyond (more HCUs in flight):
+       * 860 HCUs 53 ms for a run with 256 threads, 56 with 512, 67 with 1024;
+       * 100 HCUs 80 ms with 1024, 82 with 512 */
+      _block_threads = _nwg_pop <= 256 ? 1024 : 256;
     }
     if (_block_arg > 0 && !_block)
       throw Error(-2, "ProcUpdLazy: block-step needs populations of at most 128 MCUs with one "
                       "incoming projection and at most one outgoing, the population kernel's queue "
                       "push, default deferred columns, no wta-pop-max, external spikes or other plan");
     if (_block) {
-      vector<int32_t*> r2;
-      for (auto* q : _list_proj) {
-        q->rows_list1.alloc((size_t)q->_dim_hcu * q->_dim_conn);
-        r2.push_back(q->rows_list1.p);
-        q->flush_hook = [this]() { flush_deferred(); };
-      }
-      _rows2.upload(r2.data(), r2.size());
+      for (auto* q : _list_proj) q->flush_hook = [this]() { flush_deferred(); };
+      vector<gsbn_block_wg> wgs;
+      for (size_t i = 0; i < _list_pop.size(); ++i)
+        for (int h = 0; h < _list_pop[i]->_dim_hcu; ++h)
+          wgs.push_back({(int32_t)i, _in_proj_host[i], h, 0});
+      _block_wgs.upload(wgs.data(), wgs.size());
       _held_mem = active_memory()->shared_from_this();
       _held_mem->run_held = [this]() { run_held(); };
       _held_mem->count_spikes = [this](int32_t* c) { return count_held(c); };

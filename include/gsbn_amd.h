@@ -477,16 +477,17 @@ int gsbn_step_fused_batch(const gsbn_pop_args* pops_dev, int32_t npop,
  * counterpart in the reference, whose steps are separate passes. */
 #define GSBN_BLOCK_MAX 8
 typedef struct {
-  const gsbn_pop_args* pops_dev;    /* proj0.bidx names the projection in projs_dev */
+  int32_t pop, proj, hcu, pad;
+} gsbn_block_wg;
+typedef struct {
+  const gsbn_pop_args* pops_dev;
   const gsbn_rowcol_args* projs_dev;
-  const int32_t* wg_pop;
-  const int32_t* wg_hcu;
-  int32_t* const* rows2;            /* per projection, [H * C] (device) */
+  const gsbn_block_wg* wgs;         /* per workgroup (device) */
+  int32_t* const* lists;            /* per projection, [nsteps * H * C] (device) */
   const gsbn_sweep_log* logs;       /* per projection, when nlog > 0 */
   int32_t nlog, nwg, nsteps, threads; /* threads: 256, or 1024 for few HCUs */
-  int32_t max_m, max_slots;
+  int32_t max_m;
   uint32_t count_mask; /* bit s: the spikes of step s are added to check */
-  int32_t pad;
   int32_t* check;            /* [all units] */
   const float* lginp_base;   /* lginp of the first population */
 } gsbn_block_args;

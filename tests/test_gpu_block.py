@@ -71,6 +71,12 @@ def test_forms(tmp_path, k):
     _run(_spec(40, 70, 0.3, (1, 3), 900.0, train=97, **k), tmp_path)
 
 
+@pytest.mark.parametrize("H", [70, 300])
+def test_many_rows_and_recorded_changes(tmp_path, H):
+    """Rows past those held on chip, in large and small workgroups."""
+    _run(_spec(H, 3, 1.0, (1, 2), 1000.0, deferred_sweeps=1), tmp_path)
+
+
 @pytest.mark.parametrize("chunk", [1, 2, 5, 17])
 def test_reads_and_writes_between(tmp_path, chunk):
     def read(gpu, ora):

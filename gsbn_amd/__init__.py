@@ -80,6 +80,13 @@ def _p(a: np.ndarray):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+def release_memory():
+    """Give back the device memory that closed solvers left for the next ones
+    (at most an eighth of the device's)."""
+    if lib().gsbn_memory_release() != 0:
+        raise _err("release_memory")
+
+
 class Solver:
     """The reference's Solver over this library (Solver.cpp:10-92); with a
     snapshot path it resumes from that SolverState file (Solver.cpp:44-61)."""

@@ -195,6 +195,13 @@ int64_t gsbn_solver_step(gsbn_solver* s, int64_t nsteps) {
 
 int64_t gsbn_solver_run(gsbn_solver* s) { return gsbn_solver_step(s, INT64_MAX); }
 
+int gsbn_memory_release(void) {
+  return guard([&] {
+    gsbn::release_pooled_memory();
+    return 0;
+  });
+}
+
 int gsbn_solver_sync(gsbn_solver* s) {
   return guard([&] {
     if (!s || !s->s) throw Error(GSBN_ERR_ARG, "null solver");

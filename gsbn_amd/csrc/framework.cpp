@@ -48,8 +48,78 @@ SolverMemory*& active_memory() {
   return m;
 }
 
+/* Chunks of closed solvers, for the next ones: the driver clears memory that
+ * is given back, and a program that runs one 15 GB network after another (7 a
+ * second) got ahead of it: single hipMalloc and hipFree calls then took 0.3 to
+ * 4 s.  At most an eighth of the device's memory, the chunks longest unused
+ * given back first; all of it when an allocation fails or on
+ * gsbn_memory_release. */
+namespace {
+struct ChunkPool {
+  struct Entry {
+    char* base;
+    size_t size;
+    int device;
+  };
+  std::mutex mutex;
+  vector<Entry> entries; /* oldest first */
+  /* the smallest chunk of `device` with size to twice that many bytes */
+  char* take(size_t size, int device, size_t* got) {
+    std::lock_guard<std::mutex> lock(mutex);
+    auto best = entries.end();
+    for (auto it = entries.begin(); it != entries.end(); ++it)
+      if (it->device == device && it->size >= size && it->size <= 2 * size &&
+          (best == entries.end() || it->size < best->size))
+        best = it;
+    if (best == entries.end()) return nullptr;
+    char* base = best->base;
+    *got = best->size;
+    entries.erase(best);
+    return base;
+  }
+  /* no work uses the chunk any more */
+  void put(char* base, size_t size, int device) {
+    std::lock_guard<std::mutex> lock(mutex);
+    size_t avail = 0, total = 0;
+    if (hipMemGetInfo(&avail, &total) != hipSuccess) total = 0;
+    entries.push_back({base, size, device});
+    size_t held = 0;
+    for (auto& e : entries)
+      if (e.device == device) held += e.size;
+    for (auto it = entries.begin(); held > total / 8 && it != entries.end();) {
+      if (it->device != device) {
+        ++it;
+        continue;
+      }
+      (void)hipFree(it->base);
+      held -= it->size;
+      it = entries.erase(it);
+    }
+  }
+  void release() {
+    std::lock_guard<std::mutex> lock(mutex);
+    for (auto& e : entries) (void)hipFree(e.base);
+    entries.clear();
+  }
+};
+/* never destroyed: the runtime may be gone when static objects are */
+ChunkPool& chunk_pool() {
+  static ChunkPool& p = *new ChunkPool;
+  return p;
+}
+}  // namespace
+
+void release_pooled_memory() { chunk_pool().release(); }
+
 SolverMemory::~SolverMemory() {
-  for (auto& c : _chunks) (void)hipFree(c.base);
+  /* as hipFree does, the work of every stream that may use the arrays is
+   * waited for before another solver gets them */
+  int device = -1;
+  const bool keep = !_chunks.empty() && hipGetDevice(&device) == hipSuccess && device == _device &&
+                    hipDeviceSynchronize() == hipSuccess;
+  for (auto& c : _chunks)
+    if (keep) chunk_pool().put(c.base, c.size, _device);
+    else (void)hipFree(c.base);
   if (_ring) (void)hipHostFree(_ring);
   if (_bounce) (void)hipHostFree(_bounce);
   for (hipEvent_t e : _bounce_ev)
@@ -79,8 +149,20 @@ void* SolverMemory::alloc(size_t bytes) {
     size_t size = std::min(std::max(_total / 2, 4 * mb), 1024 * mb);
     size = std::max(size, need);
     size = (size + 2 * mb - 1) / (2 * mb) * (2 * mb);
-    char* base = nullptr;
-    hipError_t e = hipMalloc(&base, size);
+    int device = 0;
+    hip_check(hipGetDevice(&device), "hipGetDevice");
+    if (_chunks.empty()) _device = device;
+    if (device != _device) _device = -1; /* chunks of several devices: none is kept */
+    char* base = chunk_pool().take(size, device, &size);
+    hipError_t e = hipSuccess;
+    if (!base) {
+      e = hipMalloc(&base, size);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        release_pooled_memory();
+        e = hipMalloc(&base, size);
+      }
+    }
     if (e != hipSuccess && size > need) {
       (void)hipGetLastError();
       size = need;

@@ -94,6 +94,7 @@ class SolverMemory : public std::enable_shared_from_this<SolverMemory> {
   };
   std::mutex _mutex; /* arrays may be released from another thread */
   vector<Chunk> _chunks;
+  int _device = -1; /* of all chunks; -1: of several devices */
   map<void*, size_t> _live;
   std::multimap<size_t, void*> _free; /* released arrays by size */
   size_t _total = 0;
@@ -102,6 +103,9 @@ class SolverMemory : public std::enable_shared_from_this<SolverMemory> {
   char* _bounce = nullptr; /* pinned, two halves for large downloads */
   hipEvent_t _bounce_ev[2] = {nullptr, nullptr};
 };
+/* device memory that closed solvers left for the next ones goes back to the
+ * driver */
+void release_pooled_memory();
 /* the memory of the solver that is being built or stepped on this thread */
 SolverMemory*& active_memory();
 

@@ -912,7 +912,16 @@ struct DBuf {
     if (p) (void)hipFree(p);
     p = nullptr;
     n = count;
-    return count ? hipMalloc(&p, count * sizeof(T)) : hipSuccess;
+    if (!count) return hipSuccess;
+    hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e != hipSuccess) {
+      /* once more without the memory that closed solvers left */
+      (void)hipGetLastError();
+      p = nullptr;
+      (void)gsbn_memory_release();
+      e = hipMalloc(&p, count * sizeof(T));
+    }
+    return e;
   }
   hipError_t upload(const T* h, size_t count) {
     hipError_t e = alloc(count);

@@ -660,6 +660,10 @@ int64_t gsbn_solver_step(gsbn_solver* s, int64_t nsteps);
 /* Solver::run: until cycle-flag < 0 */
 int64_t gsbn_solver_run(gsbn_solver* s);
 int gsbn_solver_sync(gsbn_solver* s);
+/* Gives back the device memory of closed solvers that is kept for the next
+ * ones (at most an eighth of the device's; also given back when an allocation
+ * of this library fails). */
+int gsbn_memory_release(void);
 /* vector access by Database name; dtype codes 0 i8 1 i16 2 i32 3 i64 4 f16 5 f32 6 f64 */
 int64_t gsbn_solver_vector_info(gsbn_solver* s, const char* name, int* dtype);
 int64_t gsbn_solver_vector_read(gsbn_solver* s, const char* name, void* out, int64_t cap);

@@ -53,8 +53,23 @@
 #define GM_BM 256
 #define GM_BN 256
 #define GM_BK 64
-#define GM_LDK (GM_BK + 8)
-#define GM_THREADS 1024
+#define GM_GROUP 8
+/* tiles of 64 x 64 below this many of 256 x 256, half the device's CUs (64 and
+ * 256, us): 1 tile 4.6, 11; 12: 6.8, 28; 48 (1000 x 3000): 34, 76; 96 (8000 x
+ * 700): 21, 31; 144 (3000 x 3000): 87, 78; 384 (8000 x 3000): 221, 160 */
+#define GM_SMALL 128
+/* the order in which the eight MFMAs of a 16-deep step issue with the LDS
+ * reads of the next step, and with LDS writes and memory loads */
+#define GM_MFMA __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+#define GM_RD(n) __builtin_amdgcn_sched_group_barrier(0x100, n, 0);
+#define GM_WR(n) __builtin_amdgcn_sched_group_barrier(0x200, n, 0);
+#define GM_LD(n) __builtin_amdgcn_sched_group_barrier(0x020, n, 0);
+#define GM_ORDER_READS \
+  GM_MFMA GM_MFMA GM_RD(1) GM_MFMA GM_RD(1) GM_MFMA GM_RD(1) GM_MFMA GM_MFMA GM_RD(1) GM_MFMA GM_RD(1) \
+  GM_MFMA GM_RD(1)
+#define GM_ORDER_ALL                                                                              \
+  GM_MFMA GM_RD(2) GM_MFMA GM_RD(3) GM_MFMA GM_RD(1) GM_WR(2) GM_MFMA GM_WR(3) GM_MFMA GM_WR(2)   \
+  GM_MFMA GM_WR(1) GM_LD(2) GM_MFMA GM_LD(3) GM_MFMA GM_LD(3)
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 gsbn_bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float gsbn_f32x16;
@@ -747,107 +762,167 @@ __global__ void recall_weights_kernel(int H, int M, int C, int N, int Kp, const 
 }
 
 /* E[b][n] = beta E[b][n] + sum_k S[b][k] WT[n][k]: bf16 inputs, float
- * accumulation on v_mfma_f32_32x32x16_bf16.  S and WT have Kp columns (Kp a
- * multiple of GM_BK, zero padded); S has ceil(B / GM_BM) * GM_BM rows and WT
- * ceil(N / GM_BN) * GM_BN rows, so tiles never read past them.
- * A 256 x 256 output tile per workgroup of 16 waves (4 x 4, 64 x 64 each:
- * 2 x 2 MFMA blocks), K in steps of 64 through one LDS buffer (rows padded
- * by 8 bf16 against bank conflicts) with the next K tile staged in
- * registers during the current one's MFMAs.  (Measured at this problem's
- * shape: 128 x 128 tiles of 4 waves reach 0.79 PFLOP/s, double-buffered LDS
- * 0.75, 256 x 256 tiles of 16 waves 0.96; larger wave tiles, 8-wave
- * workgroups and K steps of 32 do worse.)
- * Workgroup w is remapped so that consecutive tiles of one XCD (hardware
- * workgroup w runs on XCD w % 8) share their WT tile in that XCD's L2. */
-__global__ void __launch_bounds__(GM_THREADS)
+ * accumulation on v_mfma_f32_32x32x16_bf16, k ascending.  S and WT have Kp
+ * columns (Kp a multiple of GM_BK, zero padded); S has ceil(B / GM_BM) * GM_BM
+ * rows and WT ceil(N / GM_BN) * GM_BN rows, so tiles never read past them.
+ *
+ * Large products (few tiles take 64 x 64, four waves of 32 x 32): a 256 x 256
+ * output tile per workgroup of 8 waves (128 x 64 each: 4 x 2 MFMA blocks, 6
+ * LDS reads of 16 bytes per 8 MFMAs, where 64 x 64 takes 8), K in steps of 64
+ * through two LDS buffers.  While the products of one K tile run, the next
+ * goes from registers to the other buffer and the one after that is loaded: a
+ * full K tile (1.6 us) for the loads to arrive, one barrier per K tile, behind
+ * which the last quarter of its products issues together with the first reads
+ * of the next.  Chunks are permuted within a row instead of padding (no bank
+ * conflicts; with r % 8 for r / 2 % 8, 3 of 8 LDS cycles were conflicts), and
+ * the MFMAs are interleaved with the rest (without: 1.44 ms).  Workgroup i
+ * runs on XCD i % 8: each XCD has consecutive tiles, in groups of GM_GROUP row
+ * tiles, so that its 32 workgroups share 8 + 4 tiles of operands per K step
+ * instead of 32 + 1.
+ * What bounds it: the clock under this load (2.2 GHz) and the matrix units two
+ * thirds busy; the rest is barrier skew and the tile's end, with one workgroup
+ * per CU.  8192 x 10000 x 10048: 1.27 ms, 1.30 PFLOP/s (1.60 ms with 16 waves
+ * of 64 x 64, one buffer and E read and written value by value; a vendor
+ * library's product takes 1.22-1.30 ms).  16 waves of 64 x 64 in this form
+ * 1.28 ms, K steps of 32 1.39, 128 x 256 tiles and two workgroups per CU 1.65,
+ * 128 x 128 2.6, 4 waves of 128 x 128 1.54. */
+template <int BM, int BN, int WM, int WN> /* tile, waves down and across it */
+__global__ void __launch_bounds__(64 * WM * WN)
     spike_gemm_kernel(const uint16_t* __restrict__ S, const uint16_t* __restrict__ WT,
                       float* __restrict__ E, int Bn, int N, int Kp, float beta, int mtiles,
                       int ntiles) {
-  __shared__ __attribute__((aligned(16))) uint16_t sA[GM_BM * GM_LDK];
-  __shared__ __attribute__((aligned(16))) uint16_t sB[GM_BN * GM_LDK];
+  constexpr int TM = BM / WM, TN = BN / WN, MI = TM / 32, NI = TN / 32;
+  constexpr int RP = 8 * WM * WN, NC = BM / RP; /* staged rows per pass, passes */
+  constexpr bool ORDER = MI == 4 && NI == 2 && NC == 4;
+  static_assert(BM == BN && GM_BK == 64 && RP % 16 == 0, "staging");
+  __shared__ __attribute__((aligned(16))) uint16_t sa[2][BM * GM_BK], sb[2][BN * GM_BK];
   const int nwg = mtiles * ntiles;
-  int wg = blockIdx.x;
-  if ((nwg & 7) == 0) wg = (wg & 7) * (nwg >> 3) + (wg >> 3);
-  const int nt = wg / mtiles, mt = wg - nt * mtiles;
-  const int m0 = mt * GM_BM, n0 = nt * GM_BN;
+  /* tiles of one XCD (workgroup i runs on XCD i % 8) are consecutive; there
+   * they go down GM_GROUP row tiles before the next column tile */
+  int mt, nt;
+  {
+    const int x = blockIdx.x & 7, q = nwg >> 3, r = nwg & 7;
+    const int i = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
+    const int grp = i / (GM_GROUP * ntiles), in = i - grp * GM_GROUP * ntiles;
+    const int rows = mtiles - grp * GM_GROUP < GM_GROUP ? mtiles - grp * GM_GROUP : GM_GROUP;
+    nt = in / rows;
+    mt = grp * GM_GROUP + in - nt * rows;
+  }
+  const int m0 = mt * BM, n0 = nt * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / WN, wn = wave - wm * WN;
 
-  gsbn_f32x16 acc[2][2];
+  gsbn_f32x16 acc[MI][NI];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj)
+    for (int jj = 0; jj < NI; ++jj)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][jj][r] = 0.0f;
 
-  /* global -> register staging: 2 chunks of 16 bytes per thread and matrix;
-   * chunk c = tid + 1024 i covers row c / 8, columns (c % 8) * 8 .. +7 of
-   * the K tile.  Named registers (no arrays) keep the staging out of
-   * scratch. */
-  const int crow = tid >> 3, ccol = (tid & 7) * 8; /* chunk i: row crow + 128 i */
-  const uint16_t* pa = S + (int64_t)(m0 + crow) * Kp + ccol;
-  const uint16_t* pb = WT + (int64_t)(n0 + crow) * Kp + ccol;
-  const int64_t rs = (int64_t)128 * Kp; /* 128 rows further */
-  uint4 a0, a1, b0, b1;
-#define GM_LOAD(k0)                                     \
-  a0 = *reinterpret_cast<const uint4*>(pa + (k0));      \
-  a1 = *reinterpret_cast<const uint4*>(pa + rs + (k0)); \
-  b0 = *reinterpret_cast<const uint4*>(pb + (k0));      \
-  b1 = *reinterpret_cast<const uint4*>(pb + rs + (k0));
-#define GM_STORE()                                                           \
-  *reinterpret_cast<uint4*>(&sA[(crow)*GM_LDK + ccol]) = a0;                 \
-  *reinterpret_cast<uint4*>(&sA[(crow + 128) * GM_LDK + ccol]) = a1;         \
-  *reinterpret_cast<uint4*>(&sB[(crow)*GM_LDK + ccol]) = b0;                 \
-  *reinterpret_cast<uint4*>(&sB[(crow + 128) * GM_LDK + ccol]) = b1;
+  /* 16-byte chunk c of row r of a tile lies at chunk c ^ (r / 2 % 8) of the
+   * row: the 16 rows that a 256-byte LDS access reads lie in 64 banks */
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); /* uint4 would go to scratch */
+  const int crow = tid >> 3, cc = tid & 7;
+  const uint32_t voff = (uint32_t)crow * (uint32_t)Kp * 2u + (uint32_t)cc * 16u;
+  const uint16_t* const pa = S + (int64_t)m0 * Kp;
+  const uint16_t* const pb = WT + (int64_t)n0 * Kp;
+  const int64_t rs = (int64_t)RP * Kp;
+  const int wr = crow * GM_BK + ((cc ^ ((crow >> 1) & 7)) * 8);
+  u32x4 ra[NC], rb[NC];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      ra[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(pa + i * rs + k0) + voff);
+      rb[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(pb + i * rs + k0) + voff);
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      *reinterpret_cast<u32x4*>(&sa[buf][wr + i * RP * GM_BK]) = ra[i];
+      *reinterpret_cast<u32x4*>(&sb[buf][wr + i * RP * GM_BK]) = rb[i];
+    }
+  };
+  const int arow = (wm * TM + (lane & 31)) * GM_BK, brow = (wn * TN + (lane & 31)) * GM_BK;
+  gsbn_bf16x8 af[2][MI], bf[2][NI];
+  auto frags = [&](int buf, int ks, int set) {
+    const int c = ((ks * 2 + (lane >> 5)) ^ ((lane >> 1) & 7)) * 8;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+      af[set][i] = *reinterpret_cast<const gsbn_bf16x8*>(&sa[buf][arow + i * 32 * GM_BK + c]);
+#pragma unroll
+    for (int jj = 0; jj < NI; ++jj)
+      bf[set][jj] = *reinterpret_cast<const gsbn_bf16x8*>(&sb[buf][brow + jj * 32 * GM_BK + c]);
+  };
+  auto product = [&](int set) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int jj = 0; jj < NI; ++jj)
+        acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[set][i], bf[set][jj], acc[i][jj], 0, 0, 0);
+  };
 
   const int nk = Kp / GM_BK;
-  GM_LOAD(0)
-  GM_STORE()
+  fetch(0);
+  put(0);
+  fetch(nk > 1 ? GM_BK : 0);
   __syncthreads();
+  frags(0, 0, 0);
   for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk) {
-      GM_LOAD((kt + 1) * GM_BK)
+    const int buf = kt & 1;
+    frags(buf, 1, 1);
+    product(0);
+    if constexpr (ORDER) {
+      GM_ORDER_READS
     }
-#pragma unroll
-    for (int ks = 0; ks < GM_BK / 16; ++ks) {
-      const int kk = ks * 16 + (lane >> 5) * 8;
-      gsbn_bf16x8 af[2], bf[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        af[i] = *reinterpret_cast<const gsbn_bf16x8*>(
-            &sA[(wm * 64 + i * 32 + (lane & 31)) * GM_LDK + kk]);
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
-        bf[jj] = *reinterpret_cast<const gsbn_bf16x8*>(
-            &sB[(wn * 64 + jj * 32 + (lane & 31)) * GM_LDK + kk]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-          acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bf[jj], acc[i][jj], 0, 0, 0);
+    frags(buf, 2, 0);
+    put(buf ^ 1);
+    fetch((kt + 2 < nk ? kt + 2 : nk - 1) * GM_BK); /* past the last K tile: unused */
+    product(1);
+    if constexpr (ORDER) {
+      GM_ORDER_ALL
     }
-    if (kt + 1 < nk) {
-      __syncthreads(); /* every wave is done with this K tile */
-      GM_STORE()
-      __syncthreads();
+    frags(buf, 3, 1);
+    product(0);
+    if constexpr (ORDER) {
+      GM_ORDER_READS
+    }
+    __syncthreads(); /* every wave has read this K tile and stored its part of the next */
+    frags(buf ^ 1, 0, 0);
+    product(1);
+    if constexpr (ORDER) {
+      GM_ORDER_READS
     }
   }
-#undef GM_LOAD
-#undef GM_STORE
   /* accumulator r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4 and
-   * column l % 32 of its 32 x 32 block */
+   * column l % 32 of its 32 x 32 block; a block's 16 values of E are read
+   * before the first is written (one after the other, each waits for memory) */
+  const bool inside = m0 + BM <= Bn && n0 + BN <= N; /* the whole tile */
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const int col = n0 + wn * 64 + jj * 32 + (lane & 31);
+    for (int jj = 0; jj < NI; ++jj) {
+      const int col = n0 + wn * TN + jj * 32 + (lane & 31);
+      const int row0 = m0 + wm * TM + i * 32 + (lane >> 5) * 4;
+      float v[16];
+      if (inside) {
+        float* const p = E + (int64_t)row0 * N + col;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm * 64 + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        if (row < Bn && col < N) {
-          float* p = E + (int64_t)row * N + col;
-          *p = beta * (*p) + acc[i][jj][r];
+        for (int r = 0; r < 16; ++r) v[r] = p[(int64_t)((r >> 2) * 8 + (r & 3)) * N];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          p[(int64_t)((r >> 2) * 8 + (r & 3)) * N] = beta * v[r] + acc[i][jj][r];
+      } else if (col < N) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = row0 + (r >> 2) * 8 + (r & 3);
+          v[r] = E[(int64_t)(row < Bn ? row : Bn - 1) * N + col];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int row = row0 + (r >> 2) * 8 + (r & 3);
+          if (row < Bn) E[(int64_t)row * N + col] = beta * v[r] + acc[i][jj][r];
         }
       }
     }
@@ -957,11 +1032,15 @@ extern "C" {
 int gsbn_spike_gemm(int32_t B, int32_t N, int32_t Kp, const uint16_t* S, const uint16_t* WT,
                     float* E, float beta, void* stream) {
   if (B <= 0 || N <= 0 || Kp <= 0 || Kp % GM_BK || !S || !WT || !E) return GSBN_ERR_ARG;
-  const int mtiles = (B + GM_BM - 1) / GM_BM, ntiles = (N + GM_BN - 1) / GM_BN;
-  const int64_t nwg = (int64_t)mtiles * ntiles;
-  if (nwg > 0x7fffffff) return GSBN_ERR_UNSUPPORTED;
-  hipLaunchKernelGGL(spike_gemm_kernel, dim3((unsigned)nwg), dim3(GM_THREADS), 0,
-                     (hipStream_t)stream, S, WT, E, B, N, Kp, beta, mtiles, ntiles);
+  auto launch = [&](auto kernel, int bm, int threads) {
+    const int mtiles = (B + bm - 1) / bm, ntiles = (N + bm - 1) / bm;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(mtiles * (int64_t)ntiles)), dim3(threads), 0,
+                       (hipStream_t)stream, S, WT, E, B, N, Kp, beta, mtiles, ntiles);
+  };
+  const int64_t tiles = (int64_t)((B + GM_BM - 1) / GM_BM) * ((N + GM_BN - 1) / GM_BN);
+  if (tiles > 0x7fffffff) return GSBN_ERR_UNSUPPORTED;
+  if (tiles < GM_SMALL) launch(spike_gemm_kernel<64, 64, 2, 2>, 64, 256);
+  else launch(spike_gemm_kernel<GM_BM, GM_BN, 2, 4>, GM_BM, 512);
   return ret(hipGetLastError());
 }
 

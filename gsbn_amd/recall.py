@@ -3,8 +3,9 @@
 A trained population's recurrent weights Wij and biases bj are frozen and B
 partial cues run in lock-step through the reference's recall-mode dynamics
 (prn = 0), either with float weights in the reference's summation order
-("exact") or with the support as one bfloat16 product of the spike matrix
-and W on the matrix cores ("mfma").
+("exact") or with the support of one bfloat16 product of the spike matrix
+and W on the matrix cores ("mfma"; computed from the spikes alone where that is
+cheaper, with the same bits).
 """
 
 from __future__ import annotations

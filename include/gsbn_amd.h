@@ -608,9 +608,10 @@ int gsbn_device_math(int op, int64_t n, const void* in_host, void* out_host);
  * epsc = 0, cue b drawing with Philox key seed + b, population 0.
  * GSBN_RECALL_EXACT adds float Wij of the active rows in the reference's
  * ascending row order (a single-cue solver run with the same weights gives
- * the same spikes); GSBN_RECALL_MFMA computes the support of all cues as
- * the product of the 0/1 spike matrix and W in bfloat16 on the matrix cores
- * with float accumulation (one delay for all rows required). */
+ * the same spikes); GSBN_RECALL_MFMA gives the support of all cues the value
+ * of the product of the 0/1 spike matrix and W in bfloat16 on the matrix cores
+ * with float accumulation (one delay for all rows required), computed from
+ * the spikes alone where that is cheaper, with the same bits. */
 #define GSBN_RECALL_EXACT 0
 #define GSBN_RECALL_MFMA 1
 typedef struct {

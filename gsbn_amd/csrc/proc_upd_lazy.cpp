@@ -1294,7 +1294,9 @@ class ProcUpdLazy : public ProcedureBase {
    * Per step, blocks of 3 against the best split: 10 HCUs x 10 units 3.4 us
    * (10.3), 100 x 100 6.3 us (15); batches of networks of 8-64 HCUs x 16-128
    * units: 48 networks (1784 HCUs) 12.5 us (21.5), 128 26.7 us (36.9), 256
-   * 47.6 us (60.9), 512 (18438 HCUs) 93.4 us (93.0): no upper line. */
+   * 47.6 us (60.9), 512 (18438 HCUs) 93.4 us (93.0): by default up to
+   * kBlockHcus, 64 workgroups per CU. */
+  static constexpr int kBlockHcus = 16384;
   int _block_arg = -1;
   bool _block = false;
   int _block_threads = 1024;
@@ -2012,7 +2014,7 @@ void ProcUpdLazy::update_gpu() {
     }
     if (!_defer_k || _chain_fixed > 0) _sweep_defer = 0;
     _glv.puti("deferred-sweeps", _sweep_defer ? 1 : 0);
-    _block = _block_arg != 0 && block_applies();
+    _block = _block_arg != 0 && block_applies() && (_block_arg > 0 || _nwg_pop <= kBlockHcus);
     if (_block) {
       /* one workgroup per HCU: large ones while every HCU has a CU of its own
        * (a step's rows in parallel), small ones beyond (more HCUs in flight):

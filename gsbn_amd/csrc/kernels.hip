@@ -3335,7 +3335,10 @@ int gsbn_proj_walk_batch(const gsbn_pop_args* pops_dev, const int32_t* wg_pop,
   hipLaunchKernelGGL(walk_list_kernel_batch, dim3(nwg), dim3(64), 0, s, pops_dev, wg_pop, wg_pop_hcu,
                      due);
   const int parts = (max_slots + 511) / 512 < 64 ? (max_slots + 511) / 512 : 64;
-  const dim3 g(nhcu, parts), t(RC_THREADS);
+  /* most workgroups find nothing listed: no more than fill the device a few
+   * times over (512 networks: 240 k of them, 1.3 us per step more) */
+  const int room = 65536 / nhcu > 1 ? 65536 / nhcu : 1;
+  const dim3 g(nhcu, parts < room ? parts : room), t(RC_THREADS);
 #define WALK(P)                                                                                   \
   if (n) hipLaunchKernelGGL((walk_kernel_batch<P, true>), g, t, 0, s, projs_dev, wg_proj,         \
                             wg_proj_hcu, *step, logs, n);                                         \

@@ -278,6 +278,7 @@ int gsbn_solver_check(gsbn_solver* s, int32_t* correct, int32_t* total, int32_t*
                       int32_t cap) {
   return guard([&] {
     if (!s || !s->s || !correct || !total) throw Error(GSBN_ERR_ARG, "null argument");
+    s->s->flush(); /* the window results are read on this solver's stream */
     std::vector<int> f;
     int c = 0, t = 0;
     if (!gsbn::check_results(s->s->upd(), &c, &t, &f)) throw Error(GSBN_ERR_STATE, "no ProcCheck");

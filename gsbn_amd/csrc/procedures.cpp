@@ -719,10 +719,9 @@ void ProcCheck::update_gpu() {
 void ProcCheck::report(bool final_line) {
   const int nw = (int)_window_mode.size();
   if (nw > _reported) {
-    hip_check(hipStreamSynchronize(active_stream()), "sync");
     vector<int32_t> idx((size_t)nw * _total_hcu), cnt((size_t)nw * _total_hcu);
-    hip_check(hipMemcpy(idx.data(), _res_idx.p, idx.size() * 4, hipMemcpyDeviceToHost), "D2H");
-    hip_check(hipMemcpy(cnt.data(), _res_cnt.p, cnt.size() * 4, hipMemcpyDeviceToHost), "D2H");
+    _res_idx.download(idx.data(), idx.size());
+    _res_cnt.download(cnt.data(), cnt.size());
     std::fstream out(_logfile, std::ios::out | std::ios::app);
     for (int w = _reported; w < nw; ++w) {
       const mode_t& m = _list_mode[_window_mode[w]];

@@ -908,12 +908,24 @@ void Proj::rebuild_fanout() {
 }
 
 void Proj::prepare(int simstep) {
+  bool kicks_done = false;
   for (VecBase* v : views) {
     if (v->status == VecBase::HOST_NEWER && v->view) {
       v->view->push(v);
       v->status = VecBase::SYNCED;
       if (v == _ti || v == _tij) floor_t = INT32_MIN;
+      if (v == _tij) kicks_done = true;
     }
+  }
+  if (_ii->host_version != ii_version) kicks_done = true;
+  /* the kicks of the steps so far have reached the synapses that were there
+   * (materialize_kicks, before a host write is taken over): to a synapse whose
+   * time is set back, or to a slot that gets its source now, the rings'
+   * entries would look pending, so the rings start empty again */
+  if (kicks_done && dK && last_exec >= 0) {
+    const int64_t N = (int64_t)_dim_hcu * _dim_mcu;
+    op_check(gsbn_i32_fill(dcnt.p, N, 0, active_stream()), "fill");
+    op_check(gsbn_i32_fill(dfl.p, N, 0, active_stream()), "fill");
   }
   if (_ii->host_version != ii_version || _di->host_version != di_version) {
     rebuild_fanout();

@@ -1379,7 +1379,6 @@ class ProcUpdLazy : public ProcedureBase {
   int _sweep_defer = -1;
   DevBuf<gsbn_sweep_log> _logs_dev; /* per projection */
   uint64_t _logs_tables = ~0ull, _logs_seen = ~0ull; /* what the device's logs hold */
-  int _best_split = 0;
   size_t nlog() const { return _list_proj.empty() ? 0 : _list_proj[0]->log.size(); }
   const gsbn_sweep_log* logs();
   void apply_logs(int upto, float prn);
@@ -1387,12 +1386,20 @@ class ProcUpdLazy : public ProcedureBase {
   int _defer_arg = -1; /* the argument, -1 when not given */
   int _defer_k = kDeferDefault;
   void end_deferral();
-  bool _tuned = false;
-  int _tune_pos = 0, _run_len = 0;
-  vector<int> _cand;
-  vector<hipEvent_t> _tev;
+  /* _tune[0] tunes the steps without recorded sweeps, and its choice serves
+   * all steps once it is made.  Until then, the steps with recorded sweeps,
+   * which run other kernels and no chained launch, have the samples of
+   * _tune[1]: a change recorded early (the log is emptied by reads and writes
+   * of the state only) neither mixes the two nor holds the tuning up. */
+  struct Tuner {
+    bool tuned = false;
+    int pos = 0, run_len = 0, best = 0, best_split = 0;
+    vector<int> cand;
+    vector<hipEvent_t> ev;
+  } _tune[2];
+  int _tune_kind = 0;
   int rowcol_parts(hipStream_t s, bool* timed);
-  void finish_tuning();
+  void finish_tuning(Tuner& t);
 };
 REGISTERIMPL(ProcUpdLazy);
 
@@ -1401,7 +1408,8 @@ ProcUpdLazy::~ProcUpdLazy() {
     _held_mem->run_held = nullptr;
     _held_mem->count_spikes = nullptr;
   }
-  for (hipEvent_t e : _tev) (void)hipEventDestroy(e);
+  for (Tuner& t : _tune)
+    for (hipEvent_t e : t.ev) (void)hipEventDestroy(e);
   for (auto* p : _list_proj) delete p;
   for (auto* p : _list_pop) delete p;
 }
@@ -1618,7 +1626,8 @@ void ProcUpdLazy::end_deferral() {
 }
 
 /* the plan of this step; *timed while tuning (the step belongs to run
- * _tune_pos, timed by events _tev[2 _tune_pos] and _tev[2 _tune_pos + 1]) */
+ * `pos` of the tuner _tune[_tune_kind], timed by events ev[2 pos] and
+ * ev[2 pos + 1]) */
 int ProcUpdLazy::rowcol_parts(hipStream_t s, bool* timed) {
   *timed = false;
   if (_fused_fixed) return -1;
@@ -1626,37 +1635,46 @@ int ProcUpdLazy::rowcol_parts(hipStream_t s, bool* timed) {
   if (_graded_fixed > 0) return -10 - _graded_fixed;
   if (_wave_fixed > 0) return -19 - _wave_fixed;
   if (_parts_fixed > 0) return _parts_fixed;
-  if (_tuned || execs < kTuneStart) return _parts;
-  if (_cand.empty()) {
+  const int kind = nlog() && !_tune[0].tuned ? 1 : 0;
+  Tuner& t = _tune[kind];
+  if (kind != _tune_kind) {
+    _tune_kind = kind;
+    _chain_warm = 0;
+    _glv.puti("rowcol-parts", t.tuned ? t.best : _parts);
+    _glv.puti("plan-tuned", t.tuned ? 1 : 0);
+  }
+  if (t.tuned) return t.best;
+  if (execs < kTuneStart) return _parts;
+  if (t.cand.empty()) {
     for (int c : {1, 2, 4, 8, 16, 32})
-      if ((int64_t)c * std::max(_nhcu_proj, 1) <= 262144) _cand.push_back(c);
+      if ((int64_t)c * std::max(_nhcu_proj, 1) <= 262144) t.cand.push_back(c);
     /* and the largest split whose grid the device holds at once (a grid
      * beyond it waits for a second dispatch round) */
     int32_t res = 0;
     const int prec = _list_proj.empty() ? GSBN_PREC_F32 : _list_proj[0]->prec;
     if (gsbn_rowcol_resident(prec, &res) == 0) {
       const int fit = res / std::max(_nhcu_proj, 1);
-      if (fit > 1 && fit < 32 && std::find(_cand.begin(), _cand.end(), fit) == _cand.end())
-        _cand.push_back(fit);
+      if (fit > 1 && fit < 32 && std::find(t.cand.begin(), t.cand.end(), fit) == t.cand.end())
+        t.cand.push_back(fit);
     }
-    if (_cand.empty()) _cand.push_back(1);
-    if (_fusable) _cand.push_back(-1);
-    if (_chainable) _cand.push_back(-2);
-    if (_batch && !_hcu_work.empty()) _cand.push_back(-20);
+    if (t.cand.empty()) t.cand.push_back(1);
+    if (_fusable) t.cand.push_back(-1);
+    if (_chainable && kind == 0) t.cand.push_back(-2);
+    if (_batch && !_hcu_work.empty()) t.cand.push_back(-20);
     /* graded splits; their maps are built here, before any sample is timed
      * (their one-wave forms, plans -21 to -23, are no candidates: on 512
      * networks the best of them, -21, ran within 2 % of plan -20, and every
      * candidate more spreads the tuner's samples thinner) */
     if (_batch && !_hcu_work.empty())
       for (int g = 1; g <= 3; ++g) {
-        _cand.push_back(-10 - g);
+        t.cand.push_back(-10 - g);
         if (!_gmap_n[g]) build_graded_map(g);
       }
-    _tev.resize(2 * _cand.size() * kTuneSamples);
-    for (auto& e : _tev) hip_check(hipEventCreate(&e), "hipEventCreate");
+    t.ev.resize(2 * t.cand.size() * kTuneSamples);
+    for (auto& e : t.ev) hip_check(hipEventCreate(&e), "hipEventCreate");
   }
   (void)s;
-  const int c = _cand[_tune_pos % _cand.size()];
+  const int c = t.cand[t.pos % t.cand.size()];
   /* a chained sample is the second of two chained steps (the first one
    * leaves the work that a chained launch takes over) */
   if (c == -2 && !_chain_warm) {
@@ -1668,33 +1686,33 @@ int ProcUpdLazy::rowcol_parts(hipStream_t s, bool* timed) {
   return c;
 }
 
-void ProcUpdLazy::finish_tuning() {
-  const size_t nc = _cand.size();
-  hip_check(hipEventSynchronize(_tev.back()), "hipEventSynchronize");
+void ProcUpdLazy::finish_tuning(Tuner& t) {
+  const size_t nc = t.cand.size();
+  hip_check(hipEventSynchronize(t.ev.back()), "hipEventSynchronize");
   float best = 0.0f, best_split = 0.0f;
   for (size_t c = 0; c < nc; ++c) {
-    vector<float> t;
+    vector<float> v;
     for (int k = 0; k < kTuneSamples; ++k) {
       const size_t i = (size_t)k * nc + c;
       float ms = 0.0f;
-      hip_check(hipEventElapsedTime(&ms, _tev[2 * i], _tev[2 * i + 1]), "hipEventElapsedTime");
-      t.push_back(ms / kTuneRun);
+      hip_check(hipEventElapsedTime(&ms, t.ev[2 * i], t.ev[2 * i + 1]), "hipEventElapsedTime");
+      v.push_back(ms / kTuneRun);
     }
-    std::nth_element(t.begin(), t.begin() + t.size() / 2, t.end());
-    const float med = t[t.size() / 2];
+    std::nth_element(v.begin(), v.begin() + v.size() / 2, v.end());
+    const float med = v[v.size() / 2];
     /* the measured median step time of each plan, for inspection */
-    _glv.putf("step-plan-ms" + std::to_string(_cand[c]), med);
+    _glv.putf("step-plan-ms" + std::to_string(t.cand[c]), med);
     if (c == 0 || med < best) {
       best = med;
-      _parts = _cand[c];
+      t.best = t.cand[c];
     }
-    if (_cand[c] > 0 && (_best_split == 0 || med < best_split)) {
+    if (t.cand[c] > 0 && (t.best_split == 0 || med < best_split)) {
       best_split = med;
-      _best_split = _cand[c];
+      t.best_split = t.cand[c];
     }
   }
-  _tuned = true;
-  _glv.puti("rowcol-parts", _parts);
+  t.tuned = true;
+  _glv.puti("rowcol-parts", t.best);
   /* the plan is final from the next step on */
   _glv.puti("plan-tuned", 1);
 }
@@ -2116,7 +2134,7 @@ void ProcUpdLazy::update_gpu() {
     throw Error(-2, "wmask-idx " + std::to_string(wmask_idx) + " out of range");
 
   const bool blocks = _block && (_block_arg > 0 || active_memory()->call_steps > 1);
-  if (blocks) _run_len = 0; /* a tuning run restarts after the blocks */
+  if (blocks) _tune[_tune_kind].run_len = 0; /* a tuning run restarts after the blocks */
   if (blocks && !sweep) {
     /* the first step of a block */
     flush_deferred();
@@ -2158,8 +2176,9 @@ void ProcUpdLazy::update_gpu() {
    * run the sweep between the two launches and are not tuning samples */
   bool timed = false;
   int plan = _list_proj.empty() ? 1 : blocks ? _parts0 : rowcol_parts(stream, &timed);
+  Tuner& tune = _tune[_tune_kind];
   if (sweep) {
-    if (timed) _run_len = 0; /* the run restarts after the sweep */
+    if (timed) tune.run_len = 0; /* the run restarts after the sweep */
     timed = false;
     _chain_warm = 0;
     if (plan == -1) plan = _parts0;
@@ -2167,7 +2186,7 @@ void ProcUpdLazy::update_gpu() {
   /* a chained launch has no form for recorded sweeps: the best of the
    * splits runs while there are any */
   if (_sweep_defer && plan == -2 && (sweep || nlog())) {
-    plan = _best_split ? _best_split : _parts0;
+    plan = tune.best_split ? tune.best_split : _parts0;
     timed = false;
   }
   if (plan != -2 && _pending) flush_deferred();
@@ -2182,8 +2201,8 @@ void ProcUpdLazy::update_gpu() {
     if (_ovf_exec != (int64_t)_exec - 1)
       op_check(gsbn_i32_fill(_ovf_cnt.p, kOvfCounters, 0, stream), "fill"); /* not cleared by the last step */
   }
-  const size_t ev = 2 * (size_t)_tune_pos;
-  if (timed && _run_len == 0) hip_check(hipEventRecord(_tev[ev], stream), "hipEventRecord");
+  const size_t ev = 2 * (size_t)tune.pos;
+  if (timed && tune.run_len == 0) hip_check(hipEventRecord(tune.ev[ev], stream), "hipEventRecord");
 
   gsbn_pop_args pa;
   if (!_batch) {
@@ -2371,10 +2390,10 @@ void ProcUpdLazy::update_gpu() {
       q->kick_kp = q->_taupdt * prn;
       q->kicks_pending = true;
     }
-  if (timed && ++_run_len == kTuneRun) {
-    hip_check(hipEventRecord(_tev[ev + 1], stream), "hipEventRecord");
-    _run_len = 0;
-    if (++_tune_pos == (int)(_cand.size() * kTuneSamples)) finish_tuning();
+  if (timed && ++tune.run_len == kTuneRun) {
+    hip_check(hipEventRecord(tune.ev[ev + 1], stream), "hipEventRecord");
+    tune.run_len = 0;
+    if (++tune.pos == (int)(tune.cand.size() * kTuneSamples)) finish_tuning(tune);
   }
   if (touched)
     for (auto* q : _list_proj) q->mark_views_device();

@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "../../include/gsbn_amd.h"
+#include "dbuf.h"
 #include "detfast.h"
 #include "detmath.h"
 #include "gsbn_core.h"
@@ -975,35 +976,6 @@ __global__ void re_decay(float* E, int64_t n, float beta) {
        i += (int64_t)gridDim.x * blockDim.x)
     E[i] = beta * E[i] + 0.0f;
 }
-
-template <typename T>
-struct DBuf {
-  T* p = nullptr;
-  size_t n = 0;
-  ~DBuf() {
-    if (p) (void)hipFree(p);
-  }
-  hipError_t alloc(size_t count) {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    n = count;
-    if (!count) return hipSuccess;
-    hipError_t e = hipMalloc(&p, count * sizeof(T));
-    if (e != hipSuccess) {
-      /* once more without the memory that closed solvers left */
-      (void)hipGetLastError();
-      p = nullptr;
-      (void)gsbn_memory_release();
-      e = hipMalloc(&p, count * sizeof(T));
-    }
-    return e;
-  }
-  hipError_t upload(const T* h, size_t count) {
-    hipError_t e = alloc(count);
-    if (e == hipSuccess && count) e = hipMemcpy(p, h, count * sizeof(T), hipMemcpyHostToDevice);
-    return e;
-  }
-};
 
 }  // namespace
 

@@ -1159,6 +1159,10 @@ gsbn_recall* gsbn_recall_new(const gsbn_recall_desc* d) {
   if (r->wave) {
     ok(r->src_cnt.alloc((size_t)r->R * B));
     ok(r->src_list.alloc((size_t)r->R * B * N));
+  } else if (d->mode == GSBN_RECALL_MFMA) {
+    /* the spike matrices of the product (a handle of the wave kernel makes
+     * them in its first run that asks for the product's time) */
+    ok(r->S.alloc((size_t)RE_RING * r->Bp * r->Kp));
   }
   ok(hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking));
   ok(hipEventCreate(&r->ev0));
@@ -1262,10 +1266,11 @@ int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, in
       }
     } else {
       const int64_t ns = (int64_t)RE_RING * r->Bp * r->Kp;
-      if (!r->S.p && (e = r->S.alloc((size_t)ns)) != hipSuccess)
+      if (!r->S.p && steps > 0 && (e = r->S.alloc((size_t)ns)) != hipSuccess)
         return fail((int)e, "gsbn_recall_run: spike matrices");
-      hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(ns / 2)), dim3(256), 0, s,
-                         reinterpret_cast<float*>(r->S.p), ns / 2, 0.0f);
+      if (steps > 0)
+        hipLaunchKernelGGL(re_fill_f32, dim3(grid_of(ns / 2)), dim3(256), 0, s,
+                           reinterpret_cast<float*>(r->S.p), ns / 2, 0.0f);
     }
     if (raster && (int64_t)r->raster.n < BN) {
       e = r->raster.alloc((size_t)BN);

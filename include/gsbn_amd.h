@@ -635,7 +635,10 @@ void gsbn_recall_free(gsbn_recall* r);
  * t > count_from are counted; out_idx/out_cnt[b*H + h] = first strict maximum
  * of the counts and its count (-1 / 0 without spikes, ProcCheck/Pop.cpp:35-50).
  * raster (optional, host, steps*batch*H*M int8) receives every step's spikes;
- * support_ms (optional) the summed time of the support products (mfma). */
+ * support_ms (optional) the summed time of the support products (mfma); a
+ * handle that otherwise computes the support without the product takes it in
+ * every step of such a run, and makes its spike matrices (128 bytes per cue
+ * and unit) in the first one. */
 int gsbn_recall_run(gsbn_recall* r, const int16_t* clamp, const float* wmask, int32_t steps,
                     int32_t count_from, int32_t* out_idx, int32_t* out_cnt, int8_t* raster,
                     double* support_ms);

@@ -721,6 +721,28 @@ __device__ __forceinline__ PopStep pop_step(const gsbn_pop_args& a, const gsbn_s
           a.wmask + st.wmask_offset, st.ovf_keep, st.ovf_cap, st.ovf_cnt, st.ovf_task};
 }
 
+/* The draws, exponentials and logarithms of a population update: by the short
+ * sequences (detfast.h) or, with the same bits, by the full ones.  The short
+ * ones save issue where a kernel has registers for them (pop_kernel at 100 x
+ * 100 9.8 -> 9.0 us); the batched kernels, held to 80 registers, spilled 4 to
+ * 14 of them (512 networks 49.2 -> 56.1 us) and keep the full ones. */
+template <bool SHORT>
+__device__ __forceinline__ void draw_unit(uint64_t seed, uint32_t pop, uint32_t step, uint32_t unit,
+                                          float* u01, float* z) {
+  if constexpr (SHORT) gsbn_draw_unit_guarded(seed, pop, step, unit, u01, z);
+  else gsbn_draw_unit(seed, pop, step, unit, u01, z);
+}
+template <bool SHORT>
+__device__ __forceinline__ float exp_of(float x) {
+  if constexpr (SHORT) return gsbn_expf_guarded(x);
+  else return gsbn_expf(x);
+}
+template <bool SHORT>
+__device__ __forceinline__ float log_of(float x) {
+  if constexpr (SHORT) return gsbn_logf_guarded(x);
+  else return gsbn_logf(x);
+}
+
 /* One hypercolumn's population update.  FUSED: `f` also receives what the
  * fused step's row/column phase needs (one incoming projection).
  *
@@ -730,7 +752,7 @@ __device__ __forceinline__ PopStep pop_step(const gsbn_pop_args& a, const gsbn_s
  * contributions are read before their count is known), and every global
  * store of the update is issued after the last load: loads and stores share
  * one in-order counter, so a load issued behind stores would wait for them. */
-template <bool FUSED, int CPREC = -1, int NPRE = 4, bool SPEC = true>
+template <bool FUSED, int CPREC = -1, int NPRE = 4, bool SPEC = true, bool SHORT = true>
 __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& ps, const int h,
                                          FusedLds* f = nullptr,
                                          const gsbn_rowcol_args* rb = nullptr,
@@ -841,7 +863,7 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
   float u = 0.0f, xi = 0.0f;
   if (live) {
     float z;
-    gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)idx, &u, &z);
+    draw_unit<SHORT>(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)idx, &u, &z);
     xi = a.snoise * z;
   }
   float pj_n = 0.0f, ej_n = 0.0f, zj_n = 0.0f, bj_n = 0.0f;
@@ -855,7 +877,7 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
     ej_n = ej0 + (zj0 - ej0) * p0.ke;
     zj_n = zj0 * (1 - p0.kzj);
     bj_w = kp != 0.0f;
-    if (bj_w) bj_n = p0.bgain * gsbn_logf_guarded(pj_n + p0.eps);
+    if (bj_w) bj_n = p0.bgain * log_of<SHORT>(pj_n + p0.eps);
   }
   if (j > 0 && j < nin) sh_pend[j] = a.projs[j].pend_cnt[h];
   __syncthreads();
@@ -930,10 +952,10 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
 
   /* soft-max (Pop.cpp:280-302); the normaliser is summed in ascending unit
    * order by one thread, four LDS words per read */
-  const float maxact = gsbn_expf_guarded(a.wtagain * maxdsup);
+  const float maxact = exp_of<SHORT>(a.wtagain * maxdsup);
   float act = 0.0f;
   if (live) {
-    act = gsbn_expf_guarded(a.wtagain * (dsup - maxdsup));
+    act = exp_of<SHORT>(a.wtagain * (dsup - maxdsup));
     if (maxact < 1.0f) act *= maxact;
     sh_f[j] = act;
   }
@@ -1078,7 +1100,7 @@ __device__ __forceinline__ void pop_body(const gsbn_pop_args& a, const PopStep& 
       ej += (zj - ej) * p.ke;
       zj *= (1 - p.kzj);
       if (spk > 0) zj += p.kftj;
-      if (kp != 0.0f) a.bj[m * N + idx] = p.bgain * gsbn_logf_guarded(pj + p.eps);
+      if (kp != 0.0f) a.bj[m * N + idx] = p.bgain * log_of<SHORT>(pj + p.eps);
       p.pj[idx] = pj;
       p.ej[idx] = ej;
       p.zj[idx] = zj;
@@ -1255,7 +1277,7 @@ __global__ void __launch_bounds__(POP_MAX_THREADS, 6)
     if (w != (int)blockIdx.x) __syncthreads(); /* LDS of the previous hypercolumn */
     const gsbn_pop_args& a = arr[wg_pop[w]];
     touch_lines<sizeof(gsbn_pop_args)>(&a);
-    pop_body<false, -1, 1, false>(a, pop_step(a, st), wg_hcu[w]);
+    pop_body<false, -1, 1, false, false>(a, pop_step(a, st), wg_hcu[w]);
   }
 }
 
@@ -1324,7 +1346,7 @@ __device__ __forceinline__ void pop_body_w(const gsbn_pop_args& a, const PopStep
     bj_w[u] = false;
     if (j < M) {
       float z;
-      gsbn_draw_unit_guarded(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)(h * M + j), &ud[u],
+      gsbn_draw_unit(a.seed, (uint32_t)a.pop_id, (uint32_t)ps.simstep, (uint32_t)(h * M + j), &ud[u],
                      &z);
       xi[u] = a.snoise * z;
       if (ps.do_jxx && nin > 0) {
@@ -1333,7 +1355,7 @@ __device__ __forceinline__ void pop_body_w(const gsbn_pop_args& a, const PopStep
         ej_n[u] = ej0[u] + (zj0[u] - ej0[u]) * p0.ke;
         zj_n[u] = zj0[u] * (1 - p0.kzj);
         bj_w[u] = kp != 0.0f;
-        if (bj_w[u]) bj_n[u] = p0.bgain * gsbn_logf_guarded(pj_n[u] + p0.eps);
+        if (bj_w[u]) bj_n[u] = p0.bgain * gsbn_logf(pj_n[u] + p0.eps);
       }
     }
   }
@@ -1376,14 +1398,14 @@ __device__ __forceinline__ void pop_body_w(const gsbn_pop_args& a, const PopStep
   }
 
   /* soft-max (Pop.cpp:280-302), the normaliser in ascending unit order */
-  const float maxact = gsbn_expf_guarded(a.wtagain * maxdsup);
+  const float maxact = gsbn_expf(a.wtagain * maxdsup);
   float act[UPL];
 #pragma unroll
   for (int u = 0; u < UPL; ++u) {
     const int j = lane + 64 * u;
     act[u] = 0.0f;
     if (j < M) {
-      act[u] = gsbn_expf_guarded(a.wtagain * (dsup[u] - maxdsup));
+      act[u] = gsbn_expf(a.wtagain * (dsup[u] - maxdsup));
       if (maxact < 1.0f) act[u] *= maxact;
       sh_f[j] = act[u];
     }

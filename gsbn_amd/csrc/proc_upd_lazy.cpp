@@ -1309,6 +1309,16 @@ class ProcUpdLazy : public ProcedureBase {
    * 47.6 us (60.9), 512 (18438 HCUs) 93.4 us (93.0): by default up to
    * kBlockHcus, 64 workgroups per CU. */
   static constexpr int kBlockHcus = 16384;
+  /* A block of one step keeps the launch saved, but not the state: with a
+   * stimulus row of its own for every step (or a recorder that reads every
+   * step), 100 x 100 takes 8.0 us a step as blocks and 12.5 with the tuned
+   * plans, batches of 960 HCUs 8.9 (14.0), 1784 14.4 (16.4), 2439 19.1 (18.3),
+   * 3070 21.7 (19.2), 4659 30.7 (23.9), 14500 82.6 (47.5); blocks of two are
+   * faster at all of them.  So beyond kAloneHcus, eight workgroups per CU, the
+   * tuned plans run after three steps in a row that could not join the one
+   * before, and at the start, until one could. */
+  static constexpr int kAloneHcus = 2048;
+  int _alone = 3; /* steps in a row that could not join the one before */
   int _block_arg = -1;
   bool _block = false;
   int _block_threads = 1024;
@@ -1319,6 +1329,11 @@ class ProcUpdLazy : public ProcedureBase {
     uint32_t count_mask = 0;
     int32_t* check = nullptr;
   } _held;
+  struct { /* the step before */
+    int simstep = -1;
+    float prn = 0.0f;
+    int64_t lg_off = 0, wm_off = 0;
+  } _last;
   int _block_len = GSBN_BLOCK_MAX; /* steps the lists are sized for, at the first block */
   DevBuf<int32_t*> _block_lists;
   DevBuf<gsbn_block_wg> _block_wgs;
@@ -2093,12 +2108,20 @@ void ProcUpdLazy::update_gpu() {
   Pop* p0 = _list_pop.front();
   const int64_t lg_off = p0->_lginp->ld() <= 0 ? (int64_t)lginp_idx : (int64_t)lginp_idx * p0->_lginp->ld();
   const int64_t wm_off = p0->_wmask->ld() <= 0 ? (int64_t)wmask_idx : (int64_t)wmask_idx * p0->_wmask->ld();
+  /* whether this step goes on as the one before, so that a block may hold both */
+  const bool joins = !sweep && simstep == _last.simstep + 1 && !memcmp(&prn, &_last.prn, 4) &&
+                     lg_off == _last.lg_off && wm_off == _last.wm_off &&
+                     VecBase::host_epoch() == _epoch_seen &&
+                     VecBase::host_write_epoch() == _write_epoch_seen && !_args_dirty &&
+                     _tables.version == _tables_seen && simstep <= _tables.sim_end;
+  _alone = joins ? 0 : _alone + 1;
+  _last.simstep = simstep;
+  _last.prn = prn;
+  _last.lg_off = lg_off;
+  _last.wm_off = wm_off;
   if (_held.n) {
-    /* one more step of the block being held, if it goes on as before */
-    if (!sweep && _held.n < block_max() && simstep == _held.simstep + _held.n &&
-        !memcmp(&prn, &_held.prn, 4) && lg_off == _held.lg_off && wm_off == _held.wm_off &&
-        VecBase::host_epoch() == _epoch_seen && VecBase::host_write_epoch() == _write_epoch_seen &&
-        !_args_dirty && _tables.version == _tables_seen && simstep <= _tables.sim_end) {
+    /* one more step of the block being held */
+    if (joins && _held.n < block_max()) {
       ++_held.n;
       for (auto* q : _list_proj) {
         q->last_exec = _exec;
@@ -2133,7 +2156,9 @@ void ProcUpdLazy::update_gpu() {
   if (wmask_idx < 0 || wm_off + _total_hcus > (int64_t)p0->_wmask->size())
     throw Error(-2, "wmask-idx " + std::to_string(wmask_idx) + " out of range");
 
-  const bool blocks = _block && (_block_arg > 0 || active_memory()->call_steps > 1);
+  const bool blocks =
+      _block && (_block_arg > 0 || (active_memory()->call_steps > 1 &&
+                                    (_nwg_pop <= kAloneHcus || _alone <= 2)));
   if (blocks) _tune[_tune_kind].run_len = 0; /* a tuning run restarts after the blocks */
   if (blocks && !sweep) {
     /* the first step of a block */

@@ -142,6 +142,11 @@ struct DevBuf {
     else
       hip_check(hipStreamSynchronize(active_stream()), "sync");
   }
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+    mem.swap(o.mem);
+  }
 
  private:
   std::shared_ptr<SolverMemory> mem;

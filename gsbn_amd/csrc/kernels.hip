@@ -2672,6 +2672,21 @@ __global__ void walk_list_kernel_batch(const gsbn_pop_args* __restrict__ arr,
   list_due(a.proj0, wg_hcu[blockIdx.x], a.M, due);
 }
 
+/* gsbn_ring_deepen: a unit's last K0 - 1 kicks, oldest first, from the start of
+ * its ring of K1 (the counts restart with them, so that no entry before them is
+ * ever read) */
+__global__ void ring_deepen_kernel(const gsbn_ring_move* __restrict__ moves, int K0, int K1) {
+  const gsbn_ring_move m = moves[blockIdx.y];
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m.N;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int T = m.dcnt[i], n = T < K0 - 1 ? T : K0 - 1;
+    for (int q = 0; q < n; ++q) m.to[i * K1 + q] = m.from[i * K0 + ((T - n + q) & (K0 - 1))];
+    const int since = T - m.dfl[i];
+    m.dcnt[i] = n;
+    m.dfl[i] = since < n ? n - since : 0;
+  }
+}
+
 /* the listed units' columns: rowcol_body's column pass with no active rows
  * (no row carries the stamp -2); part blockIdx.y of the HCU's slots */
 template <int PREC, bool LOG>
@@ -3317,6 +3332,19 @@ int gsbn_proj_rowcol_log(const gsbn_rowcol_args* a, const gsbn_sweep_log* log, i
                          void* stream) {
   if (!log_ok(log, n) || !a || a->dK <= 0) return GSBN_ERR_ARG;
   return launch_rowcol(a, log, n, stream);
+}
+
+int gsbn_ring_deepen(const gsbn_ring_move* moves, int32_t n, int64_t max_units, int32_t K0,
+                     int32_t K1, void* stream) {
+  if (!moves || n < 0 || max_units < 0 || K0 < 2 || (K0 & (K0 - 1)) || K1 < K0 || (K1 & (K1 - 1)))
+    return GSBN_ERR_ARG;
+  if (n == 0 || max_units == 0) return 0;
+  /* (65535 projections at most in a grid's y) */
+  for (int32_t p = 0; p < n; p += 65535)
+    hipLaunchKernelGGL(ring_deepen_kernel,
+                       dim3(grid_for(max_units, 256, 1024), n - p < 65535 ? n - p : 65535), dim3(256),
+                       0, (hipStream_t)stream, moves + p, K0, K1);
+  return launch_status();
 }
 
 int gsbn_proj_walk(const gsbn_pop_proj* p, const gsbn_rowcol_args* a, int32_t due,

@@ -1367,16 +1367,21 @@ class ProcUpdLazy : public ProcedureBase {
   int _wave_fixed = 0;
   /* deferred-columns K: column updates deferred through rings of K spike
    * steps per unit (0: eager); see Proj::dK.  Same results for every K.
-   * GlobalVar deferred-columns reports K, 8 for one network and 16 for a
-   * batch when it is not given; the rings then hold kRing steps (GlobalVar
-   * deferred-ring) and are walked between the steps. */
+   * GlobalVar deferred-columns reports the depth in use (deferred-ring too).
+   * Without the argument: 8 for one network and 16 for a batch, walked inside
+   * the steps, until steps are run in blocks or a sweep is recorded. */
   static constexpr int kDeferDefault = 8, kDeferBatch = 16;
-  /* Without the argument, every kWalkEvery steps the units with kWalkDue or
-   * more spikes since their last walk are walked by a launch of its own over
-   * the whole device; at most kWalkDue - 1 + kWalkEvery < 63 spikes are then
-   * ever pending, so no step walks a column itself (a walk inside a step holds
-   * the step: 9900 slots by the few workgroups of one hypercolumn) */
+  /* From then on (_deep) the rings hold kRing steps, and every kWalkEvery
+   * steps the units with kWalkDue or more spikes since their last walk are
+   * walked by a launch of its own over the whole device; at most kWalkDue - 1
+   * + kWalkEvery < 63 spikes are then ever pending, so no step walks a column
+   * itself (a block cannot, and a walk with recorded sweeps inside a step holds
+   * the step: 9900 slots by the few workgroups of one hypercolumn).  Plain
+   * steps keep the shallow rings: on 512 networks 84.8 us a step with 16, 86.3
+   * with 64 and the walk launches; 128 networks 37.5 and 38.6. */
   static constexpr int kRing = 64, kWalkEvery = 32, kWalkDue = 30;
+  bool _deep = false;
+  void deepen_rings();
   int _walk_age = 0; /* steps since the last walk launch */
   /* deferred-sweeps 1 (with deferred column updates, not with a forced
    * chained step): learning-rate changes are recorded instead of sweeping
@@ -1637,7 +1642,37 @@ void ProcUpdLazy::end_deferral() {
   _sweep_defer = 0;
   _args_dirty = true;
   _glv.puti("deferred-columns", 0);
+  _glv.puti("deferred-ring", 0);
   _glv.puti("deferred-sweeps", 0);
+}
+
+void ProcUpdLazy::deepen_rings() {
+  if (_deep || !_defer_k || _defer_arg >= 0) return;
+  flush_deferred(); /* the pending work of a chained step walks the rings as they are */
+  vector<gsbn_ring_move> moves(_list_proj.size());
+  vector<DevBuf<int32_t>> rings(_list_proj.size()); /* all of them, before one is replaced */
+  int64_t most = 0;
+  for (size_t i = 0; i < moves.size(); ++i) {
+    Proj* q = _list_proj[i];
+    const int64_t N = (int64_t)q->_dim_hcu * q->_dim_mcu;
+    rings[i].alloc((size_t)N * kRing);
+    moves[i] = {N, q->dhist.p, rings[i].p, q->dcnt.p, q->dfl.p};
+    most = std::max(most, N);
+  }
+  DevBuf<gsbn_ring_move> dev;
+  dev.upload(moves.data(), moves.size());
+  op_check(gsbn_ring_deepen(dev.p, (int32_t)moves.size(), most, _list_proj[0]->dK, kRing,
+                            active_stream()),
+           "gsbn_ring_deepen");
+  for (size_t i = 0; i < rings.size(); ++i) {
+    _list_proj[i]->dhist.swap(rings[i]);
+    _list_proj[i]->dK = kRing;
+  }
+  _deep = true;
+  _walk_age = 0; /* at most kDeferBatch - 1 kicks are pending */
+  _args_dirty = true;
+  _glv.puti("deferred-columns", kRing);
+  _glv.puti("deferred-ring", kRing);
 }
 
 /* the plan of this step; *timed while tuning (the step belongs to run
@@ -2044,10 +2079,14 @@ void ProcUpdLazy::update_gpu() {
     }
     /* the fused launch does eager column updates: asking for it asks for them */
     if (_fused_fixed) _defer_k = 0;
+    _block = _block_arg != 0 && block_applies() && (_block_arg > 0 || _nwg_pop <= kBlockHcus);
     if (_defer_k) {
       _fusable = false;
+      /* deep from the start where the first steps run in blocks */
+      _deep = _block && (_block_arg > 0 ||
+                         (active_memory()->call_steps > 1 && _nwg_pop <= kAloneHcus));
       for (auto* q : _list_proj) {
-        q->enable_deferred(_defer_arg >= 0 ? _defer_k : kRing);
+        q->enable_deferred(_deep ? kRing : _defer_k);
         q->eager_hook = [this]() { end_deferral(); };
         q->log_hook = [this]() { return logs(); };
       }
@@ -2059,7 +2098,6 @@ void ProcUpdLazy::update_gpu() {
     }
     if (!_defer_k || _chain_fixed > 0) _sweep_defer = 0;
     _glv.puti("deferred-sweeps", _sweep_defer ? 1 : 0);
-    _block = _block_arg != 0 && block_applies() && (_block_arg > 0 || _nwg_pop <= kBlockHcus);
     if (_block) {
       /* one workgroup per HCU: large ones while every HCU has a CU of its own
        * (a step's rows in parallel), small ones beyond (more HCUs in flight):
@@ -2082,7 +2120,7 @@ void ProcUpdLazy::update_gpu() {
       _held_mem->run_held = [this]() { run_held(); };
       _held_mem->count_spikes = [this](int32_t* c) { return count_held(c); };
     }
-    _glv.puti("deferred-columns", _defer_k);
+    _glv.puti("deferred-columns", _defer_k ? _list_proj[0]->dK : 0);
     _glv.puti("deferred-ring", _defer_k ? _list_proj[0]->dK : 0);
     /* GlobalVar pop-wave: units per lane of the one-wave population launch
      * of a batch (0: the block kernel, or no batch) */
@@ -2148,6 +2186,13 @@ void ProcUpdLazy::update_gpu() {
     for (auto* q : _list_proj) q->prepare(simstep);
   for (auto* q : _list_proj)
     if (q->resume_pending) q->restore_queue(_exec);
+  const bool blocks =
+      _block && (_block_arg > 0 || (active_memory()->call_steps > 1 &&
+                                    (_nwg_pop <= kAloneHcus || _alone <= 2)));
+  bool deep = blocks;
+  if (sweep && _sweep_defer)
+    for (auto* q : _list_proj) deep = deep || simstep - 1 > q->floor_t; /* see record_sweep */
+  if (deep) deepen_rings();
   if (touched || _args_dirty || _tables.version != _tables_seen) refresh_args(simstep);
 
   /* current .lginp / .wmask rows (Pop.cpp:331-332) */
@@ -2156,9 +2201,6 @@ void ProcUpdLazy::update_gpu() {
   if (wmask_idx < 0 || wm_off + _total_hcus > (int64_t)p0->_wmask->size())
     throw Error(-2, "wmask-idx " + std::to_string(wmask_idx) + " out of range");
 
-  const bool blocks =
-      _block && (_block_arg > 0 || (active_memory()->call_steps > 1 &&
-                                    (_nwg_pop <= kAloneHcus || _alone <= 2)));
   if (blocks) _tune[_tune_kind].run_len = 0; /* a tuning run restarts after the blocks */
   if (blocks && !sweep) {
     /* the first step of a block */
@@ -2394,7 +2436,7 @@ void ProcUpdLazy::update_gpu() {
   }
   /* (a chained step's row updates come with the next launch: its walks stay
    * inside the steps, as its column workgroups run them in parallel) */
-  if (_defer_k && _defer_arg < 0 && plan != -2 &&
+  if (_deep && _defer_k && plan != -2 &&
       ++_walk_age + (_block ? GSBN_BLOCK_MAX - 1 : 0) >= kWalkEvery) {
     _walk_age = 0;
     const int n = (int)nlog();

@@ -340,6 +340,20 @@ int gsbn_proj_rowcol(const gsbn_rowcol_args* a, void* stream);
 int gsbn_proj_rowcol_log(const gsbn_rowcol_args* a, const gsbn_sweep_log* log, int32_t n,
                          void* stream);
 
+/* The kicks of several projections' units moved from rings of K0 steps to
+ * deeper ones of K1, both powers of two: the last K0 - 1 of each unit, whose
+ * counts restart at that many.  moves: n of them, in device memory; max_units:
+ * the largest N. */
+typedef struct {
+  int64_t N;           /* units */
+  const int32_t* from; /* [N * K0] */
+  int32_t* to;         /* [N * K1] */
+  int32_t* dcnt;       /* spikes so far, [N] */
+  int32_t* dfl;        /* dcnt at the last column walk, [N] */
+} gsbn_ring_move;
+int gsbn_ring_deepen(const gsbn_ring_move* moves, int32_t n, int64_t max_units, int32_t K0,
+                     int32_t K1, void* stream);
+
 /* Column walks between steps: every unit of p's projection whose spikes since
  * its last walk number `due` or more has its pending column kicks (of steps
  * up to a->simstep) applied in every slot with ii >= 0, so that a ring of dK

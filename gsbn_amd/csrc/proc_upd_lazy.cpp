@@ -94,6 +94,7 @@ struct TableCache {
   std::map<std::array<uint32_t, 4>, std::unique_ptr<CoefTable>> m;
   uint64_t version = 0;
   uint64_t log_version = 0; /* changes with any projection's recorded sweeps */
+  int64_t swept = 0;        /* synapse updates of recorded sweeps, when applied */
   int sim_end = 0;
   const CoefTable& get(float kzi, float kzj, float ke, float kp, int64_t need) {
     std::array<uint32_t, 4> key;
@@ -988,6 +989,7 @@ void Proj::apply_log(const gsbn_sweep_log* logs, int upto, float kp) {
   Timing::get().begin(2, active_stream());
   op_check(gsbn_proj_sweep_log(&a, logs + _id, n, active_stream()), "gsbn_proj_sweep_log");
   Timing::get().end(2, active_stream());
+  tcache->swept += (int64_t)n * nsyn;
   floor_t = log.back().target;
   log.clear();
   ++tcache->log_version;
@@ -1230,6 +1232,7 @@ class ProcUpdLazy : public ProcedureBase {
   void update_cpu() override;
   void update_gpu() override;
   int64_t work(int i);
+  int64_t swept() const { return sweep_synapses + _tables.swept; }
   int64_t sweep_synapses = 0, sweeps = 0, execs = 0;
 
  private:
@@ -1499,6 +1502,8 @@ void ProcUpdLazy::record_sweep(int simstep, float old_prn, float prn, const gsbn
     }
   bool need = false;
   for (auto* q : _list_proj) need = need || target > q->floor_t;
+  if (!need)
+    for (auto* q : _list_proj) sweep_synapses += q->nsyn; /* a sweep that changes nothing */
   const int slot = (int)nlog();
   hipStream_t s = active_stream();
   if (need)
@@ -2368,8 +2373,9 @@ void ProcUpdLazy::update_gpu() {
     for (auto* p : _list_pop) p->flush_pending = true;
     if (sweep) {
       for (auto* q : _list_proj) {
-        if (!_sweep_defer) q->update_all(simstep, old_prn);
-        sweep_synapses += (int64_t)q->_dim_hcu * q->_dim_conn * q->_dim_mcu;
+        if (_sweep_defer) continue;
+        q->update_all(simstep, old_prn);
+        sweep_synapses += q->nsyn;
       }
       sweeps++;
       if (_sweep_defer)
@@ -2491,7 +2497,7 @@ bool updlazy_work(Upd& upd, int64_t* out5) {
     if (u) {
       out5[0] = u->work(0);
       out5[1] = u->work(1);
-      out5[2] = u->sweep_synapses;
+      out5[2] = u->swept();
       out5[3] = u->execs;
       out5[4] = u->sweeps;
       return true;

@@ -692,7 +692,8 @@ int gsbn_solver_global(gsbn_solver* s, const char* key, char type, void* out);
 int gsbn_solver_check(gsbn_solver* s, int32_t* correct, int32_t* total, int32_t* flags,
                       int32_t cap);
 /* counters: [0] row synapse updates [1] column synapse updates [2] sweep
- * synapse updates [3] executed steps [4] sweeps */
+ * synapse updates (of recorded sweeps: counted when a pass applies them)
+ * [3] executed steps [4] learning-rate changes, one sweep each */
 int gsbn_solver_work(gsbn_solver* s, int64_t* out5);
 /* per-kernel timing with HIP events on the solver stream.  enable > 0 is a
  * bit mask of the kinds to time (0 pop, 1 rowcol, 2 all, 3 jxx, 4 que, 5

@@ -40,7 +40,6 @@ hipStream_t& active_stream() {
 }
 
 /* ------------------------------------------------------------------ */
-/* ------------------------------------------------------------------ */
 /* SolverMemory */
 
 SolverMemory*& active_memory() {
@@ -63,12 +62,12 @@ struct ChunkPool {
   };
   std::mutex mutex;
   vector<Entry> entries; /* oldest first */
-  /* the smallest chunk of `device` with size to twice that many bytes */
-  char* take(size_t size, int device, size_t* got) {
+  /* the smallest chunk of `device` with size to `most` bytes */
+  char* take(size_t size, size_t most, int device, size_t* got) {
     std::lock_guard<std::mutex> lock(mutex);
     auto best = entries.end();
     for (auto it = entries.begin(); it != entries.end(); ++it)
-      if (it->device == device && it->size >= size && it->size <= 2 * size &&
+      if (it->device == device && it->size >= size && it->size <= most &&
           (best == entries.end() || it->size < best->size))
         best = it;
     if (best == entries.end()) return nullptr;
@@ -115,9 +114,10 @@ SolverMemory::~SolverMemory() {
   /* as hipFree does, the work of every stream that may use the arrays is
    * waited for before another solver gets them */
   int device = -1;
-  const bool keep = !_chunks.empty() && hipGetDevice(&device) == hipSuccess && device == _device &&
+  const auto& chunks = _arrays.chunks();
+  const bool keep = !chunks.empty() && hipGetDevice(&device) == hipSuccess && device == _device &&
                     hipDeviceSynchronize() == hipSuccess;
-  for (auto& c : _chunks)
+  for (auto& c : chunks)
     if (keep) chunk_pool().put(c.base, c.size, _device);
     else (void)hipFree(c.base);
   if (_ring) (void)hipHostFree(_ring);
@@ -128,63 +128,37 @@ SolverMemory::~SolverMemory() {
 
 void* SolverMemory::alloc(size_t bytes) {
   std::lock_guard<std::mutex> lock(_mutex);
-  const size_t need = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
-  /* a released array of at most twice the size */
-  auto f = _free.lower_bound(need);
-  if (f != _free.end() && f->first <= 2 * need) {
-    void* p = f->second;
-    _live[p] = f->first;
-    _free.erase(f);
-    return p;
-  }
-  /* the chunk with the smallest tail that holds it */
-  Chunk* at = nullptr;
-  for (auto& c : _chunks)
-    if (c.size - c.used >= need && (!at || c.size - c.used < at->size - at->used)) at = &c;
-  if (!at) {
-    /* chunks grow with what the solver holds already, from 4 MB to 1 GB, so
-     * a solver makes few of them and leaves at most a third of its memory, or
-     * 1 GB, unused */
-    const size_t mb = (size_t)1 << 20;
-    size_t size = std::min(std::max(_total / 2, 4 * mb), 1024 * mb);
-    size = std::max(size, need);
-    size = (size + 2 * mb - 1) / (2 * mb) * (2 * mb);
-    int device = 0;
-    hip_check(hipGetDevice(&device), "hipGetDevice");
-    if (_chunks.empty()) _device = device;
-    if (device != _device) _device = -1; /* chunks of several devices: none is kept */
-    char* base = chunk_pool().take(size, device, &size);
-    hipError_t e = hipSuccess;
-    if (!base) {
-      e = hipMalloc(&base, size);
-      if (e != hipSuccess) {
-        (void)hipGetLastError();
-        release_pooled_memory();
-        e = hipMalloc(&base, size);
-      }
-    }
-    if (e != hipSuccess && size > need) {
-      (void)hipGetLastError();
-      size = need;
-      e = hipMalloc(&base, size);
-    }
-    hip_check(e, "hipMalloc");
-    _chunks.push_back({base, size, 0});
-    _total += size;
-    at = &_chunks.back();
-  }
-  void* p = at->base + at->used;
-  at->used += need;
-  _live[p] = need;
+  void* p = _arrays.alloc(bytes);
+  if (!p) hip_check(_error, "hipMalloc");
   return p;
+}
+
+/* a chunk of at least `size` bytes: a kept one of up to `most`, or a new one */
+char* SolverMemory::ChunkSource::take(size_t size, size_t most, size_t* got) {
+  int device = 0;
+  hip_check(hipGetDevice(&device), "hipGetDevice");
+  if (mem->_arrays.chunks().empty()) mem->_device = device;
+  if (device != mem->_device) mem->_device = -1; /* chunks of several devices: none is kept */
+  char* base = chunk_pool().take(size, most, device, got);
+  if (base) return base;
+  hipError_t e = hipMalloc(&base, size);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    release_pooled_memory();
+    e = hipMalloc(&base, size);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    mem->_error = e;
+    return nullptr;
+  }
+  *got = size;
+  return base;
 }
 
 void SolverMemory::release(void* p) {
   std::lock_guard<std::mutex> lock(_mutex);
-  auto it = _live.find(p);
-  if (it == _live.end()) return;
-  _free.emplace(it->second, p);
-  _live.erase(it);
+  _arrays.release(p);
 }
 
 /* Up to 8 MB go through the pinned ring and return without waiting; when the

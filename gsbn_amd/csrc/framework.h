@@ -34,6 +34,8 @@
 #include <string>
 #include <vector>
 
+#include "chunks.h"
+
 namespace gsbn {
 
 using std::map;
@@ -88,16 +90,14 @@ class SolverMemory : public std::enable_shared_from_this<SolverMemory> {
   }
 
  private:
-  struct Chunk {
-    char* base;
-    size_t size, used;
+  struct ChunkSource {
+    SolverMemory* mem;
+    char* take(size_t size, size_t most, size_t* got);
   };
   std::mutex _mutex; /* arrays may be released from another thread */
-  vector<Chunk> _chunks;
+  Chunks<ChunkSource> _arrays{ChunkSource{this}};
   int _device = -1; /* of all chunks; -1: of several devices */
-  map<void*, size_t> _live;
-  std::multimap<size_t, void*> _free; /* released arrays by size */
-  size_t _total = 0;
+  hipError_t _error = hipSuccess; /* of the last allocation that failed */
   char* _ring = nullptr; /* pinned, for uploads */
   size_t _ring_size = 0, _ring_pos = 0;
   char* _bounce = nullptr; /* pinned, two halves for large downloads */

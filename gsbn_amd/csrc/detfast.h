@@ -126,10 +126,15 @@ GSBN_HD GSBN_INLINE int gsbn_round_safe(double y) {
   return d > GSBN_GUARD || d < -GSBN_GUARD;
 }
 
-/* seeds of 1/x and 1/sqrt(x), at least 22 bits */
+/* Seeds of 1/x and 1/sqrt(x), within 2^-24 relative (the instructions are
+ * specified to 2^29 units in the last place).  One Newton step on a seed that
+ * is off by e leaves e^2 = 3.6e-15 of the reciprocal and 1.5 e^2 = 5.3e-15 of
+ * the square root.  A host build can set the seeds' error (GSBN_SEED_ERROR). */
 GSBN_HD GSBN_INLINE double gsbn_rcp_seed(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_rcp(x);
+#elif defined(GSBN_SEED_ERROR)
+  return (1.0 + GSBN_SEED_ERROR) / x;
 #else
   return (double)(1.0f / (float)x);
 #endif
@@ -137,6 +142,8 @@ GSBN_HD GSBN_INLINE double gsbn_rcp_seed(double x) {
 GSBN_HD GSBN_INLINE double gsbn_rsq_seed(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return __builtin_amdgcn_rsq(x);
+#elif defined(GSBN_SEED_ERROR)
+  return (1.0 + GSBN_SEED_ERROR) / __builtin_sqrt(x);
 #else
   return (double)(1.0f / __builtin_sqrtf((float)x));
 #endif
@@ -178,7 +185,7 @@ GSBN_HD GSBN_INLINE double gsbn_exp_short(double x) {
 
 /* log x in double for a normal positive float: the same reduction and
  * series, to s^17 (truncation below 1e-15), 1/(m+1) from the seed and one
- * Newton step (below 1e-14) */
+ * Newton step (4e-15; up to 8e-15 of a logarithm that cancels) */
 GSBN_HD GSBN_INLINE double gsbn_log_short(float x) {
   const uint32_t b = gsbn_fbits(x);
   const uint32_t mb = b & 0x7fffffu;
@@ -237,17 +244,23 @@ GSBN_HD GSBN_INLINE float gsbn_logf_guarded(float x) {
   return (float)gsbn_log_cold((double)x);
 }
 
-/* The standard normal of two 24-bit words (gsbn_draw_unit) by the short forms (k1 + 1 <= 2^24 is exact in
- * float; cos(2 pi u) = sin(2 pi (1/4 - a)) with a the distance of u from the
- * nearest integer; the square root from the seed and one Newton step), in
- * full where the guard says so or u1 = 1 (whose result is a signed zero). */
-GSBN_HD GSBN_INLINE float gsbn_normal24_guarded(uint32_t k1, uint32_t k2) {
+/* The standard normal of two 24-bit words (gsbn_draw_unit) in double by the
+ * short forms (k1 + 1 <= 2^24 is exact in float; cos(2 pi u) = sin(2 pi (1/4 -
+ * a)) with a the distance of u from the nearest integer; the square root from
+ * the seed and one Newton step) */
+GSBN_HD GSBN_INLINE double gsbn_normal24_short(uint32_t k1, uint32_t k2) {
   const double t = -2.0 * gsbn_log_short((float)(k1 + 1u) * 5.9604644775390625e-08f);
   const double y = gsbn_rsq_seed(t);
   const double g = t * y;
   const double r = __builtin_fma(0.5 * g, __builtin_fma(-g, y, 1.0), g);
   const uint32_t a = k2 <= 0x800000u ? k2 : 0x1000000u - k2;
-  const double z = r * gsbn_sin2pi24(0x400000 - (int)a);
+  return r * gsbn_sin2pi24(0x400000 - (int)a);
+}
+
+/* rounded, in full where the guard says so or u1 = 1 (whose result is a signed
+ * zero) */
+GSBN_HD GSBN_INLINE float gsbn_normal24_guarded(uint32_t k1, uint32_t k2) {
+  const double z = gsbn_normal24_short(k1, k2);
   if (k1 != 0xffffffu && gsbn_round_safe(z)) return (float)z;
   return gsbn_normal24_cold(k1, k2);
 }

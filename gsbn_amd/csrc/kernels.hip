@@ -2869,6 +2869,21 @@ __global__ void __launch_bounds__(1024) que_kernel(gsbn_que_args a) {
   }
 }
 
+/* the same push taken back */
+__global__ void __launch_bounds__(1024) unque_kernel(gsbn_que_args a) {
+  const int hs = blockIdx.x;
+  for (int j = 0; j < a.Msrc; ++j) {
+    const int n = hs * a.Msrc + j;
+    if (a.si[n] <= 0) continue;
+    const int q1 = a.out.fwd_off[n + 1];
+    for (int q = a.out.fwd_off[n] + threadIdx.x; q < q1; q += blockDim.x) {
+      const int r = a.out.fwd_row[q], hh = r / a.out.C, k = r - hh * a.out.C;
+      const int slot = (a.exec + 1 + a.out.fwd_del[q]) % GSBN_FUT;
+      atomicAnd(a.out.fut + ((int64_t)slot * a.out.H + hh) * a.out.W + (k >> 5), ~(1u << (k & 31)));
+    }
+  }
+}
+
 __global__ void check_count_kernel(int n, const int8_t* spike, int32_t* count) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     count[i] += (spike[i] > 0) ? 1 : 0;
@@ -3742,13 +3757,23 @@ int gsbn_step_block(const gsbn_block_args* k, const gsbn_step_args* step, void* 
   return launch_status();
 }
 
+static bool que_ok(const gsbn_que_args* a) {
+  return a && a->Hsrc > 0 && a->Msrc > 0 && a->exec >= 0 && a->si && a->out.fwd_off &&
+         a->out.fwd_row && a->out.fwd_del && a->out.fut && a->out.H > 0 && a->out.C > 0 &&
+         a->out.W == (a->out.C + 31) / 32;
+}
+
 int gsbn_proj_que(const gsbn_que_args* a, void* stream) {
-  if (!a || a->Hsrc <= 0 || a->Msrc <= 0 || a->exec < 0 || !a->si || !a->out.fwd_off ||
-      !a->out.fwd_row || !a->out.fwd_del || !a->out.fut || a->out.H <= 0 || a->out.C <= 0 ||
-      a->out.W != (a->out.C + 31) / 32)
-    return GSBN_ERR_ARG;
+  if (!que_ok(a)) return GSBN_ERR_ARG;
   const int threads = a->Msrc >= 1024 ? 1024 : ((a->Msrc + 63) / 64) * 64;
   launch_timed(que_kernel, dim3(a->Hsrc), dim3(threads), 0, (hipStream_t)stream, *a);
+  return launch_status();
+}
+
+int gsbn_proj_unque(const gsbn_que_args* a, void* stream) {
+  if (!que_ok(a)) return GSBN_ERR_ARG;
+  const int threads = a->Msrc >= 1024 ? 1024 : ((a->Msrc + 63) / 64) * 64;
+  hipLaunchKernelGGL(unque_kernel, dim3(a->Hsrc), dim3(threads), 0, (hipStream_t)stream, *a);
   return launch_status();
 }
 

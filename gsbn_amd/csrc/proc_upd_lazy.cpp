@@ -147,6 +147,7 @@ class Proj : public ProjRowOps {
   }
   gsbn_rowcol_args static_args(const float* slot_prn, int nslots, int64_t need);
   void rebuild_fanout();
+  gsbn_que_args last_push();
   TableCache* tcache = nullptr;
 
   int _id = 0, _rank = 0, _proj_in_pop = 0, _dim_conn = 0, _dim_hcu = 0, _dim_mcu = 0, _nsrc = 0;
@@ -908,6 +909,18 @@ void Proj::rebuild_fanout() {
   fwd_del.upload(del.data(), del.size());
 }
 
+/* the queue push of the last step's spikes */
+gsbn_que_args Proj::last_push() {
+  gsbn_que_args a;
+  memset(&a, 0, sizeof(a));
+  a.Hsrc = _ptr_src_pop->_dim_hcu;
+  a.Msrc = _ptr_src_pop->_dim_mcu;
+  a.exec = last_exec + 1; /* pushes as exec - 1 */
+  a.si = _ptr_src_pop->_spike->gpu_data();
+  a.out = fanout();
+  return a;
+}
+
 void Proj::prepare(int simstep) {
   bool kicks_done = false;
   for (VecBase* v : views) {
@@ -929,9 +942,17 @@ void Proj::prepare(int simstep) {
     op_check(gsbn_i32_fill(dfl.p, N, 0, active_stream()), "fill");
   }
   if (_ii->host_version != ii_version || _di->host_version != di_version) {
+    /* where the population kernel pushes, the spikes of the last step went out
+     * over the connectivity as it was; the reference pushes them at the next
+     * step, over the one it has then */
+    const bool again = direct_que && last_exec >= 0;
+    gsbn_que_args a = last_push();
+    if (again) op_check(gsbn_proj_unque(&a, active_stream()), "gsbn_proj_unque");
     rebuild_fanout();
     ii_version = _ii->host_version;
     di_version = _di->host_version;
+    a.out = fanout();
+    if (again) op_check(gsbn_proj_que(&a, active_stream()), "gsbn_proj_que");
   }
   (void)_ii->gpu_data();
   (void)_di->gpu_data();
@@ -1200,21 +1221,9 @@ void Proj::clear_rows(const vector<int32_t>& rows) {
 void Proj::rows_added() {
   flush_deferred();
   if (eager_hook) eager_hook();
-  /* the fan-out lists follow ii/di now */
+  /* the fan-out lists follow ii/di now, and the last step's push with them */
   prepare(0);
-  /* with the population kernel doing the queue push, the spikes of the last
-   * step went out over the old fan-out lists; pushing them again over the
-   * new ones adds the new rows' bits (setting a bit twice changes nothing) */
-  if (!direct_que || last_exec < 0) return;
-  gsbn_que_args a;
-  memset(&a, 0, sizeof(a));
-  a.Hsrc = _ptr_src_pop->_dim_hcu;
-  a.Msrc = _ptr_src_pop->_dim_mcu;
-  a.exec = last_exec + 1; /* pushes as exec - 1 */
-  a.si = _ptr_src_pop->_spike->gpu_data();
-  a.out = fanout();
-  op_check(gsbn_proj_que(&a, active_stream()), "gsbn_proj_que");
-  mark_views_device();
+  if (direct_que && last_exec >= 0) mark_views_device();
 }
 
 void Proj::mark_views_device() {

@@ -516,6 +516,9 @@ typedef struct {
   gsbn_fanout out;
 } gsbn_que_args;
 int gsbn_proj_que(const gsbn_que_args* a, void* stream);
+/* that push taken back, with the same arguments (before the fan-out changes;
+ * the bits it set are cleared) */
+int gsbn_proj_unque(const gsbn_que_args* a, void* stream);
 
 /* ProcCheck counting (ProcCheck/Pop.cpp:20-28) and per-HCU first strict
  * argmax with counter reset (ProcCheck/Pop.cpp:35-50). */

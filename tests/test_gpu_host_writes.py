@@ -1,6 +1,8 @@
-"""Host writes between steps (-m gpu) of the state that pending column kicks
-depend on: synapse times set back, and slots that get a source.  The kicks of
-the steps before belong to the synapses as they were; against the oracle."""
+"""Host writes between steps (-m gpu) of the state that pending column kicks and
+the queue push depend on: synapse times set back, and slots that get or change
+their source.  The kicks of the steps before belong to the synapses as they
+were, the push of the last step's spikes to the connectivity as it is; against
+the oracle."""
 
 import numpy as np
 import pytest
@@ -30,7 +32,7 @@ def _set_back(s):
 
 def _new_sources(s):
     ii, di = s.vector("ii_0"), s.vector("di_0")
-    free = np.flatnonzero(ii < 0)
+    free = np.flatnonzero(ii < 0)[::2]
     assert free.size > 3
     ii[free] = 1 + np.arange(free.size, dtype=np.int32) % 7
     di[free] = 2
@@ -38,11 +40,21 @@ def _new_sources(s):
     s.write("di_0", di)
 
 
-@pytest.mark.parametrize("write", [_set_back])
+def _other_sources(s):
+    """Taken slots whose source or delay changes."""
+    ii, di = s.vector("ii_0"), s.vector("di_0")
+    taken = np.flatnonzero(ii >= 0)
+    ii[taken[::3]] = (ii[taken[::3]] + 11) % 72
+    di[taken[1::3]] = 5
+    s.write("ii_0", ii)
+    s.write("di_0", di)
+
+
+@pytest.mark.parametrize("write", [_set_back, _new_sources, _other_sources])
 @pytest.mark.parametrize("chunk", [1, 50])
 @pytest.mark.parametrize("k", [dict(), dict(deferred_columns=4), dict(deferred_columns=64),
                                dict(deferred_columns=0), dict(deferred_sweeps=1),
-                               dict(chained_step=1)])
+                               dict(chained_step=1), dict(exchange_direct=False)])
 def test_kicks_of_before_a_write(tmp_path, write, chunk, k):
     spec = _spec(k)
     gpu = Solver(configs.write(spec, str(tmp_path)))

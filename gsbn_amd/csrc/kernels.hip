@@ -137,13 +137,6 @@ unsigned loop_grid(K kernel, int threads, size_t lds, int64_t n) {
   return (unsigned)n;
 }
 
-/* LDS operations of a wave are processed in order; this only keeps the
- * compiler from moving them across */
-__device__ __forceinline__ void wave_order() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 /* exclusive prefix sum across the workgroup (blockDim multiple of 64);
  * sh needs blockDim/64 + 1 ints */
 __device__ int block_excl_scan(int v, int* sh, int* total) {

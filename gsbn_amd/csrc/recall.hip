@@ -373,13 +373,6 @@ __global__ void __launch_bounds__(256) recall_pop_wave_kernel(ReArgs a, int t) {
 
 #define RW_WAVES 4 /* cues per workgroup of recall_wave_kernel */
 
-/* LDS operations of a wave are processed in order; this only keeps the
- * compiler from moving them across */
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 /* acc[u] (unit lane + 64 u) += W's 16-source block `blk`, sources of `bits`,
  * by the matrix instruction of spike_gemm_kernel on the same operands: rows 0
  * and 4 of the A block hold the cue, so accumulator 0 of a lane (row 0 for
@@ -661,7 +654,7 @@ __global__ void __launch_bounds__(64 * RW_WAVES, BF ? (UPL == 1 ? 5 : UPL == 2 ?
       const int span = BF ? N : a.C;
       for (int w0 = 0; w0 < span; w0 += 2048) {
         sh_bm[wave][lane] = 0u;
-        wave_lds_fence();
+        wave_order();
         for (int d = a.dmin; d <= a.dmax; ++d) {
           const int s = t - d - 2;
           if (s < 1) break;
@@ -682,9 +675,9 @@ __global__ void __launch_bounds__(64 * RW_WAVES, BF ? (UPL == 1 ? 5 : UPL == 2 ?
             }
           }
         }
-        wave_lds_fence();
+        wave_order();
         const int word = (int)sh_bm[wave][lane];
-        wave_lds_fence();
+        wave_order();
         for (uint64_t nz = __ballot(word != 0); nz; nz &= nz - 1) {
           const int l = __builtin_ctzll(nz);
           uint32_t bits = (uint32_t)__builtin_amdgcn_readlane(word, l);

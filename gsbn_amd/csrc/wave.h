@@ -12,6 +12,13 @@
 #include <math.h>
 #include <stdint.h>
 
+/* LDS operations of a wave are processed in order; this only keeps the
+ * compiler from moving them across */
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 /* Wave-wide inclusive prefix sum with DPP moves (gfx9 DPP: row shifts by
  * 1, 2, 4, 8 within each 16-lane row, out-of-row sources reading 0, then
  * row_bcast:15 into rows 1 and 3 and row_bcast:31 into rows 2 and 3), a

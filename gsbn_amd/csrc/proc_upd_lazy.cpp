@@ -946,13 +946,18 @@ void Proj::prepare(int simstep) {
      * over the connectivity as it was; the reference pushes them at the next
      * step, over the one it has then */
     const bool again = direct_que && last_exec >= 0;
-    gsbn_que_args a = last_push();
-    if (again) op_check(gsbn_proj_unque(&a, active_stream()), "gsbn_proj_unque");
+    gsbn_que_args a;
+    if (again) {
+      a = last_push();
+      op_check(gsbn_proj_unque(&a, active_stream()), "gsbn_proj_unque");
+    }
     rebuild_fanout();
     ii_version = _ii->host_version;
     di_version = _di->host_version;
-    a.out = fanout();
-    if (again) op_check(gsbn_proj_que(&a, active_stream()), "gsbn_proj_que");
+    if (again) {
+      a.out = fanout();
+      op_check(gsbn_proj_que(&a, active_stream()), "gsbn_proj_que");
+    }
   }
   (void)_ii->gpu_data();
   (void)_di->gpu_data();

@@ -62,6 +62,7 @@ struct ChunkPool {
   };
   std::mutex mutex;
   vector<Entry> entries; /* oldest first */
+  map<int, size_t> room; /* bytes to keep, per device (asked for once: about 10 us) */
   /* the smallest chunk of `device` with size to `most` bytes */
   char* take(size_t size, size_t most, int device, size_t* got) {
     std::lock_guard<std::mutex> lock(mutex);
@@ -79,13 +80,15 @@ struct ChunkPool {
   /* no work uses the chunk any more */
   void put(char* base, size_t size, int device) {
     std::lock_guard<std::mutex> lock(mutex);
-    size_t avail = 0, total = 0;
-    if (hipMemGetInfo(&avail, &total) != hipSuccess) total = 0;
+    if (!room.count(device)) {
+      size_t avail = 0, total = 0;
+      room[device] = hipMemGetInfo(&avail, &total) == hipSuccess ? total / 8 : 0;
+    }
     entries.push_back({base, size, device});
     size_t held = 0;
     for (auto& e : entries)
       if (e.device == device) held += e.size;
-    for (auto it = entries.begin(); held > total / 8 && it != entries.end();) {
+    for (auto it = entries.begin(); held > room[device] && it != entries.end();) {
       if (it->device != device) {
         ++it;
         continue;

@@ -590,13 +590,17 @@ def frozen_recall(batch: int = 8192, steps: int = 50, clamp_frac: float = 0.4) -
             out[name] = {"cues_per_sec": batch / el, "seconds": el, "recall_correct": float(ok.mean()),
                          "hcu_winner_accuracy": float(np.mean(idx == want)), "idx": idx}
             if mode == R.MFMA:
-                # support products run from step delay+3 on
+                # the dense product in a run of its own (its products run from
+                # step delay+3 on): the timed run computes the support from
+                # the active sources instead
                 _, _, _, sup_ms = rc.run(clamp, wmask, steps, count_from=steps // 2,
                                          time_support=True)
                 N = spec.total_units
                 nprod = steps - 3
                 flops = 2.0 * batch * N * N * nprod
                 out[name]["support_ms"] = sup_ms
+                out[name]["support_run"] = ("the dense product in a run of its own; the run of "
+                                            "cues_per_sec adds the active sources' weights instead")
                 out[name]["mfma_tflops"] = flops / (sup_ms * 1e-3) / 1e12 if sup_ms > 0 else None
             rc.close()
         s.close()
@@ -643,7 +647,8 @@ def main():
                          "same with one wave per part)")
     ap.add_argument("--deferred", type=int, default=None, metavar="K",
                     help="deferred column updates with rings of K spike steps per unit "
-                         "(ProcUpdLazy deferred-columns; 0: eager; default: the library's, 8 for one network, 16 for a batch)")
+                         "(ProcUpdLazy deferred-columns; 0: eager; default: the library's, 8 for one "
+                         "network, 16 for a batch, 64 in blocks)")
     ap.add_argument("--pop-block", action="store_true",
                     help="batches: the population update with one workgroup per hypercolumn "
                          "(ProcUpdLazy pop-wave 0) instead of one wave")

@@ -157,7 +157,8 @@ class NetSpec:
     ovf_cap: Optional[int] = None
     # deferred_columns K (a power of two, 2..64): column updates deferred
     # through rings of K spike steps per postsynaptic unit; 0: eager; None:
-    # ProcUpdLazy's default (where it applies: 8 for one network, 16 for a batch)
+    # ProcUpdLazy's default (where it applies: 8 for one network, 16 for a batch,
+    # 64 from the first block or recorded sweep on)
     deferred_columns: Optional[int] = None
     # block_step 0: steps are never run several per launch; 1: every step is
     # run that way; None: ProcUpdLazy's default (in calls of several steps,

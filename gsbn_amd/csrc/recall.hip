@@ -427,7 +427,7 @@ __device__ __forceinline__ void add_block_mfma(const ReArgs& a, int h, int blk, 
  *
  * What bounds it: issue (Philox and the double sequences of the draw and the
  * soft-max): 630 vector instructions per step of up to 128 units, the vector
- * units 77 % busy.  Hence one wave per
+ * units 85 % busy (mfma 670, 72 %).  Hence one wave per
  * pair without idle waves, the normalisers of a workgroup's pairs summed by
  * as many lanes at once (100 dependent additions for one lane would
  * be 400 issue cycles per pair), and the maximum's exponential evaluated by
@@ -437,8 +437,9 @@ __device__ __forceinline__ void add_block_mfma(const ReArgs& a, int h, int blk, 
  * six waves per SIMD for exact (eight and four: 68.5 ms); the mfma form's
  * accumulators hold it at four.
  * 8192 cues x 50 steps at 100 x 100: exact 54.5 ms (a workgroup per pair and
- * one step per launch: 106.8 ms), mfma 68.2 ms (dense product 75 ms and
- * population step 43 ms: 120 ms); one cue at 10 x 10: 0.23 ms (0.94 ms). */
+ * one step per launch: 107 ms with the same short sequences), mfma 68.5 ms
+ * (dense product 75 ms and population step 43 ms: 120 ms); one cue at 10 x 10:
+ * 0.24 ms (0.94 ms). */
 template <int UPL, bool BF>
 __global__ void __launch_bounds__(64 * RW_WAVES, BF ? (UPL == 1 ? 5 : UPL == 2 ? 4 : 3) : UPL <= 2 ? 6 : 4)
     recall_wave_kernel(ReArgs a, int t0, int nt, int last) {
@@ -787,11 +788,11 @@ __global__ void recall_weights_kernel(int H, int M, int C, int N, int Kp, const 
  * runs on XCD i % 8: each XCD has consecutive tiles, in groups of GM_GROUP row
  * tiles, so that its 32 workgroups share 8 + 4 tiles of operands per K step
  * instead of 32 + 1.
- * What bounds it: the clock under this load (2.2 GHz) and the matrix units two
- * thirds busy; the rest is barrier skew and the tile's end, with one workgroup
- * per CU.  8192 x 10000 x 10048: 1.27 ms, 1.30 PFLOP/s (1.60 ms with 16 waves
- * of 64 x 64, one buffer and E read and written value by value; a vendor
- * library's product takes 1.22-1.30 ms).  16 waves of 64 x 64 in this form
+ * What bounds it: the clock under this load (2.0-2.2 GHz), with the matrix
+ * units 59 % busy; the rest is barrier skew and the tile's end, with one
+ * workgroup per CU.  8192 x 10000 x 10048: 1.27-1.28 ms, 1.28 PFLOP/s (1.60 ms
+ * with 16 waves of 64 x 64, one buffer and E read and written value by value;
+ * a vendor library's product takes 1.26 ms).  16 waves of 64 x 64 in this form
  * 1.28 ms, K steps of 32 1.39, 128 x 256 tiles and two workgroups per CU 1.65,
  * 128 x 128 2.6, 4 waves of 128 x 128 1.54. */
 template <int BM, int BN, int WM, int WN> /* tile, waves down and across it */

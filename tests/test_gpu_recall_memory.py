@@ -2,6 +2,9 @@
 the dense product with the handle where the product is its path, and otherwise
 in the first run that asks for the product's time."""
 
+import gc
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -29,25 +32,40 @@ def _handle(H, M, B):
         (clamp, np.ones((B, H), np.float32))
 
 
+def _free():
+    """Free device memory once it no longer changes: what was given back before
+    (by earlier tests, say) is cleared by the driver first and counted late."""
+    torch.cuda.synchronize()
+    gc.collect()
+    last, same = -1, 0
+    for _ in range(100):
+        now = torch.cuda.mem_get_info()[0]
+        same = same + 1 if now == last else 0
+        if same == 4:
+            break
+        last = now
+        time.sleep(0.05)
+    return now
+
+
 def _taken(f):
-    torch.cuda.synchronize()
-    free = torch.cuda.mem_get_info()[0]
+    before = _free()
     r = f()
-    torch.cuda.synchronize()
-    return free - torch.cuda.mem_get_info()[0], r
+    return before - _free(), r
 
 
 # spike matrices: 64 steps x cues rounded to 256 x units rounded to 64, bf16
-@pytest.mark.parametrize("H,M,B,dense", [(120, 10, 1024, True), (60, 64, 512, False)])
+# (0.64 and 1.0 GB: the runtime's own memory, its scratch above all, comes and
+# goes by some 0.15 GB)
+@pytest.mark.parametrize("H,M,B,dense", [(120, 10, 4096, True), (60, 64, 2048, False)])
 def test_spike_matrices(H, M, B, dense):
     gsbn_amd.release_memory()
     ring = 128 * B * ((H * M + 63) // 64 * 64)
     with_handle, (rc, args) = _taken(lambda: _handle(H, M, B))
-    assert (with_handle >= ring) == dense
-    slack = 32 << 20
-    assert _taken(lambda: rc.run(*args, 0, time_support=True))[0] < slack
-    assert _taken(lambda: rc.run(*args, 3))[0] < slack
+    assert (with_handle > ring // 2) == dense
+    assert _taken(lambda: rc.run(*args, 0, time_support=True))[0] < ring // 2
+    assert _taken(lambda: rc.run(*args, 3))[0] < ring // 2
     timed, out = _taken(lambda: rc.run(*args, 3, time_support=True))
-    assert timed < slack if dense else timed >= ring
+    assert (timed > ring // 2) != dense
     assert out[3] > 0
     rc.close()
